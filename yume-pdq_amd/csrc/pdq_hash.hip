@@ -61,7 +61,7 @@ struct Prefetch<Rgba8> {
 template <int P, int S, int D, typename T, typename Raw>
 __device__ __forceinline__ void stream_step(const T* __restrict__ plane, int lane, int i, float (&acc)[16][2][2],
                                             Chains& cur, Chains& nxt, Raw (&pre)[D][4], float* __restrict__ buf1,
-                                            const Luma& lc) {
+                                            const Luma& lc, float& z) {
   // the rows D steps ahead, loaded unconditionally and clamped into the
   // plane (past row 510 they are not used): a load under a branch makes the
   // compiler copy the ring's registers and wait for every load in flight
@@ -70,11 +70,15 @@ __device__ __forceinline__ void stream_step(const T* __restrict__ plane, int lan
   if constexpr (std::is_same<T, float>::value) {
     // f32 rows feed from their ring slots, which reload after their last use
     chains_feed<2>(cur, pre[S][0]);
+    check_edges(z, pre[S][0]);
     load_raw(plane, row(0), lane, pre[S][0]);
     chains_feed<3>(cur, pre[S][1]);
+    check_edges(z, pre[S][1]);
     load_raw(plane, row(1), lane, pre[S][1]);
     chains_feed<4>(cur, pre[S][2]);
+    check_edges(z, pre[S][2]);
     chains_feed<5>(cur, pre[S][3]);
+    check_edges(z, pre[S][3]);
     chains_start(nxt, pre[S][2], pre[S][3]);
     load_raw(plane, row(2), lane, pre[S][2]);
     load_raw(plane, row(3), lane, pre[S][3]);
@@ -96,6 +100,9 @@ __device__ __forceinline__ void stream_step(const T* __restrict__ plane, int lan
   }
   float c0, c1;
   chains_finish(cur, c0, c1);
+  // lane 63's second value is no output (column 127): its neighbour's sums
+  // come from lane 63 itself
+  if constexpr (std::is_same<T, float>::value) z = __builtin_fmaf(c0, c1, z);
   if (buf1) {
     buf1[i * 128 + 2 * lane] = c0;
     buf1[i * 128 + 2 * lane + 1] = (lane == 63) ? 0.0f : c1;
@@ -103,8 +110,10 @@ __device__ __forceinline__ void stream_step(const T* __restrict__ plane, int lan
   stage1_acc<P>(acc, c0, c1, kDctT.v + i * 16);
 }
 
+// Returns whether this lane saw a NaN or Inf that the fast form would treat
+// differently (f32 planes).
 template <typename T, int D>
-__device__ __forceinline__ void stream_image(const T* __restrict__ plane, int lane, float (&acc)[16][2][2],
+__device__ __forceinline__ bool stream_image(const T* __restrict__ plane, int lane, float (&acc)[16][2][2],
                                              float* __restrict__ buf1, const Luma& lc) {
   using Raw = typename RawRow<T>::type;
   static_assert(4 % D == 0, "ring depth must divide the unroll factor");
@@ -117,6 +126,7 @@ __device__ __forceinline__ void stream_image(const T* __restrict__ plane, int la
   // chains are the current ones of the step after): no copies
   Chains a, b;
   Raw pre[D][4];
+  float z = 0.0f;
   {
     Raw r1, r2;
     load_raw(plane, 1, lane, r1);
@@ -129,20 +139,30 @@ __device__ __forceinline__ void stream_image(const T* __restrict__ plane, int la
     to_f32(r1, x1, lc);
     to_f32(r2, x2, lc);
     chains_start(a, x1, x2);
+    if constexpr (std::is_same<T, float>::value) {
+      check_row(z, x1);
+      check_edges(z, x2);
+    }
   }
   // The accumulator a compressed row feeds is fixed by i mod 4 (alt), so the
   // loop is unrolled by four to keep every accumulator and ring index a
   // constant.
 #pragma unroll 1
   for (int i = 0; i < 124; i += 4) {
-    stream_step<1, 0 % D, D>(plane, lane, i, acc, a, b, pre, buf1, lc);
-    stream_step<0, 1 % D, D>(plane, lane, i + 1, acc, b, a, pre, buf1, lc);
-    stream_step<0, 2 % D, D>(plane, lane, i + 2, acc, a, b, pre, buf1, lc);
-    stream_step<1, 3 % D, D>(plane, lane, i + 3, acc, b, a, pre, buf1, lc);
+    stream_step<1, 0 % D, D>(plane, lane, i, acc, a, b, pre, buf1, lc, z);
+    stream_step<0, 1 % D, D>(plane, lane, i + 1, acc, b, a, pre, buf1, lc, z);
+    stream_step<0, 2 % D, D>(plane, lane, i + 2, acc, a, b, pre, buf1, lc, z);
+    stream_step<1, 3 % D, D>(plane, lane, i + 3, acc, b, a, pre, buf1, lc, z);
   }
-  stream_step<1, 124 % D, D>(plane, lane, 124, acc, a, b, pre, buf1, lc);
-  stream_step<0, 125 % D, D>(plane, lane, 125, acc, b, a, pre, buf1, lc);
-  stream_step<0, 126 % D, D>(plane, lane, 126, acc, a, b, pre, buf1, lc);
+  stream_step<1, 124 % D, D>(plane, lane, 124, acc, a, b, pre, buf1, lc, z);
+  stream_step<0, 125 % D, D>(plane, lane, 125, acc, b, a, pre, buf1, lc, z);
+  stream_step<0, 126 % D, D>(plane, lane, 126, acc, a, b, pre, buf1, lc, z);
+  if constexpr (std::is_same<T, float>::value) {
+    // the last step's loads, clamped to row 511, left it in its last slot
+    check_row(z, pre[126 % D][3]);
+    return nonfinite(z);
+  }
+  return false;
 }
 
 // Stage-1 rows into LDS: tmp[k][j] = nan0(acc0) + nan0(acc1) (x86.rs:207-224);
@@ -221,43 +241,6 @@ __device__ __noinline__ void stream_image_literal(const T* __restrict__ plane, i
   }
 }
 
-// Does the plane hold a value the fast form would treat differently?  Every
-// position of rows 2..510 x cols 2..510 carries a non-zero tap of some output,
-// so a NaN/Inf there makes a stage-1 accumulator non-finite; the remaining
-// positions the reference reads (rows 1 and 511, cols 0, 1 and 511) are
-// checked directly.
-__device__ __forceinline__ bool plane_needs_literal(const float* __restrict__ plane, int lane,
-                                                    const float (&acc)[16][2][2]) {
-  bool bad = false;
-#pragma unroll
-  for (int k = 0; k < 16; k++)
-#pragma unroll
-    for (int jj = 0; jj < 2; jj++) bad = bad || nonfinite(acc[k][jj][0]) || nonfinite(acc[k][jj][1]);
-  Row8 r;
-  load_row(plane, 1, lane, r);
-#pragma unroll
-  for (int m = 0; m < 8; m++) bad |= nonfinite(r.v[m]);
-  load_row(plane, 511, lane, r);
-#pragma unroll
-  for (int m = 0; m < 8; m++) bad |= nonfinite(r.v[m]);
-  for (int row = 2 + lane; row <= 510; row += 64) {
-    const float* pr = plane + (size_t)row * 512;
-    bad = bad || nonfinite(pr[0]) || nonfinite(pr[1]) || nonfinite(pr[511]);
-  }
-  return wave_any(bad);
-}
-
-// u8 and colour inputs are finite by construction.
-__device__ __forceinline__ bool plane_needs_literal(const uint8_t* __restrict__, int, const float (&)[16][2][2]) {
-  return false;
-}
-__device__ __forceinline__ bool plane_needs_literal(const Rgb8* __restrict__, int, const float (&)[16][2][2]) {
-  return false;
-}
-__device__ __forceinline__ bool plane_needs_literal(const Rgba8* __restrict__, int, const float (&)[16][2][2]) {
-  return false;
-}
-
 template <typename T, int D, typename Lds>
 __device__ __forceinline__ void hash_one(const T* __restrict__ planes, uint64_t plane_stride, uint32_t img, int lane,
                                          int wv, uint32_t mode, const HashOutputs& out, Lds& L, const Luma& lc) {
@@ -266,8 +249,7 @@ __device__ __forceinline__ void hash_one(const T* __restrict__ planes, uint64_t 
   WaveLds& W = L.w[wv];
   {
     float acc[16][2][2];
-    stream_image<T, D>(plane, lane, acc, buf1, lc);
-    const bool literal = plane_needs_literal(plane, lane, acc);
+    const bool literal = wave_any(stream_image<T, D>(plane, lane, acc, buf1, lc));
     write_stage1(acc, W, lane);
     if (literal) stream_image_literal(plane, lane, W, buf1, lc);
   }
@@ -288,9 +270,11 @@ __device__ __forceinline__ void hash_one(const T* __restrict__ planes, uint64_t 
 // largest batch serves batches of any size.  Blocks of 4 waves run 3 per CU
 // (46.7 KB of LDS and 168 registers each); blocks of 16 (161.5 KB) run one
 // per CU, four waves per SIMD within 128 registers, which u8 rows reach with
-// one prefetch step in flight (D = 1).
+// one prefetch step in flight (D = 1).  f32 rows hold 32 registers of
+// prefetch, which with the accumulators do not fit 168: two waves per SIMD
+// without spills (226 registers) take 4096 f32 planes at 6.1 TB/s.
 template <typename T, int kW, int D>
-__global__ void __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(kW >= 16 ? 4 : 3))) pdq_hash_kernel(
+__global__ void __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(kW >= 16 ? 4 : std::is_same<T, float>::value ? 2 : 3))) pdq_hash_kernel(
     const T* __restrict__ planes, uint64_t plane_stride, uint32_t n_images, const uint32_t* __restrict__ d_n,
     uint32_t mode, HashOutputs out, Luma lc) {
   const uint32_t n = d_n ? min(*d_n, n_images) : n_images;

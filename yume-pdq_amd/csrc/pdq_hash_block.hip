@@ -65,7 +65,7 @@ struct BandPrefetch<uint8_t> {
 template <int S, int D, typename T, typename Raw>
 __device__ __forceinline__ void band_step(const T* __restrict__ plane, int lane, int i, int i_end, Chains& cur,
                                           Chains& nxt, Raw (&pre)[D][4], float* __restrict__ c, const Luma& lc,
-                                          bool& bad) {
+                                          float& z) {
   // The rows D steps ahead are loaded unconditionally, clamped into the
   // plane (past the band's end they are not used): a load under a branch
   // makes the compiler copy the ring's registers and wait for every load in
@@ -77,11 +77,15 @@ __device__ __forceinline__ void band_step(const T* __restrict__ plane, int lane,
     // f32 rows feed from their ring slots, which reload after their last use
     // (a copy out of the slot would cost eight moves per row)
     chains_feed<2>(cur, pre[S][0]);
+    check_edges(z, pre[S][0]);
     load_raw(plane, row(0), lane, pre[S][0]);
     chains_feed<3>(cur, pre[S][1]);
+    check_edges(z, pre[S][1]);
     load_raw(plane, row(1), lane, pre[S][1]);
     chains_feed<4>(cur, pre[S][2]);
+    check_edges(z, pre[S][2]);
     chains_feed<5>(cur, pre[S][3]);
+    check_edges(z, pre[S][3]);
     chains_start(nxt, pre[S][2], pre[S][3]);
     load_raw(plane, row(2), lane, pre[S][2]);
     load_raw(plane, row(3), lane, pre[S][3]);
@@ -105,7 +109,7 @@ __device__ __forceinline__ void band_step(const T* __restrict__ plane, int lane,
   float c0, c1;
   chains_finish(cur, c0, c1);
   if (lane == 63) c1 = 0.0f;  // column 127 is the zero pad
-  if constexpr (std::is_same<T, float>::value) bad = bad || nonfinite(c0) || nonfinite(c1);
+  if constexpr (std::is_same<T, float>::value) z = __builtin_fmaf(c0, c1, z);
   *reinterpret_cast<float2*>(&c[i * 128 + 2 * lane]) = make_float2(c0, c1);
 }
 
@@ -116,18 +120,19 @@ __device__ __forceinline__ void band_step(const T* __restrict__ plane, int lane,
 template <int S, int D, bool kAll, typename T, typename Raw>
 __device__ __forceinline__ void band_steps(const T* __restrict__ plane, int lane, int i, int i_end, Chains& a,
                                            Chains& b, Raw (&pre)[D][4], float* __restrict__ c, const Luma& lc,
-                                           bool& bad) {
+                                           float& z) {
   static_assert(D % 2 == 0, "an even number of steps returns the chain sets to their roles");
   if (kAll || i + S < i_end) {
     if constexpr (S % 2 == 0)
-      band_step<S, D>(plane, lane, i + S, i_end, a, b, pre, c, lc, bad);
+      band_step<S, D>(plane, lane, i + S, i_end, a, b, pre, c, lc, z);
     else
-      band_step<S, D>(plane, lane, i + S, i_end, b, a, pre, c, lc, bad);
+      band_step<S, D>(plane, lane, i + S, i_end, b, a, pre, c, lc, z);
   }
-  if constexpr (S + 1 < D) band_steps<S + 1, D, kAll>(plane, lane, i, i_end, a, b, pre, c, lc, bad);
+  if constexpr (S + 1 < D) band_steps<S + 1, D, kAll>(plane, lane, i, i_end, a, b, pre, c, lc, z);
 }
 
-// Compressed rows [i0, i1) into c; true if one of them is not finite.
+// Compressed rows [i0, i1) into c; true if an input value that the reference
+// reads for them is NaN or Inf (f32 planes).
 template <typename T>
 __device__ __forceinline__ bool compress_band(const T* __restrict__ plane, int lane, int i0, int i1,
                                               float* __restrict__ c, const Luma& lc) {
@@ -135,6 +140,7 @@ __device__ __forceinline__ bool compress_band(const T* __restrict__ plane, int l
   constexpr int D = BandPrefetch<T>::D;
   Chains cur, nxt;
   Raw pre[D][4];
+  float z = 0.0f;
   {
     Raw r1, r2;
     load_raw(plane, 4 * i0 + 1, lane, r1);
@@ -147,26 +153,25 @@ __device__ __forceinline__ bool compress_band(const T* __restrict__ plane, int l
     to_f32(r1, x1, lc);
     to_f32(r2, x2, lc);
     chains_start(cur, x1, x2);
+    if constexpr (std::is_same<T, float>::value) {
+      // rows 1 and 511 whole; the other bands' first two rows are the last
+      // two of the band before
+      if (i0 == 0) {
+        check_row(z, x1);
+        check_edges(z, x2);
+      }
+      if (i1 == 127) {
+        Row8 last;
+        load_row(plane, 511, lane, last);
+        check_row(z, last);
+      }
+    }
   }
-  bool bad = false;
   int i = i0;
 #pragma unroll 1
-  for (; i + D <= i1; i += D) band_steps<0, D, true>(plane, lane, i, i1, cur, nxt, pre, c, lc, bad);
-  if (i < i1) band_steps<0, D, false>(plane, lane, i, i1, cur, nxt, pre, c, lc, bad);
-  return bad;
-}
-
-// Positions the reference reads that carry no non-zero tap of any output:
-// rows 1 and 511, and columns 0, 1 and 511 of rows 2..510.
-__device__ __forceinline__ bool edges_nonfinite(const float* __restrict__ plane, int t, int n_threads) {
-  bool bad = false;
-  for (int e = t; e < 512; e += n_threads)
-    bad = bad || nonfinite(plane[512 + e]) || nonfinite(plane[511 * 512 + e]);
-  for (int row = 2 + t; row <= 510; row += n_threads) {
-    const float* pr = plane + (size_t)row * 512;
-    bad = bad || nonfinite(pr[0]) || nonfinite(pr[1]) || nonfinite(pr[511]);
-  }
-  return bad;
+  for (; i + D <= i1; i += D) band_steps<0, D, true>(plane, lane, i, i1, cur, nxt, pre, c, lc, z);
+  if (i < i1) band_steps<0, D, false>(plane, lane, i, i1, cur, nxt, pre, c, lc, z);
+  return nonfinite(z);
 }
 
 // ---------------------------------------------------------------------------
@@ -410,11 +415,10 @@ __global__ void __launch_bounds__(64 * kWaves) pdq_hash_block_kernel(const T* __
   // A. compression; the DCT table for stage 1 is copied into LDS after it,
   // so the first plane rows are requested at the kernel's start
   const int i0 = wv * kBand, i1 = min(i0 + kBand, 127);
-  bool bad = compress_band(plane, lane, i0, i1, c, lc);
+  const bool bad = compress_band(plane, lane, i0, i1, c, lc);
   if (wv == kWaves - 1) *reinterpret_cast<float2*>(&c[127 * 128 + 2 * lane]) = make_float2(0.0f, 0.0f);
   if (kPrec == kDctExact || std::is_same<T, float>::value)
     for (int e = t; e < 127 * 16; e += 64 * kWaves) L.dct_t[e] = kDctT.v[e];
-  if constexpr (std::is_same<T, float>::value) bad = bad || edges_nonfinite(plane, t, 64 * kWaves);
   const bool literal = __syncthreads_or(bad ? 1 : 0) != 0;
   if constexpr (std::is_same<T, float>::value) {
     if (literal) {
