@@ -1,0 +1,68 @@
+"""NaN / Inf at the places where the streamed test of f32 planes changes hands
+-- the first and last rows and columns the reference reads, and the rows where
+one wave's band ends and the next begins -- in every layout, and the precise
+kernel's passes: planes inside and outside the range of its fast division,
+mixed in one batch, against the oracle bit for bit."""
+import numpy as np
+import pytest
+
+from yume_pdq import synthetic
+
+pytestmark = pytest.mark.gpu
+
+# bands of 8, 16 and 32 compressed rows start at input rows 32 b + 1, 64 b + 1, 128 b + 1
+PLACES = [(r, c) for r in (1, 2, 3, 32, 33, 34, 64, 65, 66, 128, 129, 130, 509, 510, 511) for c in (1, 2, 511)] + \
+         [(2, 0), (33, 0), (510, 0), (511, 0), (1, 256), (511, 256)]
+
+
+def same(a, b):
+    a, b = np.asarray(a, np.float32), np.asarray(b, np.float32)
+    return bool(np.all((a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))))
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.4e38])
+def test_nonfinite_at_edges(gpu, oracle, dev, value):
+    import torch
+    base = synthetic.images_u8(1, start=70)[0].astype(np.float32)
+    planes = np.repeat(base[None], len(PLACES), 0)
+    for k, (r, c) in enumerate(PLACES):
+        planes[k, r, c] = value
+    x = torch.from_numpy(planes).to(dev)
+    want = [oracle.hash_dihedrals(p, 1) for p in planes]
+    for layout in (gpu.LAYOUT_WAVE, gpu.LAYOUT_BLOCK4, gpu.LAYOUT_BLOCK8, gpu.LAYOUT_BLOCK16):
+        h, q, t = (y.cpu().numpy() for y in gpu.hash_batch(x, layout=layout))
+        for k, (H, Q, T, _) in enumerate(want):
+            where = f"layout {layout}, {value} at {PLACES[k]}"
+            assert np.array_equal(h[k], H), where
+            assert same(q[k], Q) and same(t[k], T), where
+
+
+def ref_planes(n, seed):
+    """Ordinary planes, with every third one outside the fast division's
+    range: a value below 2^-25, above 2^100, NaN or Inf, at a corner."""
+    rng = np.random.default_rng(seed)
+    planes = synthetic.images_u8(n, start=seed).astype(np.float32)
+    planes += rng.uniform(0, 1, planes.shape).astype(np.float32)
+    planes[0, :40, :40] = 0.0
+    planes[0, 40, :] = np.float32(2.0 ** -25)  # the smallest value inside the range
+    odd = [2.0 ** -26, 1e-40, 2.0 ** 101, np.nan, -np.inf]
+    for k in range(1, n, 3):
+        r, c = [(0, 0), (511, 511), (0, 511), (511, 0), (255, 300)][k % 5]
+        planes[k, r, c] = odd[(k // 3) % 5]
+    return planes
+
+
+# image counts around the eight images that share a round of blocks
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 17])
+def test_ref_passes(gpu, oracle, dev, n):
+    import torch
+    planes = ref_planes(n, 80 + n)
+    for kind in ("f32", "u8"):
+        p = planes if kind == "f32" else np.clip(np.nan_to_num(planes), 0, 255).astype(np.uint8)
+        h, q, t, f = (y.cpu().numpy() for y in gpu.hash_ref_batch(torch.from_numpy(p).to(dev), want_pdqf=True))
+        for k in range(n):
+            H, T, Q, P = oracle.hash_ref32(p[k].astype(np.float32))
+            where = f"{kind} image {k} of {n}"
+            assert same(f[k], P), where
+            assert np.array_equal(h[k], H), where
+            assert same(q[k], Q) and same(t[k], T), where
