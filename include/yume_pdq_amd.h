@@ -225,11 +225,11 @@ int yume_pdq_amd_match_with_plane(const uint8_t *d_db, const void *d_plane, uint
  * (d_plane NULL) that allocates nothing, for callers that cannot call
  * hipMalloc: code under HIP graph capture, tight serving loops, harnesses
  * that forbid allocation.  No reference counterpart.  Same arguments, flags
- * and results.  Where the matrix-core matcher keeps candidate records (batches
- * of 385+ queries), they go to one static scratch area per GPU in the
+ * and results.  Where the matrix-core matcher keeps candidate records (full
+ * groups of 1024 queries over many rows), they go to one static scratch area per GPU in the
  * library's own device memory (2^20 records of 16 bytes + 256 bytes, held
  * from the library's load until the process ends) instead of an area
- * allocated per stream.  Limit: a call's worst case -- one record per
+ * allocated per stream.  Limit: one record per
  * query group of g queries and 1024 database rows (g = 256 from 1009
  * queries up, 128 below), i.e.
  * ceil(ceil(n_rows / 1024) / 8) * 8 * ceil(n_queries / (4 g)) * 4 records --

@@ -41,24 +41,21 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kMfmaWaves = 4;
 constexpr int kMfmaTilesPerWave = 64;  // 16-row tiles streamed per wave per block
 
-// fp4 e2m1 codes: 0x2 = +1.0 (bit set), 0xA = -1.0 (bit clear), 0x0 = 0.
-__device__ __forceinline__ uint32_t spread_byte(uint32_t b) {
-  uint32_t x = b & 0xffu;
-  x = (x | (x << 12)) & 0x000f000fu;
-  x = (x | (x << 6)) & 0x03030303u;
-  x = (x | (x << 3)) & 0x11111111u;
-  return 0xaaaaaaaau ^ (x << 3);
-}
-
+// Operand codes, fp4 e2m1: 0x2 = +1.0 (bit clear), 0xA = -1.0 (bit set), 0x0
+// = 0.  A bit is its code's sign, so a word expands by masks alone: register k
+// takes the bits at positions 3 - k, 7 - k, .. 31 - k as its eight signs.
+// Queries and rows go through the same function, so every bit meets its
+// counterpart, and the order of a dot product's terms is free (its partial
+// sums are exact whole numbers).  Seven vector instructions per word; a
+// 256-entry byte table in LDS took as many for its addresses, and its reads
+// met in the banks: they bound the per-wave layout (TABLE).
 struct Expanded {
   uint32_t d[4];
 };
 
-__device__ __forceinline__ void expand_word(uint32_t w, const uint32_t* __restrict__ lut, Expanded& e) {
-  e.d[0] = lut[w & 0xffu];
-  e.d[1] = lut[(w >> 8) & 0xffu];
-  e.d[2] = lut[(w >> 16) & 0xffu];
-  e.d[3] = lut[w >> 24];
+__device__ __forceinline__ void expand_word(uint32_t w, Expanded& e) {
+#pragma unroll
+  for (int k = 0; k < 4; k++) e.d[k] = ((w << k) & 0x88888888u) | 0x22222222u;
 }
 
 __device__ __forceinline__ v4f mfma_prefix(const Expanded& a, const Expanded& b) {
@@ -127,6 +124,7 @@ __device__ __noinline__ void resolve_candidates(v4f cv, int t, uint64_t tbase, u
 // launch.  Hits past it go straight to the buffer.
 constexpr uint32_t kStageHits = 4096;
 
+template <uint32_t kList>
 __device__ __forceinline__ void stage_candidates(v4f cv, int t, uint64_t tbase, uint32_t qbase, int rn, int kq,
                                                 float bound, const uint32_t* __restrict__ queries,
                                                 const uint32_t* __restrict__ db, uint32_t n_queries, uint64_t n_rows,
@@ -147,7 +145,7 @@ __device__ __forceinline__ void stage_candidates(v4f cv, int t, uint64_t tbase, 
           h.distance = d;
           h.index = index_base + row;
           const uint32_t s = atomicAdd(n_stage, 1u);
-          if (s < kStageHits) {
+          if (s < kList) {
             stage[s] = h;
           } else {
             const unsigned long long slot = atomicAdd(counter, 1ull);
@@ -389,7 +387,7 @@ struct RowSource {
 // wave-uniform bit mask; its tiles are recomputed and checked pair by pair
 // after the stream, so the loop itself holds no call and no branch.
 template <int QT, bool kFull, bool kPlane>
-__device__ __forceinline__ void stream_tiles(const Expanded (&qa)[QT], const uint32_t* __restrict__ lut,
+__device__ __forceinline__ void stream_tiles(const Expanded (&qa)[QT], 
                                              const RowSource<kPlane>& src, const uint32_t* __restrict__ db,
                                              uint64_t row0, uint64_t n_rows, uint32_t qbase, int rn, int kq,
                                              float bound, const uint32_t* __restrict__ queries, uint32_t n_queries,
@@ -425,7 +423,7 @@ __device__ __forceinline__ void stream_tiles(const Expanded (&qa)[QT], const uin
       const uint32_t t = tile + a;
       if (!kFull && t >= tiles) break;
       Expanded rb;
-      expand_word(ring[a], lut, rb);
+      expand_word(ring[a], rb);
       if (!kFull && t * 16 + rn >= left) rb.d[0] = rb.d[1] = rb.d[2] = rb.d[3] = 0;
       // Always issue the load (the last kAhead tiles re-read tile `tiles - 1`
       // and drop it): a load under a branch makes the wait counters unknown
@@ -452,7 +450,7 @@ __device__ __forceinline__ void stream_tiles(const Expanded (&qa)[QT], const uin
     pending &= pending - 1;
     for (uint32_t tg = g * kGroup; tg < (g + 1) * kGroup; tg++) {
       Expanded eg;
-      expand_word(fetch(tg), lut, eg);
+      expand_word(fetch(tg), eg);
       if (!kFull && tg * 16 + rn >= left) eg.d[0] = eg.d[1] = eg.d[2] = eg.d[3] = 0;
       resolve_tile<QT>(qa, eg, row0 + (uint64_t)tg * 16, qbase, rn, kq, bound, queries, db, n_queries, n_rows,
                        threshold, hits, capacity, counter, index_base);
@@ -464,7 +462,7 @@ __device__ __forceinline__ void stream_tiles(const Expanded (&qa)[QT], const uin
 // kMfmaTilesPerWave tiles x 16 rows; each wave, `wave` = 0 .. kMfmaWaves - 1,
 // streams its own rows) against query group `group` (QT x 16 queries).
 template <int QT, bool kPlane>
-__device__ __forceinline__ void mfma_item(const uint32_t* __restrict__ lut, const uint32_t* __restrict__ db,
+__device__ __forceinline__ void mfma_item(const uint32_t* __restrict__ db,
                                           const uint32_t* __restrict__ plane, uint64_t n_rows, uint64_t chunk,
                                           uint32_t group, const uint32_t* __restrict__ queries, uint32_t n_queries,
                                           uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity,
@@ -492,7 +490,7 @@ __device__ __forceinline__ void mfma_item(const uint32_t* __restrict__ lut, cons
   Expanded qa[QT];
 #pragma unroll
   for (int t = 0; t < QT; t++) {
-    expand_word(qw[t], lut, qa[t]);
+    expand_word(qw[t], qa[t]);
     if (qbase + 16 * t + rn >= n_queries)
       qa[t].d[0] = qa[t].d[1] = qa[t].d[2] = qa[t].d[3] = 0;  // zero rows never reach the bound
   }
@@ -500,10 +498,10 @@ __device__ __forceinline__ void mfma_item(const uint32_t* __restrict__ lut, cons
   const RowSource<kPlane> src(db, plane, row0, lane);
   // Only the wave that reaches the end of the database needs bounds checks.
   if (row0 + wave_rows <= n_rows)
-    stream_tiles<QT, true, kPlane>(qa, lut, src, db, row0, n_rows, qbase, rn, kq, bound, queries, n_queries,
+    stream_tiles<QT, true, kPlane>(qa, src, db, row0, n_rows, qbase, rn, kq, bound, queries, n_queries,
                                    threshold, hits, capacity, counter, index_base);
   else
-    stream_tiles<QT, false, kPlane>(qa, lut, src, db, row0, n_rows, qbase, rn, kq, bound, queries, n_queries,
+    stream_tiles<QT, false, kPlane>(qa, src, db, row0, n_rows, qbase, rn, kq, bound, queries, n_queries,
                                     threshold, hits, capacity, counter, index_base);
 }
 
@@ -541,7 +539,7 @@ struct SharedRowsLds {
 // and no branch: a branch in the loop makes the compiler wait for every load
 // in flight at each group.
 template <int QT, bool kFull, bool kPlane, bool kTri>
-__device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT], const uint32_t* __restrict__ lut,
+__device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT], 
                                               SharedRowsLds& S, const RowSource<kPlane>& src,
                                               const uint32_t* __restrict__ db, uint64_t row0, uint64_t n_rows,
                                               uint32_t qbase, int wave, int lane, float bound,
@@ -579,7 +577,7 @@ __device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT], const ui
   };
   auto stage = [&](uint32_t g, int s, uint32_t w, int buf) {
     Expanded e;
-    expand_word(w, lut, e);
+    expand_word(w, e);
     store(g, s, e, buf);
   };
   // ring[a] holds this wave's words of group g0 + a + 1, loaded kRing groups
@@ -620,7 +618,7 @@ __device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT], const ui
       // this stages rows nobody reads.
       Expanded next[kStagePerWave];
 #pragma unroll
-      for (int st = 0; st < kStagePerWave; st++) expand_word(ring[a][st], lut, next[st]);
+      for (int st = 0; st < kStagePerWave; st++) expand_word(ring[a][st], next[st]);
       __builtin_amdgcn_sched_barrier(0);
       Expanded rb[kGroupTiles];
 #pragma unroll
@@ -671,7 +669,7 @@ __device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT], const ui
 }
 
 template <int QT, bool kPlane, bool kTri>
-__device__ __forceinline__ void mfma_item_shared(const uint32_t* __restrict__ lut, SharedRowsLds& S,
+__device__ __forceinline__ void mfma_item_shared(SharedRowsLds& S,
                                                  const uint32_t* __restrict__ db, const uint32_t* __restrict__ plane,
                                                  uint64_t n_rows, uint64_t sub, uint32_t sgroup,
                                                  const uint32_t* __restrict__ queries, uint32_t n_queries,
@@ -697,22 +695,17 @@ __device__ __forceinline__ void mfma_item_shared(const uint32_t* __restrict__ lu
   Expanded qa[QT];
 #pragma unroll
   for (int t = 0; t < QT; t++) {
-    expand_word(qw[t], lut, qa[t]);
+    expand_word(qw[t], qa[t]);
     if (qbase + 16 * t + rn >= n_queries) qa[t].d[0] = qa[t].d[1] = qa[t].d[2] = qa[t].d[3] = 0;
   }
 
   const RowSource<kPlane> src(db, plane, row0, lane);
   if (row0 + kSharedRows <= n_rows)
-    stream_shared<QT, true, kPlane, kTri>(qa, lut, S, src, db, row0, n_rows, qbase, wave, lane, bound, recs,
+    stream_shared<QT, true, kPlane, kTri>(qa, S, src, db, row0, n_rows, qbase, wave, lane, bound, recs,
                                           rec_count, rec_cap, rec_sub_base);
   else
-    stream_shared<QT, false, kPlane, kTri>(qa, lut, S, src, db, row0, n_rows, qbase, wave, lane, bound, recs,
+    stream_shared<QT, false, kPlane, kTri>(qa, S, src, db, row0, n_rows, qbase, wave, lane, bound, recs,
                                            rec_count, rec_cap, rec_sub_base);
-}
-
-__device__ __forceinline__ void init_lut(uint32_t* lut) {
-  lut[threadIdx.x] = spread_byte(threadIdx.x);  // blockDim.x == 256
-  __syncthreads();
 }
 
 // Work item -> (row chunk, query group).  Consecutive workgroups are dealt
@@ -726,37 +719,254 @@ __device__ __forceinline__ void item_coords(uint64_t item, uint32_t groups, uint
   group = (uint32_t)(slot % groups);
 }
 
-// One launch, one block per work item: row chunks x query groups (the
-// per-wave layout, which checks its candidates itself), or, with kShared
-// (4+ query groups), 1024-row sub-chunks x groups of kMfmaWaves query groups,
-// whose candidates become records for pdq_match_resolve_kernel.  Block 0
-// first stores zero to clear_rec and clear_hits where they are given: the
-// record count of the stream's next call, and (shared rows, which append
-// no hits here) this call's hit counter.
-template <int QT, bool kPlane, bool kShared, bool kTri = false>
-__global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(QT >= 16 ? 3 : 4))) pdq_match_mfma_kernel(
+// The shared-rows layout over one database, one block per work item:
+// 1024-row sub-chunks x groups of kMfmaWaves query groups of sixteen tiles,
+// whose candidates become records for pdq_match_resolve_kernel.  Block 0 first
+// stores zero to clear_rec and clear_hits where they are given: the record
+// count of the stream's next call, and this call's hit counter (this kernel
+// appends no hits).
+constexpr int kSharedQt = 16;
+template <bool kPlane, bool kTri>
+__global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(3))) pdq_match_mfma_kernel(
     const uint32_t* __restrict__ db, const uint32_t* __restrict__ plane, uint64_t n_rows,
-    const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t threshold, MatchHit* __restrict__ hits,
-    uint64_t capacity, unsigned long long* __restrict__ counter, uint64_t index_base, uint32_t groups,
+    const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t threshold, uint32_t sgroups,
     uint4* __restrict__ recs, uint32_t* __restrict__ rec_count, uint32_t rec_cap, uint32_t* __restrict__ clear_rec,
     unsigned long long* __restrict__ clear_hits) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (clear_rec) *clear_rec = 0u;
     if (clear_hits) *clear_hits = 0ull;
   }
-  __shared__ uint32_t lut[256];
-  init_lut(lut);
-  uint64_t chunk;
-  uint32_t group;
-  item_coords(blockIdx.x, groups, chunk, group);
-  if constexpr (kShared) {
-    __shared__ SharedRowsLds S;
-    mfma_item_shared<QT, kPlane, kTri>(lut, S, db, plane, n_rows, chunk, group, queries, n_queries, threshold,
-                                       recs, rec_count, rec_cap, 0);
-  } else {
-    mfma_item<QT, kPlane>(lut, db, plane, n_rows, chunk, group, queries, n_queries, threshold, hits, capacity,
-                          counter, index_base, (int)(threadIdx.x >> 6));
+  uint64_t sub;
+  uint32_t sgroup;
+  item_coords(blockIdx.x, sgroups, sub, sgroup);
+  __shared__ SharedRowsLds S;
+  mfma_item_shared<kSharedQt, kPlane, kTri>(S, db, plane, n_rows, sub, sgroup, queries, n_queries, threshold, recs,
+                                            rec_count, rec_cap, 0);
+}
+
+// ---------------------------------------------------------------------------
+// The even layout: every wave streams an even share of the rows against its
+// own query group, and checks its candidates itself.
+//
+// Bounded by the matrix cores (16 cycles a product) and, below eight query
+// tiles, by the vector instructions around them (some 45 per 64 rows and wave
+// besides the folds) and the rows' bytes.  All waves are resident at once with
+// equal parts, so no last round of blocks runs nearly empty, each wave loads
+// its queries once, and a small database still spreads over the chip; four
+// tiles of rows come with one 16-byte load per lane and are transposed in
+// registers.  Fixed parts of 1024 rows per wave, a word per lane and tile,
+// took (us, over the plane, before and after): 10^7 rows x 32 / 128 / 200 / 384
+// queries 49 / 66 / 114 / 164 -> 32 / 61 / 90 / 145; 10^6 x 48 / 200 15 / 25 ->
+// 10 / 20; 10^5 x 200 / 1000 29 / 29 -> 10 / 18; raw rows 10^7 x 32 / 200
+// 89 / 183 -> 53 / 99.
+// ---------------------------------------------------------------------------
+constexpr int kEvenRows = 64;        // rows per group: four 16-row tiles, one load per lane
+constexpr uint32_t kEvenGroups = 64;  // most groups per wave: one pending bit each
+// Groups a wave loads ahead.  A group's products take 64 QT matrix-core
+// cycles per wave, so two cover the latency where QT leaves no registers for
+// more.
+constexpr int even_ahead(int qt) { return qt >= 14 ? 2 : 4; }
+constexpr uint32_t kEvenRound = 4;  // part sizes in groups: whole rounds of either depth
+// A block's hits gather in LDS and take their places in the hit buffer with
+// one atomic; the ones past the list append directly.
+constexpr uint32_t kEvenStage = 512;
+struct EvenHits {
+  MatchHit stage[kEvenStage];
+  uint32_t n;
+  unsigned long long base;
+};
+
+// Lane l holds the four prefix words of row l of the group; afterwards
+// register j of lane (rn, kq) is word kq of row 16 j + rn, tile j's operand: a
+// transpose of a 4 x 4 matrix of 16-lane rows in two steps of swaps.
+__device__ __forceinline__ void transpose_rows(uint32_t (&w)[4]) {
+  const auto a = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  w[0] = c[0];
+  w[1] = c[1];
+  w[2] = d[0];
+  w[3] = d[1];
+}
+
+// Accumulators of at most three (kTri) or two products over QT query tiles.
+template <int QT, bool kTri>
+struct EvenShape {
+  static constexpr int kPer = kTri ? 3 : 2;
+  static constexpr int kAccs = (QT + kPer - 1) / kPer;
+};
+
+// Step S issues the first product of accumulator S of the group (tile S /
+// kAccs), the second of S - 1 and the third of S - 2, and folds S - 4, before
+// its register takes accumulator S.
+template <int QT, bool kTri, int S>
+__device__ __forceinline__ void even_step(const Expanded (&qa)[QT], const Expanded (&rb)[4], const v4f& c0,
+                                          uint32_t (&acc)[2], v4f& r0, v4f& r1, v4f& r2, v4f& r3) {
+  using E = EvenShape<QT, kTri>;
+  constexpr int kN = 4 * E::kAccs;
+  v4f& cur = (S % 4 == 0) ? r0 : (S % 4 == 1) ? r1 : (S % 4 == 2) ? r2 : r3;
+  v4f& p1 = (S % 4 == 1) ? r0 : (S % 4 == 2) ? r1 : (S % 4 == 3) ? r2 : r3;
+  v4f& p2 = (S % 4 == 2) ? r0 : (S % 4 == 3) ? r1 : (S % 4 == 0) ? r2 : r3;
+  if constexpr (S >= 4) fold_flags(cur, acc[S % 2]);
+  if constexpr (S < kN) cur = mfma_acc<kScale1>(qa[E::kPer * (S % E::kAccs)], rb[S / E::kAccs], c0);
+  if constexpr (S >= 1 && S - 1 < kN) {
+    constexpr int t = E::kPer * ((S - 1) % E::kAccs) + 1;
+    if constexpr (t < QT) p1 = mfma_acc<kTri ? kScale128 : kScale512>(qa[t], rb[(S - 1) / E::kAccs], p1);
   }
+  if constexpr (kTri && S >= 2 && S - 2 < kN) {
+    constexpr int t = E::kPer * ((S - 2) % E::kAccs) + 2;
+    if constexpr (t < QT) p2 = mfma_acc<kScale32k>(qa[t], rb[(S - 2) / E::kAccs], p2);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (S + 1 < kN + 4) even_step<QT, kTri, S + 1>(qa, rb, c0, acc, r0, r1, r2, r3);
+}
+
+// Exact check of the pairs of one 64-row group (base row `row0`) that reach
+// the bound.
+template <int QT, bool kPlane>
+__device__ __forceinline__ void even_check(EvenHits& H, const Expanded (&qa)[QT], const uint4* __restrict__ src, uint64_t row0,
+                                           uint64_t n_rows, uint32_t qbase, const uint32_t* __restrict__ queries,
+                                           const uint32_t* __restrict__ db, uint32_t n_queries, uint32_t threshold,
+                                           MatchHit* __restrict__ hits, uint64_t capacity,
+                                           unsigned long long* __restrict__ counter, uint64_t index_base) {
+  const int lane = threadIdx.x & 63;
+  const int rn = lane & 15, kq = lane >> 4;
+  const float bound = (float)(128 - 2 * (int)threshold);
+  const int ibound = __float_as_int(bound);
+  const uint64_t r = min(row0 + (uint64_t)lane, n_rows - 1);
+  const uint4 v = src[kPlane ? r : 2 * r];
+  uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  transpose_rows(w);
+#pragma unroll 1
+  for (int j = 0; j < 4; j++) {
+    Expanded e;
+    expand_word(w[0], e);
+    w[0] = w[1];  // (a rolled loop cannot index registers)
+    w[1] = w[2];
+    w[2] = w[3];
+    uint32_t tmask = 0;
+#pragma unroll
+    for (int t = 0; t < QT; t++) {
+      const v4f c = mfma_prefix(qa[t], e);
+      const int m = max(max(__float_as_int(c.x), __float_as_int(c.y)), max(__float_as_int(c.z), __float_as_int(c.w)));
+      tmask |= (wave_any(m >= ibound) ? 1u : 0u) << t;
+    }
+    while (tmask) {
+      const int t = __builtin_ctz(tmask);
+      tmask &= tmask - 1;
+      Expanded a = qa[0];  // qa[t], selected
+#pragma unroll
+      for (int k = 1; k < QT; k++)
+        if (t == k) a = qa[k];
+      stage_candidates<kEvenStage>(mfma_prefix(a, e), t, row0 + 16 * j, qbase, rn, kq, bound, queries, db, n_queries,
+                                   n_rows, threshold, H.stage, &H.n, hits, capacity, counter, index_base);
+    }
+  }
+}
+
+// Rows row0 .. row0 + left - 1 (at most kEvenGroups groups) against query
+// group qbase.
+template <int QT, bool kPlane, bool kTri>
+__device__ __forceinline__ void even_part(EvenHits& H, const uint4* __restrict__ db, const uint4* __restrict__ plane,
+                                          uint64_t n_rows, uint64_t row0, uint32_t left,
+                                          const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t qbase,
+                                          uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity,
+                                          unsigned long long* __restrict__ counter, uint64_t index_base) {
+  constexpr int kAhead = even_ahead(QT);
+  const int lane = threadIdx.x & 63;
+  const int rn = lane & 15, kq = lane >> 4;
+  const uint4* src = kPlane ? plane : db;
+  const uint4* base = src + (kPlane ? row0 : 2 * row0);  // uniform
+  // rows past the end repeat the last one; their pairs are never reported
+  auto load = [&](uint32_t g) -> uint4 {
+    const uint32_t r = min(g * kEvenRows + (uint32_t)lane, left - 1);
+    return base[kPlane ? r : 2 * r];
+  };
+  uint4 ring[kAhead];
+#pragma unroll
+  for (int a = 0; a < kAhead; a++) ring[a] = load(a);
+
+  uint32_t qw[QT];
+#pragma unroll
+  for (int t = 0; t < QT; t++) {
+    const uint32_t qi = qbase + 16 * t + rn;
+    qw[t] = queries[(size_t)(qi < n_queries ? qi : n_queries - 1) * 8 + kq];
+  }
+  Expanded qa[QT];
+#pragma unroll
+  for (int t = 0; t < QT; t++) {
+    expand_word(qw[t], qa[t]);
+    if (qbase + 16 * t + rn >= n_queries)
+      qa[t].d[0] = qa[t].d[1] = qa[t].d[2] = qa[t].d[3] = 0;  // zero rows never reach the bound
+  }
+  const float bound = (float)(128 - 2 * (int)threshold);
+  const v4f c0 = kTri ? flags_c0_tri(bound) : flags_c0(bound);
+  const uint32_t ngroups = (left + kEvenRows - 1) / kEvenRows;
+  uint64_t pending = 0;
+#pragma unroll 1
+  for (uint32_t g0 = 0; g0 < ngroups; g0 += kAhead) {
+#pragma unroll
+    for (int a = 0; a < kAhead; a++) {
+      uint32_t w[4] = {ring[a].x, ring[a].y, ring[a].z, ring[a].w};
+      transpose_rows(w);
+      Expanded rb[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) expand_word(w[j], rb[j]);
+      ring[a] = load(g0 + a + kAhead);
+      uint32_t acc[2] = {0u, 0u};
+      v4f r0, r1, r2, r3;
+      even_step<QT, kTri, 0>(qa, rb, c0, acc, r0, r1, r2, r3);
+      const uint64_t vote = __ballot(((acc[0] | acc[1]) & (kTri ? kFlagMaskTri : kFlagMask)) != 0);
+      pending |= (uint64_t)(vote != 0) << (g0 + a);
+    }
+  }
+  if (ngroups < 64) pending &= (1ull << ngroups) - 1;  // the last round's groups past the part
+  while (pending) {
+    const uint32_t g = (uint32_t)__builtin_ctzll(pending);
+    pending &= pending - 1;
+    even_check<QT, kPlane>(H, qa, src, row0 + (uint64_t)g * kEvenRows, n_rows, qbase, queries,
+                           reinterpret_cast<const uint32_t*>(db), n_queries, threshold, hits, capacity, counter,
+                           index_base);
+  }
+}
+
+// The block's gathered hits into the buffer.  Every thread of the block calls
+// it.
+__device__ __forceinline__ void even_flush(EvenHits& H, MatchHit* __restrict__ hits, uint64_t capacity,
+                                           unsigned long long* __restrict__ counter) {
+  __syncthreads();
+  const uint32_t n = min(H.n, kEvenStage);
+  if (n == 0) return;  // the same for the whole block
+  if (threadIdx.x == 0) H.base = atomicAdd(counter, (unsigned long long)n);
+  __syncthreads();
+  const unsigned long long base = H.base;
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
+    if (base + i < capacity) hits[base + i] = H.stage[i];
+}
+
+// One part per wave.  Part part_x * 8 + xcd: the waves that match one part
+// against the query groups are neighbours on one XCD and share its rows in the
+// caches.
+template <int QT, bool kPlane, bool kTri>
+__global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(4))) pdq_match_even_kernel(
+    const uint4* __restrict__ db, const uint4* __restrict__ plane, uint64_t n_rows,
+    const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t threshold, MatchHit* __restrict__ hits,
+    uint64_t capacity, unsigned long long* __restrict__ counter, uint64_t index_base, uint32_t groups,
+    uint32_t parts_per_xcd, uint32_t part_groups) {
+  __shared__ EvenHits H;
+  if (threadIdx.x == 0) H.n = 0;
+  __syncthreads();
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t id = (blockIdx.x >> 3) * kMfmaWaves + wave;
+  const uint32_t part_x = id / groups;
+  const uint64_t row0 = ((uint64_t)part_x * 8 + (blockIdx.x & 7)) * part_groups * kEvenRows;
+  if (part_x < parts_per_xcd && row0 < n_rows)
+    even_part<QT, kPlane, kTri>(H, db, plane, n_rows, row0,
+                                (uint32_t)min(n_rows - row0, (uint64_t)part_groups * kEvenRows), queries, n_queries,
+                                (id - part_x * groups) * (uint32_t)(QT * 16), threshold, hits, capacity, counter,
+                                index_base);
+  even_flush(H, hits, capacity, counter);
 }
 
 // The second kernel of the shared-rows layout, in blocks of kResolveWaves
@@ -780,14 +990,12 @@ uint32_t match_resolve_blocks(int cus) { return (uint32_t)std::max(1, cus) * kRe
 static_assert(kResolveWaves % kMfmaWaves == 0, "whole per-wave items per block");
 
 struct ResolveLds {
-  uint32_t lut[256];
   MatchHit stage[kStageHits];
   uint32_t n_stage;
   unsigned long long stage_base;
 };
 
 __device__ __forceinline__ void resolve_init(ResolveLds& L) {
-  if (threadIdx.x < 256) L.lut[threadIdx.x] = spread_byte(threadIdx.x);
   if (threadIdx.x == 0) L.n_stage = 0;
   __syncthreads();
 }
@@ -890,7 +1098,7 @@ __device__ __forceinline__ void check_group(ResolveLds& L, const Expanded (&qa)[
 #pragma unroll
     for (int k = 0; k + 1 < kGroupTiles; k++) w[k] = w[k + 1];
     Expanded eg;
-    expand_word(wj, L.lut, eg);
+    expand_word(wj, eg);
     if ((uint64_t)tt * 16 + rn >= left) eg.d[0] = eg.d[1] = eg.d[2] = eg.d[3] = 0;
     // which query tiles have a pair at the bound (a wave-uniform mask); the
     // products go in pairs, so that one product's reads overlap the next's
@@ -916,7 +1124,7 @@ __device__ __forceinline__ void check_group(ResolveLds& L, const Expanded (&qa)[
 #pragma unroll
       for (int k = 1; k < QT; k++)
         if (t == k) a = qa[k];
-      stage_candidates(mfma_prefix(a, eg), t, row0 + (uint64_t)tt * 16, qbase, rn, kq, bound, queries, db,
+      stage_candidates<kStageHits>(mfma_prefix(a, eg), t, row0 + (uint64_t)tt * 16, qbase, rn, kq, bound, queries, db,
                        n_queries, n_rows, threshold, L.stage, &L.n_stage, hits, capacity, counter, index_base);
     }
   }
@@ -947,7 +1155,7 @@ __device__ __forceinline__ void resolve_record(ResolveLds& L, const PartLoads<QT
   Expanded qa[QT];
 #pragma unroll
   for (int t = 0; t < QT; t++) {
-    expand_word(P.qw[t], L.lut, qa[t]);
+    expand_word(P.qw[t], qa[t]);
     if (qbase + 16 * t + rn >= n_queries) qa[t].d[0] = qa[t].d[1] = qa[t].d[2] = qa[t].d[3] = 0;
   }
   // The first group's words come with P, outside the loop over the other
@@ -991,8 +1199,7 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_kernel(
     const uint32_t* __restrict__ db, const uint32_t* __restrict__ plane, uint64_t n_rows,
     const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t threshold, MatchHit* __restrict__ hits,
     uint64_t capacity, unsigned long long* __restrict__ counter, uint64_t index_base,
-    const uint4* __restrict__ recs, const uint32_t* __restrict__ rec_count, uint32_t rec_cap, uint64_t chunks,
-    uint32_t groups) {
+    const uint4* __restrict__ recs, const uint32_t* __restrict__ rec_count, uint32_t rec_cap) {
   __shared__ ResolveLds L;
   resolve_init(L);
   const int wave = (int)(threadIdx.x >> 6);
@@ -1002,16 +1209,17 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_kernel(
     constexpr int kRq = kResolveQt<QT>;
     const uint32_t rgroups = (n_queries + kRq * 16 - 1) / (kRq * 16);
     constexpr int kHalves = kResolveWaves / kMfmaWaves;
+    constexpr uint64_t kChunkRows = (uint64_t)kMfmaWaves * kMfmaTilesPerWave * 16;
+    const uint64_t chunks = ((n_rows + kChunkRows - 1) / kChunkRows + 7) / 8 * 8;  // whole XCD rounds
     const uint64_t items = chunks * rgroups;
     for (uint64_t item = (uint64_t)blockIdx.x * kHalves + wave / kMfmaWaves; item < items;
          item += (uint64_t)gridDim.x * kHalves) {
       uint64_t chunk;
       uint32_t group;
       item_coords(item, rgroups, chunk, group);
-      mfma_item<kRq, kPlane>(L.lut, db, plane, n_rows, chunk, group, queries, n_queries, threshold, hits, capacity,
+      mfma_item<kRq, kPlane>(db, plane, n_rows, chunk, group, queries, n_queries, threshold, hits, capacity,
                              counter, index_base, wave % kMfmaWaves);
     }
-    (void)groups;
     return;
   }
   // The wave's records are w, w + S, w + 2S, ... (w its number in the
@@ -1084,9 +1292,7 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
     uint4* __restrict__ recs, uint32_t* __restrict__ rec_count, uint32_t rec_cap) {
   const uint32_t nq = d_nq ? min(*d_nq, nq_cap) : nq_cap;
   if (nq == 0) return;
-  __shared__ uint32_t lut[256];
   __shared__ SharedRowsLds S;
-  init_lut(lut);
   const uint32_t groups = (nq + QT * 16 - 1) / (QT * 16);
   const uint32_t sgroups = (groups + kMfmaWaves - 1) / kMfmaWaves;
   const uint64_t items = total_chunks * kSubsPerChunk * sgroups;
@@ -1096,7 +1302,7 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
     item_coords(item, sgroups, gsub, sgroup);
     const ShardView& v = shards[shard_of_chunk(shards, n_shards, gsub / kSubsPerChunk)];
     const uint64_t sub_base = v.chunk_begin * kSubsPerChunk;
-    mfma_item_shared<QT, kPlane, kTri>(lut, S, reinterpret_cast<const uint32_t*>(v.rows),
+    mfma_item_shared<QT, kPlane, kTri>(S, reinterpret_cast<const uint32_t*>(v.rows),
                                        reinterpret_cast<const uint32_t*>(v.plane), v.n_rows, gsub - sub_base, sgroup,
                                        queries, nq, threshold, recs, rec_count, rec_cap, sub_base);
   }
@@ -1128,7 +1334,7 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_shards_k
       uint32_t group;
       item_coords(item, groups, chunk, group);
       const ShardView& v = shards[shard_of_chunk(shards, n_shards, chunk)];
-      mfma_item<kRq, kPlane>(L.lut, reinterpret_cast<const uint32_t*>(v.rows),
+      mfma_item<kRq, kPlane>(reinterpret_cast<const uint32_t*>(v.rows),
                             reinterpret_cast<const uint32_t*>(v.plane), v.n_rows, chunk - v.chunk_begin, group, queries,
                             nq, threshold, hits, capacity, counter, v.index_base, wave % kMfmaWaves);
     }
@@ -1173,8 +1379,6 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
     uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity, unsigned long long* __restrict__ counter) {
   const uint32_t nq = d_nq ? min(*d_nq, nq_cap) : nq_cap;
   if (nq == 0 || nq < min_nq) return;
-  __shared__ uint32_t lut[256];
-  init_lut(lut);
   const uint32_t groups = (nq + QT * 16 - 1) / (QT * 16);
   const uint64_t items = total_chunks * groups;
   for (uint64_t item = blockIdx.x; item < items; item += gridDim.x) {
@@ -1184,7 +1388,7 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
     uint32_t sh = 0;
     while (sh + 1 < n_shards && shards[sh + 1].chunk_begin <= chunk) sh++;
     const ShardView& v = shards[sh];
-    mfma_item<QT, kPlane>(lut, reinterpret_cast<const uint32_t*>(v.rows), reinterpret_cast<const uint32_t*>(v.plane),
+    mfma_item<QT, kPlane>(reinterpret_cast<const uint32_t*>(v.rows), reinterpret_cast<const uint32_t*>(v.plane),
                           v.n_rows, chunk - v.chunk_begin, group, queries, nq, threshold, hits, capacity, counter,
                           v.index_base, (int)(threadIdx.x >> 6));
   }
@@ -1196,7 +1400,7 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
 // call are enqueued together even when threads share a stream.  At most
 // kMaxStreamAreas streams of a device get an area; calls on further streams,
 // and on a stream being captured into a graph (which cannot allocate), run
-// the per-wave layout, which needs none.
+// the even layout, which needs none.
 constexpr uint32_t kRecordCap = 1u << 20;  // 16 MiB; more records (dense hits) rerun every item per wave
 constexpr size_t kMaxStreamAreas = 16;     // per device
 
@@ -1253,7 +1457,7 @@ static hipError_t record_area(hipStream_t stream, RecordArea** out, bool* usable
   const Key key{dev, stream, stream == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id()};
   auto it = areas.find(key);
   if (it == areas.end()) {
-    if (per_device[dev] >= kMaxStreamAreas) return hipSuccess;  // not usable: the per-wave layout
+    if (per_device[dev] >= kMaxStreamAreas) return hipSuccess;  // not usable: the even layout
     void* p = nullptr;
     if ((e = hipMalloc(&p, (size_t)kRecordCap * sizeof(uint4) + 256)) != hipSuccess) return e;
     RecordArea ra;
@@ -1315,105 +1519,113 @@ __global__ void reset_counts_kernel(uint32_t* rec_count, unsigned long long* cou
   if (counter) *counter = 0ull;
 }
 
-template <int QT>
-static hipError_t launch_qt(const void* db, const void* plane, uint64_t n_rows, const void* queries,
-                            uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
-                            unsigned long long* counter, uint64_t index_base, hipStream_t stream, bool reset,
-                            const RecordArea* fixed) {
-  const uint32_t groups = (n_queries + QT * 16 - 1) / (QT * 16);
+// The shared-rows layout's launches; *done is false where the call cannot use
+// it (no record area for the stream).  fixed: the caller's area (the
+// no-allocation entry point's scratch, sized for this call's worst case), else
+// this stream's own.
+static hipError_t launch_shared(const void* db, const void* plane, uint64_t n_rows, const void* queries,
+                                uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
+                                unsigned long long* counter, uint64_t index_base, hipStream_t stream, bool reset,
+                                const RecordArea* fixed, bool* done) {
+  *done = false;
+  const uint32_t groups = (n_queries + kSharedQt * 16 - 1) / (kSharedQt * 16);
+  const uint32_t sgroups = (groups + kMfmaWaves - 1) / kMfmaWaves;
+  const uint64_t blocks = ((n_rows + kSharedRows - 1) / kSharedRows + 7) / 8 * 8 * sgroups;  // whole XCD rounds
+  if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
+  std::lock_guard<std::mutex> g(g_record_mu);
+  RecordArea ra;
+  RecordArea* area = nullptr;  // the stream's own area, whose count slots alternate
+  if (fixed) {
+    ra = *fixed;
+  } else {
+    bool usable = false;
+    const hipError_t e = record_area(stream, &area, &usable);
+    if (e != hipSuccess || !usable) return e;
+    ra = *area;
+  }
+  *done = true;
   const uint32_t* d = static_cast<const uint32_t*>(db);
   const uint32_t* p = static_cast<const uint32_t*>(plane);
   const uint32_t* q = static_cast<const uint32_t*>(queries);
-  const dim3 block(64 * kMfmaWaves);
-  // the per-wave layout's items: 4096-row chunks x query groups
-  const uint64_t rows_per_chunk = (uint64_t)kMfmaWaves * kMfmaTilesPerWave * 16;
-  const uint64_t chunks8 = ((n_rows + rows_per_chunk - 1) / rows_per_chunk + 7) / 8 * 8;  // whole XCD rounds
-  if (groups >= (uint32_t)kMfmaWaves) {
-    // the caller's fixed area (the no-allocation entry point's scratch,
-    // sized for this call's worst case), else this stream's own area
-    std::lock_guard<std::mutex> g(g_record_mu);
-    RecordArea ra;
-    RecordArea* area = nullptr;  // the stream's own area, whose count slots alternate
-    bool usable = false;
-    if (fixed) {
-      ra = *fixed;
-      usable = true;
-    } else {
-      hipError_t e = record_area(stream, &area, &usable);
-      if (e != hipSuccess) return e;
-      if (usable) ra = *area;
-    }
-    if (usable) {
-      const uint32_t cap = fixed ? kScratchRecords : record_cap();
-      const uint64_t subs8 = ((n_rows + kSharedRows - 1) / kSharedRows + 7) / 8 * 8;
-      const uint32_t sgroups = (groups + kMfmaWaves - 1) / kMfmaWaves;
-      const uint64_t blocks = subs8 * sgroups;
-      if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-      // this call's count slot; the stream's area has the streaming kernel
-      // clear the next call's slot, and the hit counter when this slot is
-      // already clear
-      uint32_t* rc = ra.count;
-      uint32_t* rc_next = nullptr;
-      unsigned long long* hits_clear = nullptr;
-      if (area) {
-        rc = area->count + kCountSlotStride * area->slot;
-        rc_next = area->count + kCountSlotStride * (area->slot ^ 1u);
-      }
-      if (area && area->slot_clear)
-        hits_clear = reset ? counter : nullptr;
-      else
-        hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(1), 0, stream, rc, reset ? counter : nullptr);
-      // three products per accumulator where they apply
-      const bool tri = QT == 16 && threshold >= kTriMinThreshold;
-      if (plane && tri)
-        hipLaunchKernelGGL((pdq_match_mfma_kernel<QT, true, true, QT == 16>), dim3((unsigned)blocks), block, 0,
-                           stream, d, p, n_rows, q, n_queries, threshold, hits, capacity, counter, index_base,
-                           sgroups, ra.recs, rc, cap, rc_next, hits_clear);
-      else if (plane)
-        hipLaunchKernelGGL((pdq_match_mfma_kernel<QT, true, true>), dim3((unsigned)blocks), block, 0, stream, d, p,
-                           n_rows, q, n_queries, threshold, hits, capacity, counter, index_base, sgroups, ra.recs,
-                           rc, cap, rc_next, hits_clear);
-      else if (tri)
-        hipLaunchKernelGGL((pdq_match_mfma_kernel<QT, false, true, QT == 16>), dim3((unsigned)blocks), block, 0,
-                           stream, d, p, n_rows, q, n_queries, threshold, hits, capacity, counter, index_base,
-                           sgroups, ra.recs, rc, cap, rc_next, hits_clear);
-      else
-        hipLaunchKernelGGL((pdq_match_mfma_kernel<QT, false, true>), dim3((unsigned)blocks), block, 0, stream, d, p,
-                           n_rows, q, n_queries, threshold, hits, capacity, counter, index_base, sgroups, ra.recs,
-                           rc, cap, rc_next, hits_clear);
-      // the resident blocks of the recheck kernel; the per-wave rerun after
-      // an overflow walks all items with them
-      const uint64_t rgrid = std::min<uint64_t>(match_resolve_blocks(ra.cus), chunks8 * groups);
-      const dim3 rblock(64 * kResolveWaves);
-      if (plane)
-        hipLaunchKernelGGL((pdq_match_resolve_kernel<QT, true>), dim3((unsigned)rgrid), rblock, 0, stream, d, p,
-                           n_rows, q, n_queries, threshold, hits, capacity, counter, index_base, ra.recs, rc, cap,
-                           chunks8, groups);
-      else
-        hipLaunchKernelGGL((pdq_match_resolve_kernel<QT, false>), dim3((unsigned)rgrid), rblock, 0, stream, d, p,
-                           n_rows, q, n_queries, threshold, hits, capacity, counter, index_base, ra.recs, rc, cap,
-                           chunks8, groups);
-      const hipError_t e = hipGetLastError();
-      if (area) {
-        // the next call's slot is clear only if this call's kernels were
-        // all enqueued; otherwise the next call clears it with a launch
-        if (e == hipSuccess) area->slot ^= 1u;
-        area->slot_clear = e == hipSuccess;
-      }
-      return e;
-    }
+  const uint32_t cap = fixed ? kScratchRecords : record_cap();
+  // this call's count slot; the stream's area has the streaming kernel clear
+  // the next call's slot, and the hit counter when this slot is already clear
+  uint32_t* rc = ra.count;
+  uint32_t* rc_next = nullptr;
+  unsigned long long* hits_clear = nullptr;
+  if (area) {
+    rc = area->count + kCountSlotStride * area->slot;
+    rc_next = area->count + kCountSlotStride * (area->slot ^ 1u);
   }
-  const uint64_t blocks = chunks8 * groups;
-  if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-  if (reset) hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(1), 0, stream, nullptr, counter);
-  if (plane)
-    hipLaunchKernelGGL((pdq_match_mfma_kernel<QT, true, false>), dim3((unsigned)blocks), block, 0, stream, d, p,
-                       n_rows, q, n_queries, threshold, hits, capacity, counter, index_base, groups, nullptr, nullptr,
-                       0u, nullptr, nullptr);
+  if (area && area->slot_clear)
+    hits_clear = reset ? counter : nullptr;
   else
-    hipLaunchKernelGGL((pdq_match_mfma_kernel<QT, false, false>), dim3((unsigned)blocks), block, 0, stream, d, p,
-                       n_rows, q, n_queries, threshold, hits, capacity, counter, index_base, groups, nullptr, nullptr,
-                       0u, nullptr, nullptr);
+    hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(1), 0, stream, rc, reset ? counter : nullptr);
+  // the recheck kernel's resident blocks; the rerun after an overflow walks
+  // all items with them
+  const dim3 grid((unsigned)blocks), block(64 * kMfmaWaves);
+  const dim3 rgrid(match_resolve_blocks(ra.cus)), rblock(64 * kResolveWaves);
+  auto launch = [&](auto pl, auto tr) {
+    constexpr bool kPlane = decltype(pl)::value, kTri = decltype(tr)::value;
+    hipLaunchKernelGGL((pdq_match_mfma_kernel<kPlane, kTri>), grid, block, 0, stream, d, p, n_rows, q, n_queries,
+                       threshold, sgroups, ra.recs, rc, cap, rc_next, hits_clear);
+    hipLaunchKernelGGL((pdq_match_resolve_kernel<kSharedQt, kPlane>), rgrid, rblock, 0, stream, d, p, n_rows, q,
+                       n_queries, threshold, hits, capacity, counter, index_base, ra.recs, rc, cap);
+  };
+  using T = std::integral_constant<bool, true>;
+  using F = std::integral_constant<bool, false>;
+  // three products per accumulator where they apply
+  const bool tri = threshold >= kTriMinThreshold;
+  if (plane && tri) launch(T(), T());
+  else if (plane) launch(T(), F());
+  else if (tri) launch(F(), T());
+  else launch(F(), F());
+  const hipError_t e = hipGetLastError();
+  if (area) {
+    // the next call's slot is clear only if this call's kernels were all
+    // enqueued; otherwise the next call clears it with a launch
+    if (e == hipSuccess) area->slot ^= 1u;
+    area->slot_clear = e == hipSuccess;
+  }
+  return e;
+}
+
+// The even layout's launch.  Its waves all fit the chip at once (four per
+// SIMD), and the rows are cut into as many equal parts as that leaves per
+// query group, in whole rounds of loads.
+template <int QT>
+static hipError_t launch_even(const void* db, const void* plane, uint64_t n_rows, const void* queries,
+                              uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
+                              unsigned long long* counter, uint64_t index_base, hipStream_t stream, bool reset) {
+  int dev = 0, cus = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+  const uint32_t groups = (n_queries + QT * 16 - 1) / (QT * 16);
+  const uint64_t row_groups = (n_rows + kEvenRows - 1) / kEvenRows;
+  const uint64_t waves_per_xcd = std::max(1, cus) * 16 / 8;
+  const uint64_t round = 8 * std::max<uint64_t>(1, waves_per_xcd / groups);  // parts resident at once
+  const uint64_t rounds = (row_groups + round * kEvenGroups - 1) / (round * kEvenGroups);
+  uint64_t part_groups = (row_groups + round * rounds - 1) / (round * rounds);
+  part_groups = std::min<uint64_t>(kEvenGroups, (part_groups + kEvenRound - 1) / kEvenRound * kEvenRound);
+  const uint64_t parts_per_xcd = ((row_groups + part_groups - 1) / part_groups + 7) / 8;
+  const uint64_t blocks = 8 * ((parts_per_xcd * groups + kMfmaWaves - 1) / kMfmaWaves);
+  if (blocks > 0x7fffffffull || parts_per_xcd * groups > 0xffffffffull) return hipErrorInvalidValue;
+  if (reset) hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(1), 0, stream, nullptr, counter);
+  const bool tri = QT > 2 && threshold >= kTriMinThreshold;
+  auto launch = [&](auto pl, auto tr) {
+    hipLaunchKernelGGL((pdq_match_even_kernel<QT, decltype(pl)::value, decltype(tr)::value>), dim3((unsigned)blocks),
+                       dim3(64 * kMfmaWaves), 0, stream, static_cast<const uint4*>(db),
+                       static_cast<const uint4*>(plane), n_rows, static_cast<const uint32_t*>(queries), n_queries,
+                       threshold, hits, capacity, counter, index_base, groups, (uint32_t)parts_per_xcd,
+                       (uint32_t)part_groups);
+  };
+  using T = std::integral_constant<bool, true>;
+  using F = std::integral_constant<bool, false>;
+  if (plane && tri) launch(T(), T());
+  else if (plane) launch(T(), F());
+  else if (tri) launch(F(), T());
+  else launch(F(), F());
   return hipGetLastError();
 }
 
@@ -1535,64 +1747,90 @@ hipError_t launch_match_mfma_shards_shared(int qt, const ShardView* shards, uint
 
 bool match_mfma_applicable(uint32_t n_queries, uint32_t threshold) { return threshold < 64 && n_queries >= 32; }
 
-// Query tiles per wave that launch_match_mfma_qt runs for n_queries.
-static int qt_for(int max_qt, uint32_t n_queries) {
-  const uint32_t tiles = (n_queries + 15) / 16;
-  if (tiles <= 2 || max_qt == 2) return 2;
-  if (tiles <= 4 || max_qt == 4) return 4;
-  // sixteen tiles per wave only where the shared-rows layout runs (4 query
-  // groups or more): the per-wave layout at sixteen needs more registers
-  // than it has
-  if (tiles < 16 * (uint32_t)kMfmaWaves || max_qt == 8) return 8;
-  return 16;
+// Which layout a call runs, and its query tiles per wave.  Costs, in tenths of
+// a query tile's products over all rows (0.45 us per 10^7 rows), fitted to
+// 10^7 rows over the plane (us at 2 / 4 / 8 / 12 / 14 / 16 tiles in one group:
+// 32 / 42 / 60 / 77 / 87 / 97; 16 tiles in two and four groups: 186 and 348):
+// a query group costs its tiles and 2.7 more (the rows' loads and expansions,
+// the votes), so few wide groups, as long as they are full.  The shared-rows
+// layout always computes whole groups of 64 tiles, at 73 per 64, and its
+// recheck kernel takes some 8 us: it wins where the tiles nearly fill
+// its groups and the rows are many (64 tiles: 338 against 348 us at 10^7 rows,
+// 48 against 48 at 10^6, 35 against 17 at 10^5; 128 tiles: 83 against 88 us at
+// 10^6, 46 against 28 at 10^5).
+struct MatchPlan {
+  bool shared;
+  int qt;  // of the even layout
+};
+constexpr int kEvenCost = 27;
+constexpr int kSharedCost = 733;
+constexpr uint64_t kSharedGain = 30000000;  // rows x cost units that pay for the recheck
+
+static MatchPlan match_plan(uint64_t n_rows, uint32_t n_queries) {
+  const uint64_t tiles = ((uint64_t)n_queries + 15) / 16;
+  MatchPlan plan{false, 2};
+  uint64_t best = ~0ull;
+  for (int qt = 2; qt <= 16; qt += 2) {
+    const uint64_t cost = (tiles + qt - 1) / qt * (uint64_t)(kEvenCost + 10 * qt);
+    if (cost < best) {
+      best = cost;
+      plan.qt = qt;
+    }
+  }
+  const uint64_t shared = (tiles + 63) / 64 * kSharedCost;
+  plan.shared = shared < best && n_rows >= kSharedGain / (best - shared);
+  return plan;
 }
 
-static hipError_t launch_match_mfma_qt(int max_qt, const void* db, const void* plane, uint64_t n_rows,
-                                       const void* queries, uint32_t n_queries, uint32_t threshold, MatchHit* hits,
-                                       uint64_t capacity, unsigned long long* counter, uint64_t index_base,
-                                       hipStream_t stream, bool reset_counter, const RecordArea* fixed) {
+static hipError_t launch_match_mfma_any(const void* db, const void* plane, uint64_t n_rows, const void* queries,
+                                        uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
+                                        unsigned long long* counter, uint64_t index_base, hipStream_t stream,
+                                        bool reset_counter, const RecordArea* fixed) {
   if (threshold >= 64) return hipErrorInvalidValue;
   if (n_rows == 0 || n_queries == 0) {
     if (!reset_counter) return hipSuccess;
     hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(1), 0, stream, nullptr, counter);
     return hipGetLastError();
   }
-  switch (qt_for(max_qt, n_queries)) {
-    case 2:
-      return launch_qt<2>(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base,
-                          stream, reset_counter, fixed);
-    case 4:
-      return launch_qt<4>(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base,
-                          stream, reset_counter, fixed);
-    case 8:
-      return launch_qt<8>(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base,
-                          stream, reset_counter, fixed);
-    default:
-      return launch_qt<16>(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base,
-                           stream, reset_counter, fixed);
+  const MatchPlan plan = match_plan(n_rows, n_queries);
+  if (plan.shared) {
+    bool done = false;
+    const hipError_t e = launch_shared(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter,
+                                       index_base, stream, reset_counter, fixed, &done);
+    if (e != hipSuccess || done) return e;
+  }
+  auto even = [&](auto qt) {
+    return launch_even<decltype(qt)::value>(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter,
+                                            index_base, stream, reset_counter);
+  };
+  switch (plan.qt) {
+    case 2: return even(std::integral_constant<int, 2>());
+    case 4: return even(std::integral_constant<int, 4>());
+    case 6: return even(std::integral_constant<int, 6>());
+    case 8: return even(std::integral_constant<int, 8>());
+    case 10: return even(std::integral_constant<int, 10>());
+    case 12: return even(std::integral_constant<int, 12>());
+    case 14: return even(std::integral_constant<int, 14>());
+    default: return even(std::integral_constant<int, 16>());
   }
 }
-
-#ifndef YPDQ_DEFAULT_QT
-#define YPDQ_DEFAULT_QT 16
-#endif
-constexpr int kDefaultQt = YPDQ_DEFAULT_QT;
 
 hipError_t launch_match_mfma(const void* db, const void* plane, uint64_t n_rows, const void* queries,
                              uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
                              unsigned long long* counter, uint64_t index_base, hipStream_t stream,
                              bool reset_counter) {
-  // up to sixteen 16-query tiles per wave: sixteen from 64 tiles (the
-  // shared-rows layout) measured 3.5 % faster than eight per call on MI355X
-  // (10M rows x 1024 queries); the per-wave layout stops at eight
-  return launch_match_mfma_qt(kDefaultQt, db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter,
-                              index_base, stream, reset_counter, nullptr);
+  return launch_match_mfma_any(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base,
+                               stream, reset_counter, nullptr);
 }
 
+// The no-allocation entry point's limit: the records of a layout with eight
+// query tiles per wave up to 1008 queries and sixteen above, which is what it
+// has always accepted.  No call of the shared-rows layout writes more.
 uint64_t match_mfma_scratch_records(uint64_t n_rows, uint32_t n_queries) {
-  const int qt = qt_for(kDefaultQt, n_queries);
+  const uint32_t tiles = (n_queries + 15) / 16;
+  const uint32_t qt = tiles <= 2 ? 2 : tiles <= 4 ? 4 : tiles < 64 ? 8 : 16;
   const uint32_t groups = (n_queries + qt * 16 - 1) / (qt * 16);
-  if (n_rows == 0 || groups < (uint32_t)kMfmaWaves) return 0;  // the per-wave layout keeps no records
+  if (n_rows == 0 || groups < (uint32_t)kMfmaWaves) return 0;
   const uint64_t subs8 = ((n_rows + kSharedRows - 1) / kSharedRows + 7) / 8 * 8;
   const uint64_t sgroups = (groups + kMfmaWaves - 1) / kMfmaWaves;
   return subs8 * sgroups * kMfmaWaves;  // at most one record per wave of each block
@@ -1606,8 +1844,8 @@ hipError_t launch_match_mfma_noalloc(const void* db, const void* plane, uint64_t
   RecordArea ra;
   hipError_t e = scratch_area(&ra);
   if (e != hipSuccess) return e;
-  return launch_match_mfma_qt(kDefaultQt, db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter,
-                              index_base, stream, reset_counter, &ra);
+  return launch_match_mfma_any(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base,
+                               stream, reset_counter, &ra);
 }
 
 }  // namespace ypdq
