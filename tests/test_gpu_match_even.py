@@ -1,7 +1,7 @@
 """The matrix-core matcher's even layout at its edges -- rows around its 64-row
 groups, parts and rounds, queries around its tiles and query groups, thresholds
 around the change from two to three products per accumulator, hits past a
-block's list -- and the rule that leaves full groups of 64 query tiles over
+block's list, shards of every such size -- and the rule that leaves full groups of 64 query tiles over
 many rows to the shared-rows layout, with and without room for its records."""
 import numpy as np
 import pytest
@@ -100,3 +100,25 @@ def test_full_groups_over_many_rows(gpu, dev, cap):
     n3, h3 = gpu.match(db, q, 31, path="valu")
     assert n1 == n2 == n3 > 0
     assert np.array_equal(triples(h1), triples(h3)) and np.array_equal(triples(h2), triples(h3))
+
+
+@pytest.mark.parametrize("nq", [32, 33, 65, 129, 193, 257, 513, 1100])
+def test_shards_around_their_groups(gpu, oracle, dev, nq):
+    """Shards of one row, around one group, a round, a part: the hits of every
+    shard carry its own base, at thresholds on both sides of the change of the
+    products per accumulator."""
+    import torch
+    sizes = [1, 63, 64, 65, 255, 257, 1, 4095, 4097, 130]
+    queries = synthetic.random_db(nq, seed=nq)
+    parts = [planted(n, queries, 50 + i) for i, n in enumerate(sizes)]
+    q = torch.from_numpy(queries).to(dev)
+    s = gpu.Shards()
+    try:
+        for p in parts:
+            s.add(p)
+        for threshold in (27, 28, 63):
+            n, want = oracle.match_all(np.concatenate(parts), queries, threshold)
+            total, hits = s.match(q, threshold, capacity=1 << 18)
+            assert total == n and np.array_equal(triples(hits), want), threshold
+    finally:
+        s.close()

@@ -102,7 +102,7 @@ int yume_pdq_amd_shards_match(const YumePdqAmdShards* s, const uint8_t* d_querie
   ypdq::MatcherChoice c;
   c.mfma = (flags & YUME_PDQ_AMD_MATCH_MFMA) ||
            (!(flags & YUME_PDQ_AMD_MATCH_VALU) && ypdq::match_mfma_applicable(n_queries, threshold));
-  c.qt = 8;
+  c.width = ypdq::match_plan(s->set->total_rows(), n_queries).qt;
   return status(s->set->launch_match(c, d_queries, nullptr, n_queries, threshold,
                                      reinterpret_cast<ypdq::MatchHit*>(d_hits), capacity, d_count, st));
 }

@@ -17,11 +17,13 @@
 namespace ypdq {
 
 // Which matcher a batch uses: the vector-ALU scan, or the matrix-core filter
-// with qt 16-query tiles per wave, in the per-wave layout or (shared, with a
-// record area) with a block's waves sharing their rows.
+// with at most qt 16-query tiles per wave: in the even layout, whose waves hold
+// `width` tiles each (the batch spread over as many query groups as qt makes),
+// or (shared, with a record area) with a block's waves sharing their rows.
 struct MatcherChoice {
   bool mfma = false;
   int qt = 8;
+  int width = 8;
   bool shared = false;
 };
 
@@ -87,7 +89,7 @@ class ShardSet {
   // One persistent launch over every shard.  d_nq: device query count (or
   // null for nq_cap).  A shared-rows choice needs record_area
   // (match_record_area_bytes(), used by nothing else in flight); without it
-  // the per-wave layout runs.
+  // the even layout runs.
   hipError_t launch_match(const MatcherChoice& c, const void* d_queries, const uint32_t* d_nq, uint32_t nq_cap,
                           uint32_t threshold, MatchHit* hits, uint64_t capacity, unsigned long long* counter,
                           hipStream_t stream, void* record_area = nullptr) const;
@@ -118,7 +120,7 @@ class ShardSet {
   std::mutex mu_;
   std::vector<Shard> shards_;
   ShardView* d_views_ = nullptr;
-  uint64_t total_chunks_ = 0, total_rblocks_ = 0;
+  uint64_t total_chunks_ = 0, total_rblocks_ = 0, total_groups_ = 0;
   uint64_t version_ = 0;
 };
 

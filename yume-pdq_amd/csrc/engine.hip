@@ -260,7 +260,7 @@ hipError_t ShardSet::replace(uint32_t shard, const uint64_t* d_local_rows, const
 
 hipError_t ShardSet::rebuild_views_locked() {
   std::vector<ShardView> v(shards_.size());
-  uint64_t chunk = 0, rblock = 0;
+  uint64_t chunk = 0, rblock = 0, group = 0;
   const MatchTuning vt = default_plane_tuning(0, 0);
   for (size_t i = 0; i < shards_.size(); i++) {
     v[i].rows = reinterpret_cast<const uint4*>(shards_[i].rows);
@@ -269,11 +269,14 @@ hipError_t ShardSet::rebuild_views_locked() {
     v[i].index_base = shards_[i].index_base;
     v[i].chunk_begin = chunk;
     v[i].rblock_begin = rblock;
+    v[i].group_begin = group;
     chunk += mfma_chunks(shards_[i].n_rows);
     rblock += valu_rblocks(vt, shards_[i].n_rows);
+    group += match_row_groups(shards_[i].n_rows);
   }
   total_chunks_ = chunk;
   total_rblocks_ = rblock;
+  total_groups_ = group;
   if (d_views_) (void)hipFree(d_views_);
   d_views_ = nullptr;
   if (v.empty()) return hipSuccess;
@@ -324,27 +327,19 @@ hipError_t ShardSet::launch_match(const MatcherChoice& c, const void* d_queries,
   if (shards_.empty()) return hipSuccess;
   const int cus = cus_;
   if (c.mfma && c.shared && record_area) {
-    // resident blocks of the streaming kernel as below, and of the recheck
+    // resident blocks of the streaming kernel (four per CU) and of the recheck
     // kernel
-    uint64_t grid = (uint64_t)cus * (c.qt >= 16 ? 2 : 4);
-    const uint64_t groups = (nq_cap + c.qt * 16 - 1) / (c.qt * 16);
-    const uint64_t items = total_chunks_ * 4 * ((groups + 3) / 4);
+    uint64_t grid = (uint64_t)cus * 4;
+    const uint64_t items = total_chunks_ * 4 * (((uint64_t)nq_cap + 1023) / 1024);
     if (grid > items) grid = (items + 7) / 8 * 8;
     grid = std::max<uint64_t>(8, grid / 8 * 8);
-    return launch_match_mfma_shards_shared(c.qt, d_views_, (uint32_t)shards_.size(), total_chunks_, true, d_queries,
-                                           d_nq, nq_cap, threshold, hits, capacity, counter, record_area,
-                                           (uint32_t)grid, match_resolve_blocks(cus), stream);
+    return launch_match_shared_shards(d_views_, (uint32_t)shards_.size(), total_chunks_, d_queries, d_nq, nq_cap,
+                                      threshold, hits, capacity, counter, record_area, (uint32_t)grid,
+                                      match_resolve_blocks(cus), stream);
   }
-  if (c.mfma) {
-    // resident blocks: 4 waves per SIMD at 2..8 query tiles, 2 at 16
-    uint64_t grid = (uint64_t)cus * (c.qt >= 16 ? 2 : 4);
-    const uint64_t groups = (nq_cap + c.qt * 16 - 1) / (c.qt * 16);
-    const uint64_t items = total_chunks_ * groups;
-    if (grid > items) grid = (items + 7) / 8 * 8;
-    grid = std::max<uint64_t>(8, grid / 8 * 8);
-    return launch_match_mfma_shards(c.qt, d_views_, (uint32_t)shards_.size(), total_chunks_, true, d_queries, d_nq,
-                                    nq_cap, 0, threshold, hits, capacity, counter, (uint32_t)grid, stream);
-  }
+  if (c.mfma)
+    return launch_match_even_shards(c.width, d_views_, (uint32_t)shards_.size(), total_groups_, d_queries, d_nq,
+                                    nq_cap, threshold, hits, capacity, counter, cus, stream);
   const MatchTuning vt = default_plane_tuning(0, 0);
   uint64_t grid = (uint64_t)cus * 16;
   if (grid > total_rblocks_) grid = total_rblocks_;
@@ -416,9 +411,16 @@ uint64_t BatchContext::device_bytes() const {
   return plane_stride_ * max_images_ + out_bytes(hit_capacity_) + 16 + match_record_area_bytes();
 }
 
-// Rows shared by a block's waves pay off from 4 query groups (one per wave).
-static bool shared_pays(const MatcherChoice& c, uint32_t nq) {
-  return c.mfma && (nq + c.qt * 16 - 1) / (c.qt * 16) >= 4;
+// What a choice of at most c.qt query tiles per wave launches for nq queries:
+// the tiles spread evenly over the query groups that qt makes, or the
+// shared-rows layout where that is the better one for these rows.
+static void set_layout(MatcherChoice* c, uint64_t rows, uint32_t nq) {
+  c->shared = false;
+  if (!c->mfma) return;
+  const int tiles = (int)std::max<uint32_t>(1, (nq + 15) / 16);
+  const int groups = (tiles + c->qt - 1) / c->qt;
+  c->width = ((tiles + groups - 1) / groups + 1) / 2 * 2;
+  c->shared = c->qt == 16 && match_plan(rows, nq).shared;
 }
 
 void BatchContext::refresh_choices() const {
@@ -441,7 +443,7 @@ bool BatchContext::tuned() const {
 // 10^8 rows at 512 queries take 3.75 / 2.52 / 2.04 / 2.05 ms at 2 / 4 / 8 / 16.
 static double mfma_query_cost(int qt) { return qt >= 8 ? 1.0 : qt == 4 ? 1.25 : 1.8; }
 
-// Queries the matrix-core matcher computes for nq: whole groups of 16 qt.
+// Queries in whole groups of 16 qt for nq.
 static uint64_t padded_queries(uint32_t nq, int qt) {
   const uint64_t g = (uint64_t)qt * 16;
   return (nq + g - 1) / g * g;
@@ -449,38 +451,39 @@ static uint64_t padded_queries(uint32_t nq, int qt) {
 
 MatcherChoice BatchContext::choice_for(uint32_t nq) const {
   refresh_choices();
-  // without tuning: vector ALU below 32 queries, eight query tiles per wave
-  // on the matrix cores from 32
   auto it = choices_.upper_bound(nq);
   MatcherChoice c;
   if (it != choices_.begin()) {
     --it;
     c = it->second;
-  } else {
-    c.mfma = threshold_ < 64 && nq >= 32;
-    c.qt = 8;
-  }
-  if (c.mfma) {
-    // a bucket is tuned at its first query count, where every candidate's
-    // groups are full; above it, the last group of a wide tile can be mostly
-    // padding (nq = 320 at 16 tiles computes 512 queries).  Take the narrower
-    // tile when its padded work costs less.
-    int best = c.qt;
-    double best_cost = (double)padded_queries(nq, c.qt) * mfma_query_cost(c.qt);
-    for (int qt = c.qt / 2; qt >= 2; qt /= 2) {
-      const double cost = (double)padded_queries(nq, qt) * mfma_query_cost(qt);
-      if (cost < best_cost) {
-        best = qt;
-        best_cost = cost;
+    if (c.mfma) {
+      // a bucket is tuned at its first query count, where every candidate's
+      // groups are full; above it, the last group of a wide tile can be mostly
+      // empty (nq = 320 at 16 tiles makes groups for 512 queries).  Take the
+      // narrower tile when its whole groups cost less.
+      int best = c.qt;
+      double best_cost = (double)padded_queries(nq, c.qt) * mfma_query_cost(c.qt);
+      for (int qt = c.qt / 2; qt >= 2; qt /= 2) {
+        const double cost = (double)padded_queries(nq, qt) * mfma_query_cost(qt);
+        if (cost < best_cost) {
+          best = qt;
+          best_cost = cost;
+        }
       }
+      c.qt = best;
     }
-    c.qt = best;
+  } else {
+    // without tuning: vector ALU below 32 queries, on the matrix cores from 32
+    // the single-database matcher's plan
+    const MatchPlan plan = match_plan(shards_->total_rows(), nq);
+    c.mfma = threshold_ < 64 && nq >= 32;
+    c.qt = plan.shared ? 16 : plan.qt;
   }
-  c.shared = shared_pays(c, nq);
+  set_layout(&c, shards_->total_rows(), nq);
   return c;
 }
 
-static int choice_key(const MatcherChoice& c) { return c.mfma ? c.qt * 2 + (c.shared ? 1 : 0) : 0; }
+static int choice_key(const MatcherChoice& c) { return c.mfma ? c.width * 2 + (c.shared ? 1 : 0) : 0; }
 
 hipError_t BatchContext::enqueue_body(const MatcherChoice& c, hipStream_t s) {
   HashOutputs o;
@@ -582,7 +585,7 @@ hipError_t BatchContext::autotune(int iterations, std::vector<TuneRecord>* recor
         MatcherChoice m;
         m.mfma = true;
         m.qt = qt;
-        m.shared = shared_pays(m, nq);
+        set_layout(&m, shards_->total_rows(), nq);
         cands.push_back(m);
       }
     float best = 1e30f;

@@ -99,8 +99,9 @@ hipError_t launch_match(const void* db, uint64_t n_rows, const void* queries, ui
                         MatchHit* hits, uint64_t capacity, unsigned long long* counter, uint64_t index_base,
                         hipStream_t stream);
 // A database shard as the persistent multi-shard matchers see it.  Work
-// items are numbered over all shards: MFMA row chunks from chunk_begin (a
-// multiple of 8), vector-ALU row blocks from rblock_begin.
+// items are numbered over all shards: shared-rows chunks from chunk_begin (a
+// multiple of 8), vector-ALU row blocks from rblock_begin, the even layout's
+// row groups from group_begin.
 struct ShardView {
   const uint4* rows;   // n_rows x 32 bytes
   const uint4* plane;  // prefix plane (may be null for the raw-row kernels)
@@ -108,24 +109,33 @@ struct ShardView {
   uint64_t index_base;  // global index of row 0
   uint64_t chunk_begin;
   uint64_t rblock_begin;
+  uint64_t group_begin;
 };
-uint64_t mfma_chunks(uint64_t n_rows);  // MFMA work-item chunks of one shard (multiple of 8)
-hipError_t launch_match_mfma_shards(int qt, const ShardView* shards, uint32_t n_shards, uint64_t total_chunks,
-                                    bool plane, const void* queries, const uint32_t* d_nq, uint32_t nq_cap,
-                                    uint32_t min_nq, uint32_t threshold, MatchHit* hits, uint64_t capacity,
-                                    unsigned long long* counter, uint32_t grid, hipStream_t stream);
-// The shared-rows layout over a set of shards (4 or more query groups pay
-// off): record-count reset, persistent streaming kernel, recheck kernel.
-// record_area: match_record_area_bytes() of device memory used by no other
-// launch in flight (a batch context's own).
+uint64_t mfma_chunks(uint64_t n_rows);       // shared-rows chunks of one shard (multiple of 8)
+uint64_t match_row_groups(uint64_t n_rows);  // the even layout's row groups of one shard
+// The matrix-core matcher for n_queries over n_rows rows: the shared-rows
+// layout, or the even layout with qt (2, 4, .. 16) query tiles per wave.
+struct MatchPlan {
+  bool shared;
+  int qt;
+};
+MatchPlan match_plan(uint64_t n_rows, uint32_t n_queries);
+// The even layout over a set of shards (their prefix planes), on a GPU of
+// `cus` compute units.
+hipError_t launch_match_even_shards(int qt, const ShardView* shards, uint32_t n_shards, uint64_t row_groups,
+                                    const void* queries, const uint32_t* d_nq, uint32_t nq_cap, uint32_t threshold,
+                                    MatchHit* hits, uint64_t capacity, unsigned long long* counter, int cus,
+                                    hipStream_t stream);
+// The shared-rows layout over a set of shards: record-count reset, persistent
+// streaming kernel, recheck kernel.  record_area: match_record_area_bytes() of
+// device memory used by no other launch in flight (a batch context's own).
 uint64_t match_record_area_bytes();
 // Grid of the shared-rows recheck kernel on a GPU of `cus` compute units.
 uint32_t match_resolve_blocks(int cus);
-hipError_t launch_match_mfma_shards_shared(int qt, const ShardView* shards, uint32_t n_shards, uint64_t total_chunks,
-                                           bool plane, const void* queries, const uint32_t* d_nq, uint32_t nq_cap,
-                                           uint32_t threshold, MatchHit* hits, uint64_t capacity,
-                                           unsigned long long* counter, void* record_area, uint32_t grid,
-                                           uint32_t rgrid, hipStream_t stream);
+hipError_t launch_match_shared_shards(const ShardView* shards, uint32_t n_shards, uint64_t total_chunks,
+                                      const void* queries, const uint32_t* d_nq, uint32_t nq_cap, uint32_t threshold,
+                                      MatchHit* hits, uint64_t capacity, unsigned long long* counter,
+                                      void* record_area, uint32_t grid, uint32_t rgrid, hipStream_t stream);
 hipError_t launch_match_valu_shards(const MatchTuning& t, const ShardView* shards, uint32_t n_shards,
                                     uint64_t total_rblocks, bool plane, const void* queries, const uint32_t* d_nq,
                                     uint32_t nq_cap, uint32_t max_nq, uint32_t threshold, MatchHit* hits,

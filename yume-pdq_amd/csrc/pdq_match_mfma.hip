@@ -46,9 +46,9 @@ constexpr int kMfmaTilesPerWave = 64;  // 16-row tiles streamed per wave per blo
 // takes the bits at positions 3 - k, 7 - k, .. 31 - k as its eight signs.
 // Queries and rows go through the same function, so every bit meets its
 // counterpart, and the order of a dot product's terms is free (its partial
-// sums are exact whole numbers).  Seven vector instructions per word; a
-// 256-entry byte table in LDS took as many for its addresses, and its reads
-// met in the banks: they bound the per-wave layout (TABLE).
+// sums are exact whole numbers).  Seven vector instructions per word, as many
+// as the addresses of a byte table in LDS took, without its reads, its set-up
+// at each block's start or its barrier (same times at full occupancy).
 struct Expanded {
   uint32_t d[4];
 };
@@ -73,62 +73,46 @@ __device__ __forceinline__ uint32_t full_distance(const uint32_t* __restrict__ a
   return d;
 }
 
+// A block's hits gather in LDS and take their places in the hit buffer with
+// one atomic: thousands of appends to the one global counter from a short
+// kernel serialise on it (measured in the recheck kernel: 49 of 68
+// microseconds for 4938 hits).  Hits past the list append directly.
+template <uint32_t kList>
+struct HitList {
+  MatchHit stage[kList];
+  uint32_t n;
+  unsigned long long base;
+};
+constexpr uint32_t kStageHits = 4096;  // recheck kernel: two blocks per CU, about two million per launch
+constexpr uint32_t kEvenStage = 512;   // even layout
+
+template <uint32_t kList>
+__device__ __forceinline__ void hits_init(HitList<kList>& L) {
+  if (threadIdx.x == 0) L.n = 0;
+  __syncthreads();
+}
+
+// The gathered hits into the buffer: one run of places.  Every thread of the
+// block calls it.
+template <uint32_t kList>
+__device__ __forceinline__ void hits_flush(HitList<kList>& L, MatchHit* __restrict__ hits, uint64_t capacity,
+                                           unsigned long long* __restrict__ counter) {
+  __syncthreads();
+  const uint32_t n = min(L.n, kList);
+  if (n == 0) return;  // the same for the whole block
+  if (threadIdx.x == 0) L.base = atomicAdd(counter, (unsigned long long)n);
+  __syncthreads();
+  const unsigned long long base = L.base;
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
+    if (base + i < capacity) hits[base + i] = L.stage[i];
+}
+
 // Exact check of query tile t's candidates in this lane's four outputs.
-__device__ __forceinline__ void check_candidates(v4f cv, int t, uint64_t tbase, uint32_t qbase, int rn, int kq,
-                                                 float bound, const uint32_t* __restrict__ queries,
-                                                 const uint32_t* __restrict__ db, uint32_t n_queries, uint64_t n_rows,
-                                                 uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity,
-                                                 unsigned long long* __restrict__ counter, uint64_t index_base) {
-  const uint64_t row = tbase + rn;
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const float v = r == 0 ? cv.x : r == 1 ? cv.y : r == 2 ? cv.z : cv.w;
-    if (v >= bound) {
-      const uint32_t qi = qbase + 16 * t + 4 * kq + r;
-      if (qi < n_queries && row < n_rows) {
-        const uint32_t d = full_distance(queries + (size_t)qi * 8, db + row * 8);
-        if (d <= threshold) {
-          const unsigned long long slot = atomicAdd(counter, 1ull);
-          if (slot < capacity) {
-            MatchHit h;
-            h.query = qi;
-            h.distance = d;
-            h.index = index_base + row;
-            hits[slot] = h;
-          }
-        }
-      }
-    }
-  }
-}
-
-// The same out of line, for the per-wave layout, whose rare path keeps the
-// stream's query operands (inlined there it spills registers into the tile
-// loop).  (The shared-rows streaming kernel checks nothing itself: a call
-// anywhere in it, even one that never runs, cost its tile loop about 12 %,
-// and inline checks 9 %; its second kernel checks with stage_candidates.)
-__device__ __noinline__ void resolve_candidates(v4f cv, int t, uint64_t tbase, uint32_t qbase, int rn, int kq,
-                                                float bound, const uint32_t* __restrict__ queries,
-                                                const uint32_t* __restrict__ db, uint32_t n_queries, uint64_t n_rows,
-                                                uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity,
-                                                unsigned long long* __restrict__ counter, uint64_t index_base) {
-  check_candidates(cv, t, tbase, qbase, rn, kq, bound, queries, db, n_queries, n_rows, threshold, hits, capacity,
-                   counter, index_base);
-}
-
-// The shared-rows layout's second kernel appends to its block's hit list in
-// LDS (stage, n_stage) and takes its slots in the hit buffer once per block:
-// thousands of appends to the one global counter from a short kernel
-// serialise on it (measured: 49 of 68 microseconds for 4938 hits).  The list
-// (64 KiB) holds 4096 hits: with one block per CU, about a million per
-// launch.  Hits past it go straight to the buffer.
-constexpr uint32_t kStageHits = 4096;
-
 template <uint32_t kList>
 __device__ __forceinline__ void stage_candidates(v4f cv, int t, uint64_t tbase, uint32_t qbase, int rn, int kq,
                                                 float bound, const uint32_t* __restrict__ queries,
                                                 const uint32_t* __restrict__ db, uint32_t n_queries, uint64_t n_rows,
-                                                uint32_t threshold, MatchHit* stage, uint32_t* n_stage,
+                                                uint32_t threshold, HitList<kList>& L,
                                                 MatchHit* __restrict__ hits, uint64_t capacity,
                                                 unsigned long long* __restrict__ counter, uint64_t index_base) {
   const uint64_t row = tbase + rn;
@@ -144,9 +128,9 @@ __device__ __forceinline__ void stage_candidates(v4f cv, int t, uint64_t tbase, 
           h.query = qi;
           h.distance = d;
           h.index = index_base + row;
-          const uint32_t s = atomicAdd(n_stage, 1u);
+          const uint32_t s = atomicAdd(&L.n, 1u);
           if (s < kList) {
-            stage[s] = h;
+            L.stage[s] = h;
           } else {
             const unsigned long long slot = atomicAdd(counter, 1ull);
             if (slot < capacity) hits[slot] = h;
@@ -154,29 +138,6 @@ __device__ __forceinline__ void stage_candidates(v4f cv, int t, uint64_t tbase, 
         }
       }
     }
-  }
-}
-
-// Maximum over one 16-row tile of the dot products with every query tile of
-// the wave, kept in four running maxima (query tile t feeds mx[t % 4]) so the
-// max instructions of consecutive products do not wait on each other.  The
-// products are integers in [-128, 128] and the bound is positive, so
-// comparing float bit patterns as signed integers orders them exactly
-// (negative floats are negative integers); integer max3 needs no NaN
-// canonicalisation.  (Element-wise __float_as_int: a bit cast of a vector
-// element expression is miscompiled to element 0 by this toolchain.)
-constexpr int kMaxChains = 4;
-
-template <int QT>
-__device__ __forceinline__ void tile_max(const Expanded (&qa)[QT], const Expanded& rb, int (&mx)[kMaxChains]) {
-#pragma unroll
-  for (int t = 0; t < QT; t++) {
-    const v4f c = mfma_prefix(qa[t], rb);
-    const int c0 = __float_as_int(c.x), c1 = __float_as_int(c.y);
-    const int c2 = __float_as_int(c.z), c3 = __float_as_int(c.w);
-    int& m = mx[t % kMaxChains];
-    m = max(max(m, c0), c1);
-    m = max(max(m, c2), c3);
   }
 }
 
@@ -349,22 +310,6 @@ __device__ __forceinline__ void group_flags_tri(const Expanded (&qa)[16], const 
   group_flags_tri_step<kTiles, 0>(qa, rb, c0, acc, r0, r1, r2, r3);
 }
 
-// The rare path: recompute one tile's products and re-check every pair that
-// clears the bound with the exact 256-bit distance.
-template <int QT>
-__device__ __forceinline__ void resolve_tile(const Expanded (&qa)[QT], const Expanded& rb, uint64_t tbase,
-                                             uint32_t qbase, int rn, int kq, float bound,
-                                             const uint32_t* __restrict__ queries, const uint32_t* __restrict__ db,
-                                             uint32_t n_queries, uint64_t n_rows, uint32_t threshold,
-                                             MatchHit* __restrict__ hits, uint64_t capacity,
-                                             unsigned long long* __restrict__ counter, uint64_t index_base) {
-  for (int t = 0; t < QT; t++) {
-    const v4f c = mfma_prefix(qa[t], rb);
-    resolve_candidates(c, t, tbase, qbase, rn, kq, bound, queries, db, n_queries, n_rows, threshold, hits, capacity,
-                       counter, index_base);
-  }
-}
-
 // Where a wave's row words come from.  Lane (rn, kq) needs word kq of row
 // 16 * tile + rn.  Raw rows: db[r * 8 + kq] -- 16 of every 32 bytes,
 // scattered over 4 cache lines per tile.  Prefix plane (the first 16 bytes of
@@ -379,131 +324,6 @@ struct RowSource {
     return p[(size_t)tile * (kPlane ? 64 : 128)];
   }
 };
-
-// Stream the wave's tiles: loads run kAhead tiles ahead, each tile's word is
-// expanded to fp4 codes just before its products, and the bound is tested
-// once per kGroup tiles.  A group that reaches it (about once per
-// million tiles on random data, plus the true hits) is only noted in a
-// wave-uniform bit mask; its tiles are recomputed and checked pair by pair
-// after the stream, so the loop itself holds no call and no branch.
-template <int QT, bool kFull, bool kPlane>
-__device__ __forceinline__ void stream_tiles(const Expanded (&qa)[QT], 
-                                             const RowSource<kPlane>& src, const uint32_t* __restrict__ db,
-                                             uint64_t row0, uint64_t n_rows, uint32_t qbase, int rn, int kq,
-                                             float bound, const uint32_t* __restrict__ queries, uint32_t n_queries,
-                                             uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity,
-                                             unsigned long long* __restrict__ counter, uint64_t index_base) {
-  constexpr int kAhead = 8;
-  constexpr int kGroup = kFull ? 4 : 1;
-  static_assert(kMfmaTilesPerWave % kAhead == 0 && kAhead % kGroup == 0, "tile loop shape");
-  static_assert(kMfmaTilesPerWave / kGroup <= 64, "one mask bit per group");
-  // rows of this wave that exist (the last wave of the database only)
-  const uint32_t left = kFull ? 0u : (uint32_t)(n_rows - row0);
-  const uint32_t tiles = kFull ? (uint32_t)kMfmaTilesPerWave : (left + 15) / 16;
-  auto fetch = [&](uint32_t tile) -> uint32_t {
-    if (kFull || kPlane) return src(tile);  // the plane is padded to whole tiles
-    return (tile * 16 + rn < left) ? src(tile) : 0u;
-  };
-  uint32_t ring[kAhead];
-#pragma unroll
-  for (int a = 0; a < kAhead; a++) ring[a] = fetch(a < (int)tiles ? a : tiles - 1);
-  int mx[kMaxChains];
-  uint32_t acc[kFlagChains];
-#pragma unroll
-  for (int m = 0; m < kMaxChains; m++) mx[m] = INT32_MIN;
-#pragma unroll
-  for (int m = 0; m < kFlagChains; m++) acc[m] = 0u;
-  const int ibound = __float_as_int(bound);
-  const v4f c0 = flags_c0(bound);
-  uint64_t pending = 0;  // groups whose products reached the bound
-#pragma unroll 1
-  for (uint32_t tile = 0; tile < tiles; tile += kAhead) {
-#pragma unroll
-    for (int a = 0; a < kAhead; a++) {
-      const uint32_t t = tile + a;
-      if (!kFull && t >= tiles) break;
-      Expanded rb;
-      expand_word(ring[a], rb);
-      if (!kFull && t * 16 + rn >= left) rb.d[0] = rb.d[1] = rb.d[2] = rb.d[3] = 0;
-      // Always issue the load (the last kAhead tiles re-read tile `tiles - 1`
-      // and drop it): a load under a branch makes the wait counters unknown
-      // to the compiler, which then waits for every load in flight.
-      ring[a] = fetch(t + kAhead < tiles ? t + kAhead : tiles - 1);
-      if constexpr (QT >= 8) {
-        const Expanded rbs[1] = {rb};
-        group_flags<QT, 1>(qa, rbs, c0, acc);
-      } else {
-        tile_max<QT>(qa, rb, mx);
-      }
-      if (a % kGroup == kGroup - 1) {
-        const int mall = max(max(mx[0], mx[1]), max(mx[2], mx[3]));
-        pending |= (uint64_t)(wave_any(mall >= ibound || flags_set(acc)) ? 1u : 0u) << (t / kGroup);
-#pragma unroll
-        for (int m = 0; m < kMaxChains; m++) mx[m] = INT32_MIN;
-#pragma unroll
-        for (int m = 0; m < kFlagChains; m++) acc[m] = 0u;
-      }
-    }
-  }
-  while (pending) {
-    const uint32_t g = (uint32_t)__builtin_ctzll(pending);
-    pending &= pending - 1;
-    for (uint32_t tg = g * kGroup; tg < (g + 1) * kGroup; tg++) {
-      Expanded eg;
-      expand_word(fetch(tg), eg);
-      if (!kFull && tg * 16 + rn >= left) eg.d[0] = eg.d[1] = eg.d[2] = eg.d[3] = 0;
-      resolve_tile<QT>(qa, eg, row0 + (uint64_t)tg * 16, qbase, rn, kq, bound, queries, db, n_queries, n_rows,
-                       threshold, hits, capacity, counter, index_base);
-    }
-  }
-}
-
-// One work item: row chunk `chunk` of a database (kMfmaWaves waves x
-// kMfmaTilesPerWave tiles x 16 rows; each wave, `wave` = 0 .. kMfmaWaves - 1,
-// streams its own rows) against query group `group` (QT x 16 queries).
-template <int QT, bool kPlane>
-__device__ __forceinline__ void mfma_item(const uint32_t* __restrict__ db,
-                                          const uint32_t* __restrict__ plane, uint64_t n_rows, uint64_t chunk,
-                                          uint32_t group, const uint32_t* __restrict__ queries, uint32_t n_queries,
-                                          uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity,
-                                          unsigned long long* __restrict__ counter, uint64_t index_base,
-                                          int wave) {
-  const int lane = threadIdx.x & 63;
-  const int rn = lane & 15;  // operand row (query m / db row n) of this lane
-  const int kq = lane >> 4;  // K quarter = word index of the prefix
-  const float bound = (float)(128 - 2 * (int)threshold);
-
-  const uint64_t wave_rows = (uint64_t)kMfmaTilesPerWave * 16;
-  const uint64_t row0 = (chunk * kMfmaWaves + wave) * wave_rows;
-  if (row0 >= n_rows) return;
-
-  // query operands: tile t, query qbase + 16t + rn, word kq
-  const uint32_t qbase = group * (uint32_t)(QT * 16);
-  // All QT words are loaded before any is used (loads clamped in bounds rather
-  // than branched around, so they overlap instead of waiting one by one).
-  uint32_t qw[QT];
-#pragma unroll
-  for (int t = 0; t < QT; t++) {
-    const uint32_t qi = qbase + 16 * t + rn;
-    qw[t] = queries[(size_t)(qi < n_queries ? qi : n_queries - 1) * 8 + kq];
-  }
-  Expanded qa[QT];
-#pragma unroll
-  for (int t = 0; t < QT; t++) {
-    expand_word(qw[t], qa[t]);
-    if (qbase + 16 * t + rn >= n_queries)
-      qa[t].d[0] = qa[t].d[1] = qa[t].d[2] = qa[t].d[3] = 0;  // zero rows never reach the bound
-  }
-
-  const RowSource<kPlane> src(db, plane, row0, lane);
-  // Only the wave that reaches the end of the database needs bounds checks.
-  if (row0 + wave_rows <= n_rows)
-    stream_tiles<QT, true, kPlane>(qa, src, db, row0, n_rows, qbase, rn, kq, bound, queries, n_queries,
-                                   threshold, hits, capacity, counter, index_base);
-  else
-    stream_tiles<QT, false, kPlane>(qa, src, db, row0, n_rows, qbase, rn, kq, bound, queries, n_queries,
-                                    threshold, hits, capacity, counter, index_base);
-}
 
 // Shared-rows work item, for batches of kMfmaWaves or more query groups: the
 // block's waves stream the same kSharedTiles 16-row tiles (rows
@@ -767,14 +587,6 @@ constexpr uint32_t kEvenGroups = 64;  // most groups per wave: one pending bit e
 // more.
 constexpr int even_ahead(int qt) { return qt >= 14 ? 2 : 4; }
 constexpr uint32_t kEvenRound = 4;  // part sizes in groups: whole rounds of either depth
-// A block's hits gather in LDS and take their places in the hit buffer with
-// one atomic; the ones past the list append directly.
-constexpr uint32_t kEvenStage = 512;
-struct EvenHits {
-  MatchHit stage[kEvenStage];
-  uint32_t n;
-  unsigned long long base;
-};
 
 // Lane l holds the four prefix words of row l of the group; afterwards
 // register j of lane (rn, kq) is word kq of row 16 j + rn, tile j's operand: a
@@ -824,8 +636,8 @@ __device__ __forceinline__ void even_step(const Expanded (&qa)[QT], const Expand
 
 // Exact check of the pairs of one 64-row group (base row `row0`) that reach
 // the bound.
-template <int QT, bool kPlane>
-__device__ __forceinline__ void even_check(EvenHits& H, const Expanded (&qa)[QT], const uint4* __restrict__ src, uint64_t row0,
+template <int QT, bool kPlane, uint32_t kList>
+__device__ __forceinline__ void even_check(HitList<kList>& H, const Expanded (&qa)[QT], const uint4* __restrict__ src, uint64_t row0,
                                            uint64_t n_rows, uint32_t qbase, const uint32_t* __restrict__ queries,
                                            const uint32_t* __restrict__ db, uint32_t n_queries, uint32_t threshold,
                                            MatchHit* __restrict__ hits, uint64_t capacity,
@@ -859,16 +671,34 @@ __device__ __forceinline__ void even_check(EvenHits& H, const Expanded (&qa)[QT]
 #pragma unroll
       for (int k = 1; k < QT; k++)
         if (t == k) a = qa[k];
-      stage_candidates<kEvenStage>(mfma_prefix(a, e), t, row0 + 16 * j, qbase, rn, kq, bound, queries, db, n_queries,
-                                   n_rows, threshold, H.stage, &H.n, hits, capacity, counter, index_base);
+      stage_candidates(mfma_prefix(a, e), t, row0 + 16 * j, qbase, rn, kq, bound, queries, db, n_queries, n_rows,
+                       threshold, H, hits, capacity, counter, index_base);
     }
   }
 }
 
+// How the rows' groups are cut: the waves of one XCD, all resident at once,
+// hold as many parts as they have room for per query group; more rows take
+// several equal rounds.  Parts are whole rounds of loads.
+struct EvenParts {
+  uint32_t groups;   // row groups per part
+  uint32_t per_xcd;  // parts per XCD
+};
+__host__ __device__ inline EvenParts even_parts(uint32_t row_groups, uint32_t query_groups, uint32_t waves_per_xcd) {
+  const uint32_t at_once = waves_per_xcd / query_groups;
+  const uint64_t round = 8ull * (at_once ? at_once : 1);  // parts resident at once
+  const uint64_t rounds = ((uint64_t)row_groups + round * kEvenGroups - 1) / (round * kEvenGroups);
+  const uint64_t all = round * (rounds ? rounds : 1);
+  uint32_t n = (uint32_t)(((uint64_t)row_groups + all - 1) / all);
+  n = (n + kEvenRound - 1) / kEvenRound * kEvenRound;
+  n = n == 0 ? kEvenRound : n > kEvenGroups ? kEvenGroups : n;
+  return EvenParts{n, (uint32_t)((((uint64_t)row_groups + n - 1) / n + 7) / 8)};
+}
+
 // Rows row0 .. row0 + left - 1 (at most kEvenGroups groups) against query
 // group qbase.
-template <int QT, bool kPlane, bool kTri>
-__device__ __forceinline__ void even_part(EvenHits& H, const uint4* __restrict__ db, const uint4* __restrict__ plane,
+template <int QT, bool kPlane, bool kTri, uint32_t kList>
+__device__ __forceinline__ void even_part(HitList<kList>& H, const uint4* __restrict__ db, const uint4* __restrict__ plane,
                                           uint64_t n_rows, uint64_t row0, uint32_t left,
                                           const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t qbase,
                                           uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity,
@@ -931,20 +761,6 @@ __device__ __forceinline__ void even_part(EvenHits& H, const uint4* __restrict__
   }
 }
 
-// The block's gathered hits into the buffer.  Every thread of the block calls
-// it.
-__device__ __forceinline__ void even_flush(EvenHits& H, MatchHit* __restrict__ hits, uint64_t capacity,
-                                           unsigned long long* __restrict__ counter) {
-  __syncthreads();
-  const uint32_t n = min(H.n, kEvenStage);
-  if (n == 0) return;  // the same for the whole block
-  if (threadIdx.x == 0) H.base = atomicAdd(counter, (unsigned long long)n);
-  __syncthreads();
-  const unsigned long long base = H.base;
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
-    if (base + i < capacity) hits[base + i] = H.stage[i];
-}
-
 // One part per wave.  Part part_x * 8 + xcd: the waves that match one part
 // against the query groups are neighbours on one XCD and share its rows in the
 // caches.
@@ -954,9 +770,8 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
     const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t threshold, MatchHit* __restrict__ hits,
     uint64_t capacity, unsigned long long* __restrict__ counter, uint64_t index_base, uint32_t groups,
     uint32_t parts_per_xcd, uint32_t part_groups) {
-  __shared__ EvenHits H;
-  if (threadIdx.x == 0) H.n = 0;
-  __syncthreads();
+  __shared__ HitList<kEvenStage> H;
+  hits_init(H);
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t id = (blockIdx.x >> 3) * kMfmaWaves + wave;
   const uint32_t part_x = id / groups;
@@ -966,7 +781,7 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
                                 (uint32_t)min(n_rows - row0, (uint64_t)part_groups * kEvenRows), queries, n_queries,
                                 (id - part_x * groups) * (uint32_t)(QT * 16), threshold, hits, capacity, counter,
                                 index_base);
-  even_flush(H, hits, capacity, counter);
+  hits_flush(H, hits, capacity, counter);
 }
 
 // The second kernel of the shared-rows layout, in blocks of kResolveWaves
@@ -987,32 +802,13 @@ constexpr int kResolveWaves = 8;
 constexpr int kResolveBlocksPerCu = 2;
 
 uint32_t match_resolve_blocks(int cus) { return (uint32_t)std::max(1, cus) * kResolveBlocksPerCu; }
-static_assert(kResolveWaves % kMfmaWaves == 0, "whole per-wave items per block");
 
-struct ResolveLds {
-  MatchHit stage[kStageHits];
-  uint32_t n_stage;
-  unsigned long long stage_base;
-};
+using ResolveLds = HitList<kStageHits>;
 
-__device__ __forceinline__ void resolve_init(ResolveLds& L) {
-  if (threadIdx.x == 0) L.n_stage = 0;
-  __syncthreads();
-}
-
-// The block's gathered hits into the buffer: one run of slots.  Every thread
-// of the block calls it.
-__device__ __forceinline__ void resolve_flush(ResolveLds& L, MatchHit* __restrict__ hits, uint64_t capacity,
-                                              unsigned long long* __restrict__ counter) {
-  __syncthreads();
-  const uint32_t n = min(L.n_stage, kStageHits);
-  if (n == 0) return;  // the same for the whole block
-  if (threadIdx.x == 0) L.stage_base = atomicAdd(counter, (unsigned long long)n);
-  __syncthreads();
-  const unsigned long long base = L.stage_base;
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
-    if (base + i < capacity) hits[base + i] = L.stage[i];
-}
+// The rerun after an overflow: parts of kEvenGroups groups of rows against
+// groups of six query tiles, a wave each (eight leave one block per CU).
+constexpr int kRerunQt = 6;
+constexpr uint64_t kRerunRows = (uint64_t)kEvenGroups * kEvenRows;
 
 // The loads of one record part that do not depend on its products: the
 // query words of its tiles and the tile words of its first pending group.  A
@@ -1124,8 +920,8 @@ __device__ __forceinline__ void check_group(ResolveLds& L, const Expanded (&qa)[
 #pragma unroll
       for (int k = 1; k < QT; k++)
         if (t == k) a = qa[k];
-      stage_candidates<kStageHits>(mfma_prefix(a, eg), t, row0 + (uint64_t)tt * 16, qbase, rn, kq, bound, queries, db,
-                       n_queries, n_rows, threshold, L.stage, &L.n_stage, hits, capacity, counter, index_base);
+      stage_candidates(mfma_prefix(a, eg), t, row0 + (uint64_t)tt * 16, qbase, rn, kq, bound, queries, db, n_queries,
+                       n_rows, threshold, L, hits, capacity, counter, index_base);
     }
   }
 }
@@ -1201,25 +997,21 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_kernel(
     uint64_t capacity, unsigned long long* __restrict__ counter, uint64_t index_base,
     const uint4* __restrict__ recs, const uint32_t* __restrict__ rec_count, uint32_t rec_cap) {
   __shared__ ResolveLds L;
-  resolve_init(L);
+  hits_init(L);
   const int wave = (int)(threadIdx.x >> 6);
   const uint32_t n_recs = *rec_count;
   if (n_recs > rec_cap) {
-    // the per-wave layout, at most eight query tiles per wave
-    constexpr int kRq = kResolveQt<QT>;
-    const uint32_t rgroups = (n_queries + kRq * 16 - 1) / (kRq * 16);
-    constexpr int kHalves = kResolveWaves / kMfmaWaves;
-    constexpr uint64_t kChunkRows = (uint64_t)kMfmaWaves * kMfmaTilesPerWave * 16;
-    const uint64_t chunks = ((n_rows + kChunkRows - 1) / kChunkRows + 7) / 8 * 8;  // whole XCD rounds
-    const uint64_t items = chunks * rgroups;
-    for (uint64_t item = (uint64_t)blockIdx.x * kHalves + wave / kMfmaWaves; item < items;
-         item += (uint64_t)gridDim.x * kHalves) {
-      uint64_t chunk;
-      uint32_t group;
-      item_coords(item, rgroups, chunk, group);
-      mfma_item<kRq, kPlane>(db, plane, n_rows, chunk, group, queries, n_queries, threshold, hits, capacity,
-                             counter, index_base, wave % kMfmaWaves);
+    const uint32_t groups = (n_queries + kRerunQt * 16 - 1) / (kRerunQt * 16);
+    const uint64_t items = (n_rows + kRerunRows - 1) / kRerunRows * groups;
+    for (uint64_t item = (uint64_t)blockIdx.x * kResolveWaves + wave; item < items;
+         item += (uint64_t)gridDim.x * kResolveWaves) {
+      const uint64_t row0 = item / groups * kRerunRows;
+      even_part<kRerunQt, kPlane, false>(L, reinterpret_cast<const uint4*>(db), reinterpret_cast<const uint4*>(plane),
+                                         n_rows, row0, (uint32_t)min(n_rows - row0, kRerunRows), queries, n_queries,
+                                         (uint32_t)(item % groups) * (kRerunQt * 16), threshold, hits, capacity,
+                                         counter, index_base);
     }
+    hits_flush(L, hits, capacity, counter);
     return;
   }
   // The wave's records are w, w + S, w + 2S, ... (w its number in the
@@ -1268,7 +1060,7 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_kernel(
     rec_next = rec_after;
     P = Pn;
   }
-  resolve_flush(L, hits, capacity, counter);
+  hits_flush(L, hits, capacity, counter);
 }
 
 // The shard holding MFMA row chunk `chunk` (views in chunk order).
@@ -1285,15 +1077,15 @@ __device__ __forceinline__ uint32_t shard_of_chunk(const ShardView* __restrict__
 // kSubsPerChunk.  The query count is read from device memory (`d_nq`, capped
 // at nq_cap), so one captured launch serves batches of any size.  Records
 // carry the global sub-chunk number.
-template <int QT, bool kPlane, bool kTri = false>
-__global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(QT >= 16 ? 3 : 4))) pdq_match_mfma_shards_shared_kernel(
+template <bool kTri>
+__global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(4))) pdq_match_mfma_shards_shared_kernel(
     const ShardView* __restrict__ shards, uint32_t n_shards, uint64_t total_chunks,
     const uint32_t* __restrict__ queries, const uint32_t* __restrict__ d_nq, uint32_t nq_cap, uint32_t threshold,
     uint4* __restrict__ recs, uint32_t* __restrict__ rec_count, uint32_t rec_cap) {
   const uint32_t nq = d_nq ? min(*d_nq, nq_cap) : nq_cap;
   if (nq == 0) return;
   __shared__ SharedRowsLds S;
-  const uint32_t groups = (nq + QT * 16 - 1) / (QT * 16);
+  const uint32_t groups = (nq + kSharedQt * 16 - 1) / (kSharedQt * 16);
   const uint32_t sgroups = (groups + kMfmaWaves - 1) / kMfmaWaves;
   const uint64_t items = total_chunks * kSubsPerChunk * sgroups;
   for (uint64_t item = blockIdx.x; item < items; item += gridDim.x) {
@@ -1302,46 +1094,45 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
     item_coords(item, sgroups, gsub, sgroup);
     const ShardView& v = shards[shard_of_chunk(shards, n_shards, gsub / kSubsPerChunk)];
     const uint64_t sub_base = v.chunk_begin * kSubsPerChunk;
-    mfma_item_shared<QT, kPlane, kTri>(S, reinterpret_cast<const uint32_t*>(v.rows),
+    mfma_item_shared<kSharedQt, true, kTri>(S, reinterpret_cast<const uint32_t*>(v.rows),
                                        reinterpret_cast<const uint32_t*>(v.plane), v.n_rows, gsub - sub_base, sgroup,
                                        queries, nq, threshold, recs, rec_count, rec_cap, sub_base);
   }
 }
 
 // Its recheck kernel: as pdq_match_resolve_kernel, with each record's shard
-// found from its global sub-chunk, and the per-wave rerun after an overflow
-// walking the items of every shard.
-template <int QT, bool kPlane>
+// found from its global sub-chunk, and the rerun after an overflow walking
+// the parts of every shard.
 __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_shards_kernel(
-    const ShardView* __restrict__ shards, uint32_t n_shards, uint64_t total_chunks,
+    const ShardView* __restrict__ shards, uint32_t n_shards,
     const uint32_t* __restrict__ queries, const uint32_t* __restrict__ d_nq, uint32_t nq_cap, uint32_t threshold,
     MatchHit* __restrict__ hits, uint64_t capacity, unsigned long long* __restrict__ counter,
     const uint4* __restrict__ recs, const uint32_t* __restrict__ rec_count, uint32_t rec_cap) {
   const uint32_t nq = d_nq ? min(*d_nq, nq_cap) : nq_cap;
   if (nq == 0) return;
   __shared__ ResolveLds L;
-  resolve_init(L);
+  hits_init(L);
   const int wave = (int)(threadIdx.x >> 6);
   const uint32_t n_recs = *rec_count;
   if (n_recs > rec_cap) {
-    constexpr int kHalves = kResolveWaves / kMfmaWaves;
-    constexpr int kRq = kResolveQt<QT>;
-    const uint32_t groups = (nq + kRq * 16 - 1) / (kRq * 16);
-    const uint64_t items = total_chunks * groups;
-    for (uint64_t item = (uint64_t)blockIdx.x * kHalves + wave / kMfmaWaves; item < items;
-         item += (uint64_t)gridDim.x * kHalves) {
-      uint64_t chunk;
-      uint32_t group;
-      item_coords(item, groups, chunk, group);
-      const ShardView& v = shards[shard_of_chunk(shards, n_shards, chunk)];
-      mfma_item<kRq, kPlane>(reinterpret_cast<const uint32_t*>(v.rows),
-                            reinterpret_cast<const uint32_t*>(v.plane), v.n_rows, chunk - v.chunk_begin, group, queries,
-                            nq, threshold, hits, capacity, counter, v.index_base, wave % kMfmaWaves);
+    const uint32_t groups = (nq + kRerunQt * 16 - 1) / (kRerunQt * 16);
+    for (uint32_t sh = 0; sh < n_shards; sh++) {
+      const ShardView& v = shards[sh];
+      const uint64_t items = (v.n_rows + kRerunRows - 1) / kRerunRows * groups;
+      for (uint64_t item = (uint64_t)blockIdx.x * kResolveWaves + wave; item < items;
+           item += (uint64_t)gridDim.x * kResolveWaves) {
+        const uint64_t row0 = item / groups * kRerunRows;
+        even_part<kRerunQt, true, false>(L, v.rows, v.plane, v.n_rows, row0,
+                                           (uint32_t)min(v.n_rows - row0, kRerunRows), queries, nq,
+                                           (uint32_t)(item % groups) * (kRerunQt * 16), threshold, hits, capacity,
+                                           counter, v.index_base);
+      }
     }
+    hits_flush(L, hits, capacity, counter);
     return;
   }
   // whole records per wave, as in pdq_match_resolve_kernel
-  constexpr int kRq = kResolveQt<QT>, kParts = QT / kRq;
+  constexpr int kRq = kResolveQt<kSharedQt>, kParts = kSharedQt / kRq;
   const uint32_t stride = gridDim.x * kResolveWaves;
   uint32_t i = blockIdx.x * kResolveWaves + wave;
   uint4 rec = i < n_recs ? recs[i] : make_uint4(0, 0, 0, 0);
@@ -1357,41 +1148,58 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_shards_k
       const uint32_t qbase = rec.z + part * (kRq * 16);
       const uint32_t pending = part_groups<kParts>(rec.w, part);
       PartLoads<kRq> P;
-      part_load<kRq, kPlane>(P, rows, vplane, v.n_rows, row0, qbase, pending, queries, nq);
-      resolve_record<kRq, kPlane>(L, P, rows, vplane, v.n_rows, row0, qbase, pending, queries, nq, threshold, hits,
+      part_load<kRq, true>(P, rows, vplane, v.n_rows, row0, qbase, pending, queries, nq);
+      resolve_record<kRq, true>(L, P, rows, vplane, v.n_rows, row0, qbase, pending, queries, nq, threshold, hits,
                                   capacity, counter, v.index_base, [] {});
     }
     rec = next;
   }
-  resolve_flush(L, hits, capacity, counter);
+  hits_flush(L, hits, capacity, counter);
 }
 
-// Persistent form over a set of database shards: a fixed grid (a multiple of
-// 8 blocks) walks the work items of every shard, blockIdx.x + k * gridDim.x,
-// which keeps each item on the XCD its number selects.  The query count is
-// read from device memory (`d_nq`, capped at nq_cap), so one captured launch
-// serves batches of any size; batches of fewer than min_nq queries are left
-// to the vector-ALU kernel and this one returns at once.
-template <int QT, bool kPlane>
-__global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(QT >= 16 ? 3 : 4))) pdq_match_mfma_shards_kernel(
-    const ShardView* __restrict__ shards, uint32_t n_shards, uint64_t total_chunks,
-    const uint32_t* __restrict__ queries, const uint32_t* __restrict__ d_nq, uint32_t nq_cap, uint32_t min_nq,
-    uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity, unsigned long long* __restrict__ counter) {
+// The even layout over a set of shards.  The shards' row groups, one shard
+// after the other, are cut into parts as for one database; a part that crosses
+// a shard's end is matched piece by piece.  The query count is read from device
+// memory (`d_nq`, capped at nq_cap), so one captured launch of resident waves
+// serves batches of any size: every wave works out the parts from it.  The
+// matrix cores bound it as they do one database.  Before, a wave took 512-row
+// items of its own query group one after the other, with up to a group's
+// width of padding and a last round in which most waves had nothing left:
+// five shards, 26.1M rows together, with batches of 37 images (296 queries) took
+// 516 us and take 455, 100 images (800) 1136 and 908.
+template <int QT, bool kTri>
+__global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(4))) pdq_match_even_shards_kernel(
+    const ShardView* __restrict__ shards, uint32_t n_shards, uint32_t row_groups,
+    const uint32_t* __restrict__ queries, const uint32_t* __restrict__ d_nq, uint32_t nq_cap, uint32_t threshold,
+    MatchHit* __restrict__ hits, uint64_t capacity, unsigned long long* __restrict__ counter) {
   const uint32_t nq = d_nq ? min(*d_nq, nq_cap) : nq_cap;
-  if (nq == 0 || nq < min_nq) return;
+  if (nq == 0) return;
+  __shared__ HitList<kEvenStage> H;
+  hits_init(H);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t groups = (nq + QT * 16 - 1) / (QT * 16);
-  const uint64_t items = total_chunks * groups;
-  for (uint64_t item = blockIdx.x; item < items; item += gridDim.x) {
-    uint64_t chunk;
-    uint32_t group;
-    item_coords(item, groups, chunk, group);
+  const uint32_t waves_per_xcd = gridDim.x / 8 * kMfmaWaves;
+  const EvenParts parts = even_parts(row_groups, groups, waves_per_xcd);
+  for (uint32_t id = (blockIdx.x >> 3) * kMfmaWaves + wave;; id += waves_per_xcd) {
+    const uint32_t part_x = id / groups;
+    if (part_x >= parts.per_xcd) break;
+    const uint64_t first = ((uint64_t)part_x * 8 + (blockIdx.x & 7)) * parts.groups;
+    uint32_t g = (uint32_t)min(first, (uint64_t)row_groups);
+    const uint32_t end = (uint32_t)min(first + parts.groups, (uint64_t)row_groups);
     uint32_t sh = 0;
-    while (sh + 1 < n_shards && shards[sh + 1].chunk_begin <= chunk) sh++;
-    const ShardView& v = shards[sh];
-    mfma_item<QT, kPlane>(reinterpret_cast<const uint32_t*>(v.rows), reinterpret_cast<const uint32_t*>(v.plane),
-                          v.n_rows, chunk - v.chunk_begin, group, queries, nq, threshold, hits, capacity, counter,
-                          v.index_base, (int)(threadIdx.x >> 6));
+    while (g < end) {
+      while (sh + 1 < n_shards && shards[sh + 1].group_begin <= g) sh++;
+      const ShardView& v = shards[sh];
+      const uint32_t stop = sh + 1 < n_shards ? min(end, (uint32_t)shards[sh + 1].group_begin) : end;
+      const uint64_t row0 = (g - v.group_begin) * kEvenRows;
+      even_part<QT, true, kTri>(H, v.rows, v.plane, v.n_rows, row0,
+                                (uint32_t)min(v.n_rows - row0, (uint64_t)(stop - g) * kEvenRows), queries, nq,
+                                (id - part_x * groups) * (uint32_t)(QT * 16), threshold, hits, capacity, counter,
+                                v.index_base);
+      g = stop;
+    }
   }
+  hits_flush(H, hits, capacity, counter);
 }
 
 // Record areas of the shared-rows layout: one per (device, stream), made on
@@ -1590,9 +1398,26 @@ static hipError_t launch_shared(const void* db, const void* plane, uint64_t n_ro
   return e;
 }
 
-// The even layout's launch.  Its waves all fit the chip at once (four per
-// SIMD), and the rows are cut into as many equal parts as that leaves per
-// query group, in whole rounds of loads.
+// f(integral_constant<int, qt>()) for the widths the even layout is built for.
+template <class F>
+static hipError_t with_query_tiles(int qt, F&& f) {
+  switch (qt) {
+    case 2: return f(std::integral_constant<int, 2>());
+    case 4: return f(std::integral_constant<int, 4>());
+    case 6: return f(std::integral_constant<int, 6>());
+    case 8: return f(std::integral_constant<int, 8>());
+    case 10: return f(std::integral_constant<int, 10>());
+    case 12: return f(std::integral_constant<int, 12>());
+    case 14: return f(std::integral_constant<int, 14>());
+    case 16: return f(std::integral_constant<int, 16>());
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// The even layout's waves that are resident at once: four per SIMD.
+static uint32_t even_waves_per_xcd(int cus) { return (uint32_t)std::max(1, cus) * 16 / 8; }
+
+// The even layout's launch.
 template <int QT>
 static hipError_t launch_even(const void* db, const void* plane, uint64_t n_rows, const void* queries,
                               uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
@@ -1603,22 +1428,18 @@ static hipError_t launch_even(const void* db, const void* plane, uint64_t n_rows
   if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
   const uint32_t groups = (n_queries + QT * 16 - 1) / (QT * 16);
   const uint64_t row_groups = (n_rows + kEvenRows - 1) / kEvenRows;
-  const uint64_t waves_per_xcd = std::max(1, cus) * 16 / 8;
-  const uint64_t round = 8 * std::max<uint64_t>(1, waves_per_xcd / groups);  // parts resident at once
-  const uint64_t rounds = (row_groups + round * kEvenGroups - 1) / (round * kEvenGroups);
-  uint64_t part_groups = (row_groups + round * rounds - 1) / (round * rounds);
-  part_groups = std::min<uint64_t>(kEvenGroups, (part_groups + kEvenRound - 1) / kEvenRound * kEvenRound);
-  const uint64_t parts_per_xcd = ((row_groups + part_groups - 1) / part_groups + 7) / 8;
-  const uint64_t blocks = 8 * ((parts_per_xcd * groups + kMfmaWaves - 1) / kMfmaWaves);
-  if (blocks > 0x7fffffffull || parts_per_xcd * groups > 0xffffffffull) return hipErrorInvalidValue;
+  if (row_groups > 0xffffffffull) return hipErrorInvalidValue;
+  const EvenParts parts = even_parts((uint32_t)row_groups, groups, even_waves_per_xcd(cus));
+  const uint64_t waves = (uint64_t)parts.per_xcd * groups;  // per XCD
+  const uint64_t blocks = 8 * ((waves + kMfmaWaves - 1) / kMfmaWaves);
+  if (blocks > 0x7fffffffull || waves > 0xffffffffull) return hipErrorInvalidValue;
   if (reset) hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(1), 0, stream, nullptr, counter);
   const bool tri = QT > 2 && threshold >= kTriMinThreshold;
   auto launch = [&](auto pl, auto tr) {
     hipLaunchKernelGGL((pdq_match_even_kernel<QT, decltype(pl)::value, decltype(tr)::value>), dim3((unsigned)blocks),
                        dim3(64 * kMfmaWaves), 0, stream, static_cast<const uint4*>(db),
                        static_cast<const uint4*>(plane), n_rows, static_cast<const uint32_t*>(queries), n_queries,
-                       threshold, hits, capacity, counter, index_base, groups, (uint32_t)parts_per_xcd,
-                       (uint32_t)part_groups);
+                       threshold, hits, capacity, counter, index_base, groups, parts.per_xcd, parts.groups);
   };
   using T = std::integral_constant<bool, true>;
   using F = std::integral_constant<bool, false>;
@@ -1656,93 +1477,62 @@ uint64_t mfma_chunks(uint64_t n_rows) {
 }
 
 template <int QT>
-static hipError_t launch_shards_qt(const ShardView* shards, uint32_t n_shards, uint64_t total_chunks, bool plane,
-                                   const void* queries, const uint32_t* d_nq, uint32_t nq_cap, uint32_t min_nq,
-                                   uint32_t threshold, MatchHit* hits, uint64_t capacity, unsigned long long* counter,
-                                   uint32_t grid, hipStream_t stream) {
-  if (plane)
-    hipLaunchKernelGGL((pdq_match_mfma_shards_kernel<QT, true>), dim3(grid), dim3(64 * kMfmaWaves), 0, stream, shards,
-                       n_shards, total_chunks, static_cast<const uint32_t*>(queries), d_nq, nq_cap, min_nq, threshold,
-                       hits, capacity, counter);
+static hipError_t launch_even_shards(const ShardView* shards, uint32_t n_shards, uint64_t row_groups,
+                                     const void* queries, const uint32_t* d_nq, uint32_t nq_cap, uint32_t threshold,
+                                     MatchHit* hits, uint64_t capacity, unsigned long long* counter, int cus,
+                                     hipStream_t stream) {
+  // resident blocks, fewer where the largest batch has fewer parts
+  const uint32_t groups = (nq_cap + QT * 16 - 1) / (QT * 16);
+  const EvenParts parts = even_parts((uint32_t)row_groups, groups ? groups : 1, even_waves_per_xcd(cus));
+  const uint64_t most = ((uint64_t)parts.per_xcd * groups + kMfmaWaves - 1) / kMfmaWaves;
+  const uint64_t per_xcd = std::max<uint64_t>(1, std::min<uint64_t>(even_waves_per_xcd(cus) / kMfmaWaves, most));
+  const dim3 grid((unsigned)(8 * per_xcd)), block(64 * kMfmaWaves);
+  const uint32_t* q = static_cast<const uint32_t*>(queries);
+  if (QT > 2 && threshold >= kTriMinThreshold)
+    hipLaunchKernelGGL((pdq_match_even_shards_kernel<QT, true>), grid, block, 0, stream, shards, n_shards,
+                       (uint32_t)row_groups, q, d_nq, nq_cap, threshold, hits, capacity, counter);
   else
-    hipLaunchKernelGGL((pdq_match_mfma_shards_kernel<QT, false>), dim3(grid), dim3(64 * kMfmaWaves), 0, stream,
-                       shards, n_shards, total_chunks, static_cast<const uint32_t*>(queries), d_nq, nq_cap, min_nq,
-                       threshold, hits, capacity, counter);
+    hipLaunchKernelGGL((pdq_match_even_shards_kernel<QT, false>), grid, block, 0, stream, shards, n_shards,
+                       (uint32_t)row_groups, q, d_nq, nq_cap, threshold, hits, capacity, counter);
   return hipGetLastError();
 }
 
-hipError_t launch_match_mfma_shards(int qt, const ShardView* shards, uint32_t n_shards, uint64_t total_chunks,
-                                    bool plane, const void* queries, const uint32_t* d_nq, uint32_t nq_cap,
-                                    uint32_t min_nq, uint32_t threshold, MatchHit* hits, uint64_t capacity,
-                                    unsigned long long* counter, uint32_t grid, hipStream_t stream) {
-  if (threshold >= 64 || grid == 0 || grid % 8) return hipErrorInvalidValue;
-  switch (qt) {
-    case 2: return launch_shards_qt<2>(shards, n_shards, total_chunks, plane, queries, d_nq, nq_cap, min_nq, threshold,
-                                       hits, capacity, counter, grid, stream);
-    case 4: return launch_shards_qt<4>(shards, n_shards, total_chunks, plane, queries, d_nq, nq_cap, min_nq, threshold,
-                                       hits, capacity, counter, grid, stream);
-    case 8: return launch_shards_qt<8>(shards, n_shards, total_chunks, plane, queries, d_nq, nq_cap, min_nq, threshold,
-                                       hits, capacity, counter, grid, stream);
-    case 16: return launch_shards_qt<16>(shards, n_shards, total_chunks, plane, queries, d_nq, nq_cap, min_nq,
-                                         threshold, hits, capacity, counter, grid, stream);
-    default: return hipErrorInvalidValue;
-  }
+hipError_t launch_match_even_shards(int qt, const ShardView* shards, uint32_t n_shards, uint64_t row_groups,
+                                    const void* queries, const uint32_t* d_nq, uint32_t nq_cap, uint32_t threshold,
+                                    MatchHit* hits, uint64_t capacity, unsigned long long* counter, int cus,
+                                    hipStream_t stream) {
+  if (threshold >= 64 || row_groups > 0xffffffffull) return hipErrorInvalidValue;
+  return with_query_tiles(qt, [&](auto q) {
+    return launch_even_shards<decltype(q)::value>(shards, n_shards, row_groups, queries, d_nq, nq_cap, threshold,
+                                                  hits, capacity, counter, cus, stream);
+  });
 }
+
+uint64_t match_row_groups(uint64_t n_rows) { return (n_rows + kEvenRows - 1) / kEvenRows; }
 
 uint64_t match_record_area_bytes() { return (uint64_t)kRecordCap * sizeof(uint4) + 256; }
 
-template <int QT>
-static hipError_t launch_shards_shared_qt(const ShardView* shards, uint32_t n_shards, uint64_t total_chunks,
-                                          bool plane, const void* queries, const uint32_t* d_nq, uint32_t nq_cap,
-                                          uint32_t threshold, MatchHit* hits, uint64_t capacity,
-                                          unsigned long long* counter, void* area, uint32_t grid, uint32_t rgrid,
-                                          hipStream_t stream) {
-  uint4* recs = static_cast<uint4*>(area);
-  uint32_t* count = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(area) + (size_t)kRecordCap * sizeof(uint4));
+hipError_t launch_match_shared_shards(const ShardView* shards, uint32_t n_shards, uint64_t total_chunks,
+                                      const void* queries, const uint32_t* d_nq, uint32_t nq_cap, uint32_t threshold,
+                                      MatchHit* hits, uint64_t capacity, unsigned long long* counter,
+                                      void* record_area, uint32_t grid, uint32_t rgrid, hipStream_t stream) {
+  if (threshold >= 64 || grid == 0 || grid % 8 || rgrid == 0 || !record_area) return hipErrorInvalidValue;
+  uint4* recs = static_cast<uint4*>(record_area);
+  uint32_t* count =
+      reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(record_area) + (size_t)kRecordCap * sizeof(uint4));
   const uint32_t* q = static_cast<const uint32_t*>(queries);
   const dim3 block(64 * kMfmaWaves), rblock(64 * kResolveWaves);
   const uint32_t cap = record_cap();
   hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(1), 0, stream, count, nullptr);
-  const bool tri = QT == 16 && threshold >= kTriMinThreshold;  // three products per accumulator
-  if (plane) {
-    if (tri)
-      hipLaunchKernelGGL((pdq_match_mfma_shards_shared_kernel<QT, true, QT == 16>), dim3(grid), block, 0, stream,
-                         shards, n_shards, total_chunks, q, d_nq, nq_cap, threshold, recs, count, cap);
-    else
-      hipLaunchKernelGGL((pdq_match_mfma_shards_shared_kernel<QT, true>), dim3(grid), block, 0, stream, shards,
-                         n_shards, total_chunks, q, d_nq, nq_cap, threshold, recs, count, cap);
-    hipLaunchKernelGGL((pdq_match_resolve_shards_kernel<QT, true>), dim3(rgrid), rblock, 0, stream, shards, n_shards,
-                       total_chunks, q, d_nq, nq_cap, threshold, hits, capacity, counter, recs, count, cap);
-  } else {
-    if (tri)
-      hipLaunchKernelGGL((pdq_match_mfma_shards_shared_kernel<QT, false, QT == 16>), dim3(grid), block, 0, stream,
-                         shards, n_shards, total_chunks, q, d_nq, nq_cap, threshold, recs, count, cap);
-    else
-      hipLaunchKernelGGL((pdq_match_mfma_shards_shared_kernel<QT, false>), dim3(grid), block, 0, stream, shards,
-                         n_shards, total_chunks, q, d_nq, nq_cap, threshold, recs, count, cap);
-    hipLaunchKernelGGL((pdq_match_resolve_shards_kernel<QT, false>), dim3(rgrid), rblock, 0, stream, shards, n_shards,
-                       total_chunks, q, d_nq, nq_cap, threshold, hits, capacity, counter, recs, count, cap);
-  }
+  if (threshold >= kTriMinThreshold)  // three products per accumulator
+    hipLaunchKernelGGL((pdq_match_mfma_shards_shared_kernel<true>), dim3(grid), block, 0, stream, shards, n_shards,
+                       total_chunks, q, d_nq, nq_cap, threshold, recs, count, cap);
+  else
+    hipLaunchKernelGGL((pdq_match_mfma_shards_shared_kernel<false>), dim3(grid), block, 0, stream, shards, n_shards,
+                       total_chunks, q, d_nq, nq_cap, threshold, recs, count, cap);
+  hipLaunchKernelGGL(pdq_match_resolve_shards_kernel, dim3(rgrid), rblock, 0, stream, shards, n_shards, q, d_nq,
+                     nq_cap, threshold, hits, capacity, counter, recs, count, cap);
   return hipGetLastError();
-}
-
-hipError_t launch_match_mfma_shards_shared(int qt, const ShardView* shards, uint32_t n_shards, uint64_t total_chunks,
-                                           bool plane, const void* queries, const uint32_t* d_nq, uint32_t nq_cap,
-                                           uint32_t threshold, MatchHit* hits, uint64_t capacity,
-                                           unsigned long long* counter, void* record_area, uint32_t grid,
-                                           uint32_t rgrid, hipStream_t stream) {
-  if (threshold >= 64 || grid == 0 || grid % 8 || rgrid == 0 || !record_area) return hipErrorInvalidValue;
-  switch (qt) {
-    case 2: return launch_shards_shared_qt<2>(shards, n_shards, total_chunks, plane, queries, d_nq, nq_cap, threshold,
-                                              hits, capacity, counter, record_area, grid, rgrid, stream);
-    case 4: return launch_shards_shared_qt<4>(shards, n_shards, total_chunks, plane, queries, d_nq, nq_cap, threshold,
-                                              hits, capacity, counter, record_area, grid, rgrid, stream);
-    case 8: return launch_shards_shared_qt<8>(shards, n_shards, total_chunks, plane, queries, d_nq, nq_cap, threshold,
-                                              hits, capacity, counter, record_area, grid, rgrid, stream);
-    case 16: return launch_shards_shared_qt<16>(shards, n_shards, total_chunks, plane, queries, d_nq, nq_cap,
-                                                threshold, hits, capacity, counter, record_area, grid, rgrid, stream);
-    default: return hipErrorInvalidValue;
-  }
 }
 
 bool match_mfma_applicable(uint32_t n_queries, uint32_t threshold) { return threshold < 64 && n_queries >= 32; }
@@ -1758,15 +1548,11 @@ bool match_mfma_applicable(uint32_t n_queries, uint32_t threshold) { return thre
 // its groups and the rows are many (64 tiles: 338 against 348 us at 10^7 rows,
 // 48 against 48 at 10^6, 35 against 17 at 10^5; 128 tiles: 83 against 88 us at
 // 10^6, 46 against 28 at 10^5).
-struct MatchPlan {
-  bool shared;
-  int qt;  // of the even layout
-};
 constexpr int kEvenCost = 27;
 constexpr int kSharedCost = 733;
 constexpr uint64_t kSharedGain = 30000000;  // rows x cost units that pay for the recheck
 
-static MatchPlan match_plan(uint64_t n_rows, uint32_t n_queries) {
+MatchPlan match_plan(uint64_t n_rows, uint32_t n_queries) {
   const uint64_t tiles = ((uint64_t)n_queries + 15) / 16;
   MatchPlan plan{false, 2};
   uint64_t best = ~0ull;
@@ -1799,20 +1585,10 @@ static hipError_t launch_match_mfma_any(const void* db, const void* plane, uint6
                                        index_base, stream, reset_counter, fixed, &done);
     if (e != hipSuccess || done) return e;
   }
-  auto even = [&](auto qt) {
+  return with_query_tiles(plan.qt, [&](auto qt) {
     return launch_even<decltype(qt)::value>(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter,
                                             index_base, stream, reset_counter);
-  };
-  switch (plan.qt) {
-    case 2: return even(std::integral_constant<int, 2>());
-    case 4: return even(std::integral_constant<int, 4>());
-    case 6: return even(std::integral_constant<int, 6>());
-    case 8: return even(std::integral_constant<int, 8>());
-    case 10: return even(std::integral_constant<int, 10>());
-    case 12: return even(std::integral_constant<int, 12>());
-    case 14: return even(std::integral_constant<int, 14>());
-    default: return even(std::integral_constant<int, 16>());
-  }
+  });
 }
 
 hipError_t launch_match_mfma(const void* db, const void* plane, uint64_t n_rows, const void* queries,
