@@ -62,8 +62,8 @@ __device__ __forceinline__ v4f mfma_prefix(const Expanded& a, const Expanded& b)
   v8i av = {(int)a.d[0], (int)a.d[1], (int)a.d[2], (int)a.d[3], 0, 0, 0, 0};
   v8i bv = {(int)b.d[0], (int)b.d[1], (int)b.d[2], (int)b.d[3], 0, 0, 0, 0};
   v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
-  // cbsz = blgp = 4: both operands fp4 e2m1; scales 127 = 2^0
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 4, 4, 0, 127, 0, 127);
+  // cbsz = blgp = 4: both operands fp4 e2m1; no scales
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 4, 4, 0, 0, 0, 0);
 }
 
 __device__ __forceinline__ uint32_t full_distance(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b) {
@@ -165,11 +165,19 @@ __device__ __forceinline__ v4f flags_c0(float bound) {
   return v4f{c, c, c, c};
 }
 
+// A scale of one is left out: zero for both scale operands is the product
+// without them, whose issue costs one vector instruction less (16x16x128
+// products beside two vector instructions each: 19.8 against 23.4 cycles; 10^7
+// rows against 1000 queries 347 us with it, 336 without, 200 queries 90.1 and
+// 87.8).
 template <int kScaleA>
 __device__ __forceinline__ v4f mfma_acc(const Expanded& a, const Expanded& b, const v4f& c) {
   v8i av = {(int)a.d[0], (int)a.d[1], (int)a.d[2], (int)a.d[3], 0, 0, 0, 0};
   v8i bv = {(int)b.d[0], (int)b.d[1], (int)b.d[2], (int)b.d[3], 0, 0, 0, 0};
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 4, 4, 0, kScaleA, 0, kScale1);
+  if constexpr (kScaleA == kScale1)
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 4, 4, 0, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 4, 4, 0, kScaleA, 0, kScale1);
 }
 
 // The empty asm pins m here: without it the compiler gathers every fold of a
