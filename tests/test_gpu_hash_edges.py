@@ -66,3 +66,25 @@ def test_ref_passes(gpu, oracle, dev, n):
             assert same(f[k], P), where
             assert np.array_equal(h[k], H), where
             assert same(q[k], Q) and same(t[k], T), where
+
+
+# the scales take the threshold search's sums from subnormal over the range of
+# its short division to infinity; 127 and 120 overflow in the DCT
+@pytest.mark.parametrize("exponent", [None, -165, -150, -140, -120, -100, -95, -60, 0, 60, 85, 95, 110, 120, 127])
+def test_threshold_search_at_all_scales(gpu, oracle, dev, exponent):
+    import torch
+    planes = synthetic.images_u8(3, start=90).astype(np.float32)
+    planes -= np.float32(128)
+    planes[2] = np.abs(planes[2])
+    planes *= np.float32(2.0 ** -7)
+    planes = np.zeros_like(planes) if exponent is None else np.ldexp(planes, exponent).astype(np.float32)
+    if exponent is not None and exponent < -126:
+        planes = np.abs(planes)  # a zero's sign may differ with negative subnormals
+    x = torch.from_numpy(planes).to(dev)
+    want = [oracle.hash_dihedrals(p, 1) for p in planes]
+    for layout in (gpu.LAYOUT_BLOCK4, gpu.LAYOUT_BLOCK8, gpu.LAYOUT_BLOCK16):
+        h, q, t = (y.cpu().numpy() for y in gpu.hash_batch(x, layout=layout))
+        for k, (H, Q, T, _) in enumerate(want):
+            where = f"layout {layout}, 2^{exponent}, image {k}"
+            assert np.array_equal(h[k], H), where
+            assert same(q[k], Q) and same(t[k], T), where

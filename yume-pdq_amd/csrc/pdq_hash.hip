@@ -99,9 +99,9 @@ __device__ __forceinline__ void stream_step(const T* __restrict__ plane, int lan
     chains_start(nxt, x2, x3);
   }
   float c0, c1;
-  chains_finish(cur, c0, c1);
-  // lane 63's second value is no output (column 127): its neighbour's sums
-  // come from lane 63 itself
+  // u8 with one step of prefetch: blocks of sixteen waves
+  chains_finish<std::is_same<T, uint8_t>::value && D == 1>(cur, c0, c1);
+  // lane 63's second value is no output (column 127): it has no neighbour
   if constexpr (std::is_same<T, float>::value) z = __builtin_fmaf(c0, c1, z);
   if (buf1) {
     buf1[i * 128 + 2 * lane] = c0;

@@ -9,18 +9,17 @@
 //      lane t owns output columns 2t and 2t+1) and stores them in LDS as a
 //      128x128 f32 plane whose row and column 127 are zero.
 //   B. DCT stage 1, T = D C (16 x 128).
-//        exact:        thread (column j, group of frequencies) runs the
-//                      reference's two alternating FMA chains over
-//                      k2 = 0..126 (x86.rs:161-225) -- the chains, operands
-//                      and order of the wave form, so the values are the
-//                      same bits;
+//        exact:        v_mfma_f32_16x16x4_f32 runs the reference's two
+//                      alternating FMA chains over k2 = 0..126
+//                      (x86.rs:161-225) -- the chains, operands and order of
+//                      the wave form, so the values are the same bits;
 //        matrix cores: v_mfma_f32_16x16x32_{bf16,f16}, operands rounded to
 //                      bf16 or f16 (round to nearest even) with f32
 //                      accumulation, or the three products hi*hi + hi*lo +
 //                      lo*hi of split operands x = hi + lo.
-//   C. stage 2 (exact: x86.rs:227-272, one column of each quad per wave;
-//      matrix cores: four 16x16x32 products on wave 0), then the shared tail
-//      (dihedrals, gradients, median search, bits) on wave 0.
+//   C. stage 2 (exact: x86.rs:227-272, two AVX lanes per wave on four waves;
+//      rounded: four 16x16x32 products on wave 0), then the dihedrals on every
+//      wave, and the thresholds and bits beside the qualities.
 // Planes holding NaN/Inf take the literal 56-tap compression and the exact
 // stage 1 in every form.
 #include <hip/hip_runtime.h>
@@ -35,9 +34,12 @@ namespace ypdq {
 
 namespace {
 
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
 struct ImageTail {
   WaveLds w;
-  float d2[16 * kTS];  // DCT rows, stride kTS
+  float part[4][256];           // stage 2: the four pairs of AVX lanes
+  float grad[8 * kGradStride];  // absolute differences of the eight orientations
 };
 
 struct ImageLds {
@@ -45,7 +47,7 @@ struct ImageLds {
     float c[128 * 128];  // compressed plane, row-major, stride 128
     ImageTail tail;      // after stage 1
   } u;
-  float dct_t[127 * 16];  // exact stage 1: D transposed, dct_t[k2 * 16 + k] = D[k][k2]
+  float dct_t[128 * 16];  // exact stages: D transposed, dct_t[k2 * 16 + k] = D[k][k2], row 127 zero
 };
 
 // Rows in flight per wave in the band loop: D compressed-row steps of four
@@ -62,7 +64,7 @@ struct BandPrefetch<uint8_t> {
 // ---------------------------------------------------------------------------
 // A. compression of one band of rows into LDS
 // ---------------------------------------------------------------------------
-template <int S, int D, typename T, typename Raw>
+template <int S, int D, bool kScalar, typename T, typename Raw>
 __device__ __forceinline__ void band_step(const T* __restrict__ plane, int lane, int i, int i_end, Chains& cur,
                                           Chains& nxt, Raw (&pre)[D][4], float* __restrict__ c, const Luma& lc,
                                           float& z) {
@@ -78,31 +80,31 @@ __device__ __forceinline__ void band_step(const T* __restrict__ plane, int lane,
     // (a copy out of the slot would cost eight moves per row)
     chains_feed<2>(cur, pre[S][0]);
     check_edges(z, pre[S][0]);
-    load_raw(plane, row(0), lane, pre[S][0]);
+    load_raw<kScalar>(plane, row(0), lane, pre[S][0]);
     chains_feed<3>(cur, pre[S][1]);
     check_edges(z, pre[S][1]);
-    load_raw(plane, row(1), lane, pre[S][1]);
+    load_raw<kScalar>(plane, row(1), lane, pre[S][1]);
     chains_feed<4>(cur, pre[S][2]);
     check_edges(z, pre[S][2]);
     chains_feed<5>(cur, pre[S][3]);
     check_edges(z, pre[S][3]);
     chains_start(nxt, pre[S][2], pre[S][3]);
-    load_raw(plane, row(2), lane, pre[S][2]);
-    load_raw(plane, row(3), lane, pre[S][3]);
+    load_raw<kScalar>(plane, row(2), lane, pre[S][2]);
+    load_raw<kScalar>(plane, row(3), lane, pre[S][3]);
   } else {
     // converted rows free their slots at once
     Row8 x, x2, x3;
     to_f32(pre[S][0], x, lc);
-    load_raw(plane, row(0), lane, pre[S][0]);
+    load_raw<kScalar>(plane, row(0), lane, pre[S][0]);
     chains_feed<2>(cur, x);
     to_f32(pre[S][1], x, lc);
-    load_raw(plane, row(1), lane, pre[S][1]);
+    load_raw<kScalar>(plane, row(1), lane, pre[S][1]);
     chains_feed<3>(cur, x);
     to_f32(pre[S][2], x2, lc);
-    load_raw(plane, row(2), lane, pre[S][2]);
+    load_raw<kScalar>(plane, row(2), lane, pre[S][2]);
     chains_feed<4>(cur, x2);
     to_f32(pre[S][3], x3, lc);
-    load_raw(plane, row(3), lane, pre[S][3]);
+    load_raw<kScalar>(plane, row(3), lane, pre[S][3]);
     chains_feed<5>(cur, x3);
     chains_start(nxt, x2, x3);
   }
@@ -117,23 +119,23 @@ __device__ __forceinline__ void band_step(const T* __restrict__ plane, int lane,
 // chains are the current ones of the step after), so no step copies them.
 // kAll: every step runs (no test, so the ring's registers stay fixed);
 // otherwise the steps up to the band's end.
-template <int S, int D, bool kAll, typename T, typename Raw>
+template <int S, int D, bool kAll, bool kScalar, typename T, typename Raw>
 __device__ __forceinline__ void band_steps(const T* __restrict__ plane, int lane, int i, int i_end, Chains& a,
                                            Chains& b, Raw (&pre)[D][4], float* __restrict__ c, const Luma& lc,
                                            float& z) {
   static_assert(D % 2 == 0, "an even number of steps returns the chain sets to their roles");
   if (kAll || i + S < i_end) {
     if constexpr (S % 2 == 0)
-      band_step<S, D>(plane, lane, i + S, i_end, a, b, pre, c, lc, z);
+      band_step<S, D, kScalar>(plane, lane, i + S, i_end, a, b, pre, c, lc, z);
     else
-      band_step<S, D>(plane, lane, i + S, i_end, b, a, pre, c, lc, z);
+      band_step<S, D, kScalar>(plane, lane, i + S, i_end, b, a, pre, c, lc, z);
   }
-  if constexpr (S + 1 < D) band_steps<S + 1, D, kAll>(plane, lane, i, i_end, a, b, pre, c, lc, z);
+  if constexpr (S + 1 < D) band_steps<S + 1, D, kAll, kScalar>(plane, lane, i, i_end, a, b, pre, c, lc, z);
 }
 
 // Compressed rows [i0, i1) into c; true if an input value that the reference
 // reads for them is NaN or Inf (f32 planes).
-template <typename T>
+template <bool kScalar, typename T>
 __device__ __forceinline__ bool compress_band(const T* __restrict__ plane, int lane, int i0, int i1,
                                               float* __restrict__ c, const Luma& lc) {
   using Raw = typename RawRow<T>::type;
@@ -143,12 +145,12 @@ __device__ __forceinline__ bool compress_band(const T* __restrict__ plane, int l
   float z = 0.0f;
   {
     Raw r1, r2;
-    load_raw(plane, 4 * i0 + 1, lane, r1);
-    load_raw(plane, 4 * i0 + 2, lane, r2);
+    load_raw<kScalar>(plane, 4 * i0 + 1, lane, r1);
+    load_raw<kScalar>(plane, 4 * i0 + 2, lane, r2);
 #pragma unroll
     for (int s = 0; s < D; s++)
 #pragma unroll
-      for (int d = 0; d < 4; d++) load_raw(plane, min(4 * (i0 + s) + 3 + d, 511), lane, pre[s][d]);
+      for (int d = 0; d < 4; d++) load_raw<kScalar>(plane, min(4 * (i0 + s) + 3 + d, 511), lane, pre[s][d]);
     Row8 x1, x2;
     to_f32(r1, x1, lc);
     to_f32(r2, x2, lc);
@@ -162,93 +164,89 @@ __device__ __forceinline__ bool compress_band(const T* __restrict__ plane, int l
       }
       if (i1 == 127) {
         Row8 last;
-        load_row(plane, 511, lane, last);
+        load_row<kScalar>(plane, 511, lane, last);
         check_row(z, last);
       }
     }
   }
   int i = i0;
 #pragma unroll 1
-  for (; i + D <= i1; i += D) band_steps<0, D, true>(plane, lane, i, i1, cur, nxt, pre, c, lc, z);
-  if (i < i1) band_steps<0, D, false>(plane, lane, i, i1, cur, nxt, pre, c, lc, z);
+  for (; i + D <= i1; i += D) band_steps<0, D, true, kScalar>(plane, lane, i, i1, cur, nxt, pre, c, lc, z);
+  if (i < i1) band_steps<0, D, false, kScalar>(plane, lane, i, i1, cur, nxt, pre, c, lc, z);
   return nonfinite(z);
 }
 
 // ---------------------------------------------------------------------------
-// B. stage 1, exact: thread (column j, frequencies k0 .. k0+NK-1).
+// B. stage 1 and 2, exact, on matrix cores.
+//
+// v_mfma_f32_16x16x4_f32 is four fused multiply-adds in order of k, each
+// rounded to nearest even, subnormals, infinities and NaN included (checked
+// against fmaf chains), so the reference's FMA chains run on it as they are,
+// four terms an instruction: lane l supplies A[l%16][l/16] and B[l/16][l%16]
+// and receives D[4 (l/16) + r][l%16], r = 0..3.  On the vector ALU stage 1 was
+// bound by issue and LDS, 508 FMAs a wave on eight waves (of one u8 image's
+// 40000 cycles stage 1 with its barriers took 8400 and takes 4600, stage 2 1800
+// and 1600).  One u8 plane 16.9 -> 14.9 us in all, 1000 planes 70.1 -> 63.6.
 // ---------------------------------------------------------------------------
-// The plane and the transposed DCT both sit in LDS, so every operand load is
-// an LDS load (those complete in order) and the loads of the next chunk of
-// rows are issued before the FMAs of the current one.
-template <int NK>
-struct DctSlice {
-  float v[NK];
-};
+// The term of chain p (alt()) that lane group g supplies to its step s: chain
+// 1 takes terms 0, 3, 4, 7, 8, .., chain 0 terms 1, 2, 5, 6, 9, ...
+__device__ __forceinline__ int chain_term(int p, int s, int g) {
+  const int even = g & 2;  // the first or second pair of four terms
+  return 8 * s + 2 * even + (p == 1 ? (g & 1) * 3 : 1 + (g & 1));
+}
 
-template <int NK>
-__device__ __forceinline__ void load_slice(const float* __restrict__ p, DctSlice<NK>& s) {
-  if constexpr (NK % 4 == 0) {
+// T[:, 16 jt .. 16 jt + 15] = D C: the two chains over k2 = 0..126
+// (x86.rs:161-225; term 127 is zero on both sides), then their sum, a chain's
+// NaN as zero, column 127 zero.  c: the plane, dt: the transposed DCT.
+__device__ __forceinline__ f32x4v stage1_exact(const float* __restrict__ c, const float* __restrict__ dt, int lane,
+                                               int jt) {
+  const int m = lane & 15, g = lane >> 4;
+  f32x4v acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
 #pragma unroll
-    for (int q = 0; q < NK / 4; q++) {
-      const f32x4 v = reinterpret_cast<const f32x4*>(p)[q];
-      s.v[4 * q] = v.x; s.v[4 * q + 1] = v.y; s.v[4 * q + 2] = v.z; s.v[4 * q + 3] = v.w;
+  for (int s = 0; s < 16; s++) {
+#pragma unroll
+    for (int p = 1; p >= 0; p--) {
+      const int k = chain_term(p, s, g);
+      acc[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(dt[k * 16 + m], c[k * 128 + 16 * jt + m], acc[p], 0, 0, 0);
     }
-  } else {
-    static_assert(NK == 2, "two, four or eight frequencies per thread");
-    const float2 v = *reinterpret_cast<const float2*>(p);
-    s.v[0] = v.x; s.v[1] = v.y;
   }
-}
-
-template <int NK, int R>
-__device__ __forceinline__ void stage1_load_chunk(const float* __restrict__ c, const float* __restrict__ dt, int i0,
-                                                  float (&cv)[R], DctSlice<NK> (&dv)[R], int n = R) {
+  f32x4v t;
 #pragma unroll
-  for (int r = 0; r < R; r++)
-    if (r < n) {
-      cv[r] = c[(i0 + r) * 128];
-      load_slice<NK>(dt + (i0 + r) * 16, dv[r]);
-    }
-}
-
-// Rows i0 .. i0 + n - 1 with i0 a multiple of 4, so row i0 + r takes
-// accumulator alt(r).
-template <int NK, int R>
-__device__ __forceinline__ void stage1_fma_chunk(const float (&cv)[R], const DctSlice<NK> (&dv)[R],
-                                                 float (&acc)[NK][2], int n = R) {
-#pragma unroll
-  for (int r = 0; r < R; r++)
-    if (r < n) {
-      const int p = alt(r);
-#pragma unroll
-      for (int k = 0; k < NK; k++) acc[k][p] = __builtin_fmaf(cv[r], dv[r].v[k], acc[k][p]);
-    }
-}
-
-// acc[k][p] = the reference's two alternating chains over k2 = 0..126
-// (x86.rs:161-225) for output (k0 + k, j); c is column j of the plane, dt
-// the transposed DCT at frequency k0.  Chunks of eight rows, the loads of
-// chunk b + 1 in flight while chunk b is accumulated.
-template <int NK>
-__device__ __forceinline__ void stage1_exact(const float* __restrict__ c, const float* __restrict__ dt,
-                                             float (&acc)[NK][2]) {
-  constexpr int R = 8;
-#pragma unroll
-  for (int k = 0; k < NK; k++) acc[k][0] = acc[k][1] = 0.0f;
-  float cv0[R], cv1[R];
-  DctSlice<NK> dv0[R], dv1[R];
-  stage1_load_chunk<NK, R>(c, dt, 0, cv0, dv0);
-#pragma unroll 1
-  for (int i0 = 0; i0 < 112; i0 += 2 * R) {
-    stage1_load_chunk<NK, R>(c, dt, i0 + R, cv1, dv1);
-    stage1_fma_chunk<NK, R>(cv0, dv0, acc);
-    stage1_load_chunk<NK, R>(c, dt, i0 + 2 * R, cv0, dv0);
-    stage1_fma_chunk<NK, R>(cv1, dv1, acc);
+  for (int r = 0; r < 4; r++) {
+    const float a0 = __builtin_isnan(acc[0][r]) ? 0.0f : acc[0][r];
+    const float a1 = __builtin_isnan(acc[1][r]) ? 0.0f : acc[1][r];
+    t[r] = 16 * jt + m == 127 ? 0.0f : a0 + a1;
   }
-  // rows 112 .. 119 are in cv0; rows 120 .. 126 remain
-  stage1_load_chunk<NK, R>(c, dt, 120, cv1, dv1, 7);
-  stage1_fma_chunk<NK, R>(cv0, dv0, acc);
-  stage1_fma_chunk<NK, R>(cv1, dv1, acc, 7);
+  return t;
+}
+
+// Stage 2 (x86.rs:227-272) for AVX lanes 2 w and 2 w + 1: the two chains of
+// each over its 16 terms, 8 c + l for chunk c, and (lane 2 w) + (lane 2 w + 1)
+// of their sums, the first level of the reference's horizontal tree, into
+// part[k * 16 + j].
+__device__ __forceinline__ void stage2_exact(const WaveLds& W, const float* __restrict__ dt, int lane, int w,
+                                             float* __restrict__ part) {
+  const int m = lane & 15, g = lane >> 4;
+  f32x4v v[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int l = 2 * w + i;
+    f32x4v acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int p = 0; p < 2; p++) {
+        const int k = 8 * chain_term(p, s, g) + l;
+        // term 127 holds the reference's over-read D_flat[127 j + 127], which
+        // is D[j + 1][0] (0 after row 15)
+        const float d = dt[k < 127 ? k * 16 + m : m < 15 ? m + 1 : 0];
+        acc[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(W.t[m * kTS + k], k == 127 && m == 15 ? 0.0f : d, acc[p], 0, 0,
+                                                      0);
+      }
+    v[i] = acc[0] + acc[1];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) part[(4 * g + r) * 16 + m] = v[0][r] + v[1][r];
 }
 
 // ---------------------------------------------------------------------------
@@ -261,7 +259,6 @@ __device__ __forceinline__ void stage1_exact(const float* __restrict__ c, const 
 // ---------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4v __attribute__((ext_vector_type(4)));
 
 // bf16 bits of a finite float, rounded to nearest even.
 __device__ __forceinline__ uint32_t bf16_rne(float x) {
@@ -398,10 +395,6 @@ __global__ void __launch_bounds__(64 * kWaves) pdq_hash_block_kernel(const T* __
   static_assert(kWaves == 4 || kWaves == 8 || kWaves == 16, "four, eight or sixteen waves per image");
   static_assert(kWaves <= 8 || kPrec == kDctExact, "sixteen waves: exact arithmetic only");
   constexpr int kBand = (127 + kWaves - 1) / kWaves;  // compressed rows per wave
-  // exact stage 1 on at most eight waves: with two frequencies per thread
-  // its LDS reads of the plane double
-  constexpr int kS1Waves = kWaves > 8 ? 8 : kWaves;
-  constexpr int kNK = 16 / (kS1Waves / 2);  // exact stage 1: frequencies per thread
   const uint32_t n = d_n ? min(*d_n, n_images) : n_images;
   const uint32_t img = blockIdx.x;
   if (img >= n) return;
@@ -415,10 +408,11 @@ __global__ void __launch_bounds__(64 * kWaves) pdq_hash_block_kernel(const T* __
   // A. compression; the DCT table for stage 1 is copied into LDS after it,
   // so the first plane rows are requested at the kernel's start
   const int i0 = wv * kBand, i1 = min(i0 + kBand, 127);
-  const bool bad = compress_band(plane, lane, i0, i1, c, lc);
+  constexpr bool kScalar = kWaves == 16 || !std::is_same<T, uint8_t>::value;  // row addresses (row_words)
+  const bool bad = compress_band<kScalar>(plane, lane, i0, i1, c, lc);
   if (wv == kWaves - 1) *reinterpret_cast<float2*>(&c[127 * 128 + 2 * lane]) = make_float2(0.0f, 0.0f);
   if (kPrec == kDctExact || std::is_same<T, float>::value)
-    for (int e = t; e < 127 * 16; e += 64 * kWaves) L.dct_t[e] = kDctT.v[e];
+    for (int e = t; e < 128 * 16; e += 64 * kWaves) L.dct_t[e] = e < 127 * 16 ? kDctT.v[e] : 0.0f;
   const bool literal = __syncthreads_or(bad ? 1 : 0) != 0;
   if constexpr (std::is_same<T, float>::value) {
     if (literal) {
@@ -439,23 +433,21 @@ __global__ void __launch_bounds__(64 * kWaves) pdq_hash_block_kernel(const T* __
   }
 
   WaveLds& W = L.u.tail.w;
-  float* d2 = L.u.tail.d2;
   if (kPrec == kDctExact || literal) {
-    // B. exact stage 1: thread (j = t % 128, frequencies kNK * (t / 128) ..)
-    const int j = t & 127;
-    const int k0 = kNK * __builtin_amdgcn_readfirstlane(t >> 7);
-    const bool s1 = wv < kS1Waves;  // wave-uniform
-    float acc[kNK][2];
-    if (s1) stage1_exact<kNK>(c + j, L.dct_t + k0, acc);
-    __syncthreads();  // every read of the plane is done: T and d2 overwrite it
-    if (s1) {
+    // B. exact stage 1: wave w computes column tiles w, w + kWaves, ...
+    constexpr int kTiles = kWaves < 8 ? 8 / kWaves : 1;
+    f32x4v tile[kTiles];
+    if (wv < 8) {
 #pragma unroll
-      for (int k = 0; k < kNK; k++) {
-        float a0 = acc[k][0], a1 = acc[k][1];
-        a0 = __builtin_isnan(a0) ? 0.0f : a0;
-        a1 = __builtin_isnan(a1) ? 0.0f : a1;
-        W.t[(k0 + k) * kTS + j] = (j == 127) ? 0.0f : a0 + a1;
-      }
+      for (int q = 0; q < kTiles; q++) tile[q] = stage1_exact(c, L.dct_t, lane, wv + kWaves * q);
+    }
+    __syncthreads();  // every read of the plane is done: T overwrites it
+    if (wv < 8) {
+      const int nn = lane & 15, g = lane >> 4;
+#pragma unroll
+      for (int q = 0; q < kTiles; q++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) W.t[(4 * g + r) * kTS + 16 * (wv + kWaves * q) + nn] = tile[q][r];
     }
   } else if constexpr (kPrec != kDctExact) {
     // B'. stage 1 on matrix cores: wave w computes column tiles w, w + kWaves
@@ -472,41 +464,38 @@ __global__ void __launch_bounds__(64 * kWaves) pdq_hash_block_kernel(const T* __
 #pragma unroll
       for (int r = 0; r < 4; r++) W.t[(4 * g + r) * kTS + 16 * (wv + kWaves * q) + nn] = acc[q][r];
   }
-  if (kPrec == kDctExact || literal) {
-    // d2[j][m] = D[j][m] from the transposed copy in LDS; slot 127 holds the
-    // reference's over-read D_flat[127 j + 127] = D[j + 1][0] (0 after row 15)
-    for (int e = t; e < 16 * 128; e += 64 * kWaves) {
-      const int jj = e & 15, m = e >> 4;
-      d2[jj * kTS + m] = m < 127 ? L.dct_t[e] : (jj < 15 ? L.dct_t[jj + 1] : 0.0f);
-    }
-  }
   __syncthreads();
 
   // C. stage 2 and the tail
   if (kPrec == kDctExact || literal) {
-    if (wv < 4) stage2_column(d2, W, lane, wv);
+    if (wv < 4) stage2_exact(W, L.dct_t, lane, wv, L.u.tail.part[wv]);
+    __syncthreads();
+    if (t < 256) {
+      const float(&s)[4][256] = L.u.tail.part;
+      W.p[t] = (s[0][t] + s[1][t]) + (s[2][t] + s[3][t]);
+    }
   } else if (wv == 0) {
     typename Precision<kPrec>::Op d[4];
     dct_operands<kPrec>(lane, d);
     stage2_mfma<kPrec>(W, lane, d);
   }
+  if (wv == kWaves - 1) write_tmp(W, lane, out, img);
   __syncthreads();
-  if (wv == 0) write_tmp(W, lane, out, img);
   // the eight orientations' PDQFs, written by every wave (two orientations
-  // per element and thread with eight waves)
+  // per element and thread with sixteen waves)
   {
     constexpr int kPer = 8 / (kWaves / 4);  // orientations per thread
     const int idx = t & 255, d0 = (t >> 8) * kPer;
-    dihedral_pdqf_element(W, idx, d0, kPer, mode);
+    dihedral_pdqf_element(W, idx, d0, kPer, mode, kWaves >= 8 ? L.u.tail.grad : nullptr);
   }
   __syncthreads();
   if constexpr (kWaves >= 8) {
-    // waves 0..3 search the four thresholds and write the hashes, wave 4
-    // the qualities, the others the optional PDQF outputs
+    // waves 0..3 search the four thresholds and write the hashes, wave 4 the
+    // qualities, the others the optional PDQF outputs
     if (wv < 4) {
       tail_rows_thresholds_bits(W, lane, wv, out, img, nullptr);
     } else if (wv == 4) {
-      tail_quality(W, lane, out, img, true);
+      tail_quality_sums(L.u.tail.grad, W, lane, out, img);
     } else {
       tail_copy_pdqfs(W, t - 5 * 64, 64 * (kWaves - 5), out, img);
     }

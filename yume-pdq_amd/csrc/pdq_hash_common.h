@@ -54,10 +54,27 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // planes in the cache / from HBM: one f32 plane 48 / 20 us, one RGB8 plane 41
 // / 25 us; 600 f32 planes 153 / 137 us (block of eight waves), 4096 f32 planes
 // (a wave per image) 813 / 705 us, 6.1 TB/s.
+//
+// kScalar: the row's address, the same in all lanes, stays in scalar registers
+// with the lane's offset in one vector register (through integers; as pointer
+// arithmetic the compiler gathers the parts the other way, three vector
+// instructions per load, a ninth of a u8 step's).  The block forms gain (64 u8
+// planes 19.4 -> 18.2 us, 601 f32 planes 134 -> 130), except u8 in blocks of
+// eight waves (1000 planes 63 -> 65.5); the wave forms, near the rate of memory
+// or of their registers, do not (1100 RGBA8 planes 269 -> 278).
+template <bool kScalar, typename V>
+__device__ __forceinline__ auto row_words(const void* plane, uint32_t offset, uint32_t word) {
+  if constexpr (kScalar)
+    return reinterpret_cast<const __attribute__((address_space(1))) V*>(reinterpret_cast<uint64_t>(plane) + offset) +
+           word;
+  else
+    return reinterpret_cast<const V*>(static_cast<const uint8_t*>(plane) + (size_t)offset + sizeof(V) * word);
+}
+
+template <bool kScalar = false>
 __device__ __forceinline__ void load_row(const float* __restrict__ plane, int r, int lane, Row8& o) {
-  const f32x4* p = reinterpret_cast<const f32x4*>(plane + (size_t)r * 512 + 8 * lane);
-  f32x4 a = p[0];
-  f32x4 b = p[1];
+  const auto* p = row_words<kScalar, f32x4>(plane, 2048u * (uint32_t)r, 2u * (uint32_t)lane);
+  const f32x4 a = p[0], b = p[1];
   o.v[0] = a.x; o.v[1] = a.y; o.v[2] = a.z; o.v[3] = a.w;
   o.v[4] = b.x; o.v[5] = b.y; o.v[6] = b.z; o.v[7] = b.w;
 }
@@ -66,15 +83,16 @@ struct RowU8 {
   uint32_t lo, hi;
 };
 
+template <bool kScalar = false>
 __device__ __forceinline__ void load_raw(const uint8_t* __restrict__ plane, int r, int lane, RowU8& o) {
-  const u32x2* p = reinterpret_cast<const u32x2*>(plane + (size_t)r * 512 + 8 * lane);
-  u32x2 a = __builtin_nontemporal_load(p);
+  const u32x2 a = __builtin_nontemporal_load(row_words<kScalar, u32x2>(plane, 512u * (uint32_t)r, (uint32_t)lane));
   o.lo = a.x;
   o.hi = a.y;
 }
 
+template <bool kScalar = false>
 __device__ __forceinline__ void load_raw(const float* __restrict__ plane, int r, int lane, Row8& o) {
-  load_row(plane, r, lane, o);
+  load_row<kScalar>(plane, r, lane, o);
 }
 
 __device__ __forceinline__ void to_f32(const Row8& in, Row8& o) { o = in; }
@@ -127,15 +145,17 @@ struct RowRgba {  // 8 pixels x 4 bytes
 };
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+template <bool kScalar = false>
 __device__ __forceinline__ void load_raw(const Rgb8* __restrict__ plane, int r, int lane, RowRgb& o) {
   // 1536 bytes per row, 24 per lane: three 8-byte loads
-  const u32x2* p = reinterpret_cast<const u32x2*>(reinterpret_cast<const uint8_t*>(plane) + (size_t)r * 1536 + 24 * lane);
+  const auto* p = row_words<kScalar, u32x2>(plane, 1536u * (uint32_t)r, 3u * (uint32_t)lane);
   const u32x2 a = p[0], b = p[1], c = p[2];
   o.w[0] = a.x; o.w[1] = a.y; o.w[2] = b.x; o.w[3] = b.y; o.w[4] = c.x; o.w[5] = c.y;
 }
 
+template <bool kScalar = false>
 __device__ __forceinline__ void load_raw(const Rgba8* __restrict__ plane, int r, int lane, RowRgba& o) {
-  const u32x4* p = reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(plane) + (size_t)r * 2048 + 32 * lane);
+  const auto* p = row_words<kScalar, u32x4>(plane, 2048u * (uint32_t)r, 2u * (uint32_t)lane);
   const u32x4 a = p[0], b = p[1];
   o.w[0] = a.x; o.w[1] = a.y; o.w[2] = a.z; o.w[3] = a.w;
   o.w[4] = b.x; o.w[5] = b.y; o.w[6] = b.z; o.w[7] = b.w;
@@ -248,10 +268,26 @@ __device__ __forceinline__ void chains_start(Chains& c, const Row8& x0, const Ro
   }
 }
 
+// kDpp: the next lane's sums by DPP instead of ds_bpermute.  It takes one vector
+// instruction more per step and no trip through LDS, and the scheduler then
+// keeps more values live: the u8 wave form in blocks of sixteen, with 128
+// registers and four waves on a SIMD, gains (4096 planes 187 -> 182 us, 2048
+// 107 -> 103), the forms with more registers per wave lose to spills or do not
+// care (1100 u8 planes in blocks of four 88 -> 94).
+template <bool kDpp = false>
 __device__ __forceinline__ void chains_finish(const Chains& c, float& c0, float& c1) {
-  const float n0 = shfl_down1(c.s[0]);
-  const float n1 = shfl_down1(c.s[1]);
-  const float n2h = shfl_down1(c.s[2]);
+  auto next = [](float x) {  // lane 63's c1 is no output
+    if constexpr (kDpp) {
+      constexpr int kWaveShl1 = 0x130;
+      return __uint_as_float(static_cast<uint32_t>(
+          __builtin_amdgcn_update_dpp(0, static_cast<int>(__float_as_uint(x)), kWaveShl1, 0xf, 0xf, true)));
+    } else {
+      return shfl_down1(x);
+    }
+  };
+  const float n0 = next(c.s[0]);
+  const float n1 = next(c.s[1]);
+  const float n2h = next(c.s[2]);
   c0 = (c.s[3] + (c.s[4] + c.s[5])) + (c.s[6] + c.s[7]);
   c1 = (c.s[8] + (c.s[9] + n0)) + (n1 + n2h);
 }
@@ -352,7 +388,9 @@ using BlockLds = BlockLdsOf<kWavesPerBlock>;
 // are read from the group's lane 0, which takes the operands of the xor tree.
 template <int kCtrl>
 __device__ __forceinline__ uint32_t dpp_u(uint32_t x) {
-  return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), kCtrl, 0xf, 0xf, false));
+  // bound_ctrl set (every lane has a source here): the move folds into the
+  // instruction that uses it
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), kCtrl, 0xf, 0xf, true));
 }
 template <int kCtrl>
 __device__ __forceinline__ float dpp_f(float x) {
@@ -590,6 +628,49 @@ __device__ __forceinline__ float half_swapf(float x, int lane) {
   return __uint_as_float(half_swap(__float_as_uint(x), lane));
 }
 
+// The running extremes of median_search8 over the 32 elements of this lane's
+// AVX lane, from x, its run of eight (runs in order on rows 0, 1, 3, 2).  The
+// reference's a > b ? a : b is associative except that a NaN makes it start
+// anew, so runs fold on their own and in order, or, where a NaN is among the
+// elements, the whole chain is run.
+__device__ __forceinline__ void median_extremes_rows(const float* __restrict__ P, const float (&x)[8], int lane,
+                                                     float& mx, float& mn) {
+  float mxl = -3.40282347e+38f, mnl = 3.40282347e+38f;  // f32::MIN, f32::MAX
+  bool nan = false;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    mnl = x86min(mnl, x[e]);
+    mxl = x86max(mxl, x[e]);
+    nan |= __builtin_isnan(x[e]);
+  }
+  const auto mx2 = __builtin_amdgcn_permlane16_swap(__float_as_uint(mxl), __float_as_uint(mxl), false, false);
+  const auto mn2 = __builtin_amdgcn_permlane16_swap(__float_as_uint(mnl), __float_as_uint(mnl), false, false);
+  // [0]: the even row's of the pair, [1]: the odd row's; the odd row comes
+  // second in the lower half (runs 0, 1) and first in the upper (runs 3, 2)
+  const bool up = lane >= 32;
+  const float xa = __uint_as_float(up ? mx2[1] : mx2[0]), xb = __uint_as_float(up ? mx2[0] : mx2[1]);
+  const float na = __uint_as_float(up ? mn2[1] : mn2[0]), nb = __uint_as_float(up ? mn2[0] : mn2[1]);
+  mxl = x86max(xa, xb);
+  mnl = x86min(na, nb);
+  const auto mx4 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mxl), __float_as_uint(mxl), false, false);
+  const auto mn4 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mnl), __float_as_uint(mnl), false, false);
+  mxl = x86max(__uint_as_float(mx4[0]), __uint_as_float(mx4[1]));
+  mnl = x86min(__uint_as_float(mn4[0]), __uint_as_float(mn4[1]));
+  if (wave_any(nan)) {
+    const int l = lane & 7;
+    mxl = -3.40282347e+38f;
+    mnl = 3.40282347e+38f;
+#pragma unroll 1
+    for (int c = 0; c < 32; c++) {
+      const float v = P[8 * c + l];
+      mnl = x86min(mnl, v);
+      mxl = x86max(mxl, v);
+    }
+  }
+  mx = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(grp_max8(mxl, lane))));
+  mn = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(grp_min8(mnl, lane))));
+}
+
 // median_search8 of one PDQF on a whole wave, for latency: each of the
 // sixteen sequential sums (8 AVX lanes x the two sides of the guess, as in
 // median_search8_split) is cut into four runs of 8 elements on four rows of
@@ -601,30 +682,41 @@ __device__ __forceinline__ float half_swapf(float x, int lane) {
 // guess, on negated elements), row = lane >> 4 holds run row ^ (row >> 1).
 // The counts are integers and are summed in any order.  The guess and the
 // bounds are wave-uniform, so the search's branches are scalar.
+//
+// One wave alone: a dependent operation takes 8.5 cycles, an independent one
+// 4.2, and the 32 additions in order are the longest chain, so what else an
+// iteration needs is arranged to fill their gaps:
+//  - an element that leaves the range [mn, mx] never comes back and becomes
+//    NaN when it leaves, so one comparison per element and iteration selects
+//    (not two and their AND);
+//  - the counts decide the side, and the reciprocal of each side's count is
+//    refined, while the sums are under way; behind them remain the five
+//    operations of a correctly rounded quotient (q = s y, then twice q +=
+//    (s - c q) y, as the compiler's division ends), taken for both sides
+//    before one lane's is read.  Sums whose exponent is near either end of
+//    the range, zero and non-finite ones take the division itself.
+// 9 to 11 iterations for pictures and noise took 11800 cycles and take 9200,
+// the quality's additions on the same SIMD included, which now bound both.
 __device__ __forceinline__ void median_search_rows(const float* __restrict__ P, int lane, float& threshold,
                                                    float& bit_threshold) {
   const int l = lane & 7;
   const bool lower_side = (lane & 8) != 0;
+  const uint32_t sign = lower_side ? 0x80000000u : 0u;
   const int row = lane >> 4;
   const int run = row ^ (row >> 1);
-  float mx, mn;
-  {
-    // the reference's running extremes over the 32 elements of AVX lane l
-    float mxl = -3.40282347e+38f, mnl = 3.40282347e+38f;  // f32::MIN, f32::MAX
-#pragma unroll
-    for (int c = 0; c < 32; c++) {
-      const float v = P[8 * c + l];
-      mnl = x86min(mnl, v);
-      mxl = x86max(mxl, v);
-    }
-    mx = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(grp_max8(mxl, lane))));
-    mn = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(grp_min8(mnl, lane))));
-  }
   float x[8];
 #pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const float v = P[8 * (8 * run + e) + l];
-    x[e] = lower_side ? -v : v;
+  for (int e = 0; e < 8; e++) x[e] = P[8 * (8 * run + e) + l];
+  float mx, mn;
+  median_extremes_rows(P, x, lane, mx, mn);
+  const float kGone = __builtin_nanf("");
+  {
+    const float hi = lower_side ? -mn : mx;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const float v = __uint_as_float(__float_as_uint(x[e]) ^ sign);
+      x[e] = v <= hi ? v : kGone;
+    }
   }
   float guess = (mn + mx) * 0.5f;
   float last = guess;
@@ -632,50 +724,90 @@ __device__ __forceinline__ void median_search_rows(const float* __restrict__ P, 
 #pragma unroll 1
   for (int iter = 0; iter < 32; iter++) {
     // this lane's side: (guess, mx] above, or [mn, guess) below (negated)
-    const float lo_b = lower_side ? -guess : guess;
-    const float hi_b = lower_side ? -mn : mx;
+    const float lo = __uint_as_float(__float_as_uint(guess) ^ sign);
+    bool m[8];
     float s[8];
     uint32_t n = 0;
+    // the sequential sum, run after run; `between` is what fills its gaps
+    float acc = 0.0f;
+    auto add_run = [&](auto&& between) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        acc = acc + s[e];
+        between(e);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
 #pragma unroll
     for (int e = 0; e < 8; e++) {
-      const bool m = (x[e] > lo_b) && (x[e] <= hi_b);
-      n += m ? 1u : 0u;
-      s[e] = m ? x[e] : 0.0f;
+      m[e] = x[e] > lo;
+      s[e] = m[e] ? x[e] : 0.0f;
+      n += m[e] ? 1u : 0u;
+      acc = acc + s[e];
     }
-    // the sequential sum, run after run
-    float acc = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; e++) acc = acc + s[e];
-    acc = row_swapf(acc, lane);  // row 1 continues row 0
-#pragma unroll
-    for (int e = 0; e < 8; e++) acc = acc + s[e];
-    acc = half_swapf(acc, lane);  // row 3 continues row 1
-#pragma unroll
-    for (int e = 0; e < 8; e++) acc = acc + s[e];
-    acc = row_swapf(acc, lane);  // row 2 continues row 3
-#pragma unroll
-    for (int e = 0; e < 8; e++) acc = acc + s[e];
-    float sum = grp_sum8(acc);  // the AVX tree; rows 2 hold the whole sums
-    if (lower_side) sum = sum == 0.0f ? 0.0f : -sum;  // back to the original sign (+0 for zero)
-    n = grp_isum8(n);
-    n += row_swap(n, lane);
-    n += half_swap(n, lane);
-    const uint32_t gtc = __builtin_amdgcn_readlane(n, 0);
-    const uint32_t ltc = __builtin_amdgcn_readlane(n, 8);
-    const float sg = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sum), 32));
-    const float sl = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sum), 40));
+    __builtin_amdgcn_sched_barrier(0);
+    // a swap of a register with its copy leaves the even row's value in both
+    // rows of the pair's first result and the odd row's in the second (the
+    // halves alike): row 1 continues row 0
+    acc = __uint_as_float(
+        __builtin_amdgcn_permlane16_swap(__float_as_uint(acc), __float_as_uint(acc), false, false)[0]);
+    // both sides' counts, each in all lanes of its side
+    add_run([&](int e) {
+      if (e == 0) n += dpp_u<kDppXor1>(n);
+      if (e == 2) n += dpp_u<kDppXor2>(n);
+      if (e == 4) n += dpp_u<kDppHalfMirror>(n);
+      if (e == 6) {
+        const auto r = __builtin_amdgcn_permlane16_swap(n, n, false, false);
+        n = r[0] + r[1];
+      }
+    });
+    acc = __uint_as_float(
+        __builtin_amdgcn_permlane32_swap(__float_as_uint(acc), __float_as_uint(acc), false, false)[0]);
+    uint32_t gtc = 0, ltc = 0;
+    float c = 0.0f, y = 0.0f;
+    add_run([&](int e) {  // row 3 continues row 1
+      if (e == 0) {
+        const auto h = __builtin_amdgcn_permlane32_swap(n, n, false, false);
+        n = h[0] + h[1];
+      }
+      if (e == 2) c = (float)n;
+      if (e == 3) gtc = __builtin_amdgcn_readlane(n, 0);
+      if (e == 4) ltc = __builtin_amdgcn_readlane(n, 8);
+      if (e == 5) y = __builtin_amdgcn_rcpf(c);
+    });
+    const bool up = gtc + num_over > 128;
+    const bool down = ltc + num_under > 128;
+    // up: mn becomes the guess and what lies below it goes; down: mx, above
+    const bool goes = lower_side == up;
+    acc = __uint_as_float(
+        __builtin_amdgcn_permlane16_swap(__float_as_uint(acc), __float_as_uint(acc), false, false)[1]);
+    float fix = 0.0f;
+    add_run([&](int e) {  // row 2 continues row 3
+      if (e == 0) fix = __builtin_fmaf(-c, y, 1.0f);
+      if (e == 2) {
+        y = __builtin_fmaf(fix, y, y);
+        asm volatile("" : "+v"(y));  // not moved behind the sums
+      }
+      x[e] = m[e] && goes ? kGone : x[e];
+      asm volatile("" : "+v"(x[e]));
+    });
+    const float sum = grp_sum8(acc);  // the AVX tree; row 2 holds the whole sums
+    float q = sum * y;
+    q = __builtin_fmaf(__builtin_fmaf(-c, q, sum), y, q);
+    q = __builtin_fmaf(__builtin_fmaf(-c, q, sum), y, q);
+    __builtin_amdgcn_sched_barrier(0);
     last = guess;
-    if (gtc + num_over > 128) {
-      num_under += ltc;
-      mn = guess;
-      guess = sg / (float)gtc;
-    } else if (ltc + num_under > 128) {
-      num_over += gtc;
-      mx = guess;
-      guess = sl / (float)ltc;
-    } else {
-      break;
+    if (!up && !down) break;
+    const int from = up ? 32 : 40;
+    const uint32_t flip = up ? 0u : 0x80000000u;  // back to the original sign
+    const uint32_t sb = __builtin_amdgcn_readlane(__float_as_uint(sum), from);
+    guess = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(q), from) ^ flip);
+    if (((sb >> 23) & 0xffu) - 40u > 180u) {
+      const float z = __uint_as_float(sb);
+      guess = (z == 0.0f ? 0.0f : __uint_as_float(sb ^ flip)) / (float)(up ? gtc : ltc);
     }
+    num_under += up ? ltc : 0u;
+    num_over += up ? 0u : gtc;
   }
   threshold = guess;
   bit_threshold = last;

@@ -67,20 +67,42 @@ __device__ __forceinline__ void stage2_to_pdqf(const float* __restrict__ d2, Wav
 // mode, columns 0..7 only in the AVX2-compatible mode (x86.rs:330-376 loads
 // 8 floats per row).  Negation is exact, so the sequence of in-place flips
 // in visit_dihedrals reduces to these closed forms.
-__device__ __forceinline__ void dihedral_pdqf_element(WaveLds& W, int idx, int d0, int nd, uint32_t mode) {
+__device__ __forceinline__ float dihedral_value(int d, int i, int j, float a, float at, int ncols) {
+  const bool nr = (i & 1) == 0;
+  const bool nc = (j & 1) == 0 && j < ncols;
+  const float v = d < 4 ? a : at;
+  const int kind = d & 3;  // 0: as is, 1: sc (FLOPPED / ROT90), 2: sr.sc, 3: sr
+  // the transposed four negate (none, sr, sr.sc, sc) for d = 4, 5, 6, 7
+  const int k = d < 4 ? kind : (kind == 1 ? 3 : kind == 3 ? 1 : kind);
+  const bool neg = k == 1 ? nc : k == 2 ? (nr != nc) : k == 3 ? nr : false;
+  return neg ? v * -1.0f : v;
+}
+
+// With `grad`, also the element's part of the absolute differences that the
+// qualities add up: orientation d's at d * kGradStride, in the reference's
+// order (vertical 15 x 16, then horizontal 16 x 15).
+constexpr int kGradStride = 484;  // floats per orientation; the eight start in different banks
+
+__device__ __forceinline__ void dihedral_pdqf_element(WaveLds& W, int idx, int d0, int nd, uint32_t mode,
+                                                      float* __restrict__ grad = nullptr) {
   const int ncols = mode == kDihedralAvx2 ? 8 : 16;
   const int i = idx >> 4, j = idx & 15;
   const float a = W.p[idx];
   const float at = W.p[j * 16 + i];
-  const bool nr = (i & 1) == 0;
-  const bool nc = (j & 1) == 0 && j < ncols;
+  if (!grad) {
+    for (int d = d0; d < d0 + nd; d++) W.t[d * 256 + idx] = dihedral_value(d, i, j, a, at, ncols);
+    return;
+  }
+  // the element below and the one to the right (clamped where there is none)
+  const int i1 = min(i + 1, 15), j1 = min(j + 1, 15);
+  const float below = W.p[i1 * 16 + j], below_t = W.p[j * 16 + i1];
+  const float right = W.p[i * 16 + j1], right_t = W.p[j1 * 16 + i];
   for (int d = d0; d < d0 + nd; d++) {
-    const float v = d < 4 ? a : at;
-    const int kind = d & 3;  // 0: as is, 1: sc (FLOPPED / ROT90), 2: sr.sc, 3: sr
-    // the transposed four negate (none, sr, sr.sc, sc) for d = 4, 5, 6, 7
-    const int k = d < 4 ? kind : (kind == 1 ? 3 : kind == 3 ? 1 : kind);
-    const bool neg = k == 1 ? nc : k == 2 ? (nr != nc) : k == 3 ? nr : false;
-    W.t[d * 256 + idx] = neg ? v * -1.0f : v;
+    const float v = dihedral_value(d, i, j, a, at, ncols);
+    W.t[d * 256 + idx] = v;
+    float* g = grad + d * kGradStride;
+    if (i < 15) g[idx] = __builtin_fabsf(v - dihedral_value(d, i + 1, j, below, below_t, ncols));
+    if (j < 15) g[240 + idx - i] = __builtin_fabsf(v - dihedral_value(d, i, j + 1, right, right_t, ncols));
   }
 }
 
@@ -93,6 +115,38 @@ __device__ __forceinline__ void tail_quality(WaveLds& W, int lane, const HashOut
     const float q = adjust_quality(sum_of_gradients16(&W.t[lane * 256]));
     W.q[lane] = q;
     if (write_out) out.quality[(size_t)img * 8 + lane] = q;
+  }
+}
+
+// The latency form of the qualities: lane d adds up the differences that
+// dihedral_pdqf_element left in `grad`.  One wave for all eight: its additions
+// share a SIMD with a threshold search, which waits for the vector ALU then
+// (9200 cycles for both; 10200 with the additions, and the differences, spread
+// over four waves, a search's neighbour each).
+__device__ __forceinline__ void tail_quality_sums(const float* __restrict__ grad, WaveLds& W, int lane,
+                                                  const HashOutputs& out, uint32_t img) {
+  if (lane < 8) {
+    const f32x4* g4 = reinterpret_cast<const f32x4*>(grad + lane * kGradStride);
+    constexpr int kAhead = 4;  // loads in flight
+    f32x4 v[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; i++) v[i] = g4[i];
+    float g = 0.0f;
+#pragma unroll 1
+    for (int c = 0; c < 120; c += kAhead) {
+#pragma unroll
+      for (int i = 0; i < kAhead; i++) {
+        const f32x4 x = v[i];
+        v[i] = g4[min(c + kAhead + i, 119)];
+        g += x.x;
+        g += x.y;
+        g += x.z;
+        g += x.w;
+      }
+    }
+    const float q = adjust_quality(g);
+    W.q[lane] = q;
+    out.quality[(size_t)img * 8 + lane] = q;
   }
 }
 
