@@ -88,3 +88,17 @@ def test_threshold_search_at_all_scales(gpu, oracle, dev, exponent):
             where = f"layout {layout}, 2^{exponent}, image {k}"
             assert np.array_equal(h[k], H), where
             assert same(q[k], Q) and same(t[k], T), where
+
+
+@pytest.mark.parametrize("per_cu", [1, 5.5])
+def test_automatic_layout_around_its_lines(gpu, dev, per_cu):
+    """Batches on both sides of a change of layout equal the wave form's."""
+    import torch
+    n = int(per_cu * torch.cuda.get_device_properties(dev).multi_processor_count) + 1
+    x = torch.from_numpy(synthetic.images_u8(64)).to(dev).repeat((n + 63) // 64, 1, 1)[:n].contiguous()
+    x[-1] = 255 - x[-1]
+    want = gpu.hash_batch(x, layout=gpu.LAYOUT_WAVE)
+    for m in (n, n - 1):
+        got = gpu.hash_batch(x[n - m:])
+        for a, b in zip(got, want):
+            assert torch.equal(a, b[n - m:])

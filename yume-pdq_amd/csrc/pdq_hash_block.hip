@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "pdq_hash_common.h"
@@ -567,15 +568,20 @@ int device_cus() {
 
 int hash_layout_for(uint32_t n_images, int dct) {
   // Exact arithmetic: sixteen waves per image while the images fit one per
-  // CU, then eight (18 us for one u8 image, 23 us for 128, 71 us for 1024,
-  // against 60 / 71 / 78 us for a wave per image) until the batch is large
-  // enough that a wave per image fills the GPU with less LDS per image (1536
-  // u8 images: 91 us against 105 us; 4096: 193-208 against 261 us).
+  // CU, then eight, until the batch is large enough that a wave per image
+  // fills the GPU with less LDS per image.  The lines cross at 5.5 images per
+  // CU (u8 and RGB8 a little above, f32 and RGBA8 there); eight waves / a wave
+  // per image, in us:
+  //   images      1100        1365        1536        2048
+  //   u8        75 / 91     88 / 92     93 / 95   120 / 108
+  //   RGB8     167 / 202   201 / 226   215 / 230   282 / 292
+  //   f32      231 / 273   278 / 285   293 / 291   385 / 367
+  //   RGBA8    230 / 267   276 / 284   301 / 294   397 / 376
   // Matrix-core arithmetic exists only in the block forms of 4 and 8 waves.
   if (dct != kDctExact) return 8;
-  if (n_images > 1024) return 1;
-  const int cus = device_cus();
-  return (cus > 0 && n_images <= (uint32_t)cus) ? 16 : 8;
+  const uint32_t cus = (uint32_t)std::max(0, device_cus());
+  if (cus == 0) return n_images > 1024 ? 1 : 8;
+  return n_images <= cus ? 16 : n_images <= cus * 11 / 2 ? 8 : 1;
 }
 
 hipError_t launch_hash(const void* planes, int input_kind, uint64_t plane_stride, uint32_t n_images, uint32_t mode,
