@@ -792,6 +792,270 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
   hits_flush(H, hits, capacity, counter);
 }
 
+// ---------------------------------------------------------------------------
+// The held-rows layout: few rows against many queries.
+//
+// The even layout holds query tiles in registers and streams rows past them;
+// with few rows a part is a handful of loads, and a wave's time the latency of
+// loading and expanding its 256 queries first.  Here a block expands up to 64
+// query tiles into LDS once, together, and each of its waves holds 192 rows
+// (128 below the threshold of three products per accumulator) and runs all the
+// tiles past them: 12 products for one LDS read, no expansion in the loop.
+// The prefix products, their flags and the exact check are the even layout's.
+// The matrix cores bound a wave's loop (24 products beside about 20 vector
+// instructions per pair of tiles); the launch, 9.3 us as measured, bounds the
+// calls with the fewest rows.
+//
+// Kernel times with the reset, even layout / here, us:
+//   rows       256         512        1000        2048 queries
+//   10^4    19.1 /  9.2  20.7 /  9.2  23.9 / 12.5  29.0 / 17.4
+//   10^5    11.4 /  9.7  12.5 / 10.8  17.6 / 13.1  26.3 / 19.8
+//   3x10^5  14.9 / 12.0  17.8 / 15.6  24.0 / 22.3  43.5 / 37.1
+//   7x10^5  17.4 / 15.7  24.0 / 22.4  38.1 / 35.4  69.4 / 63.3
+// ---------------------------------------------------------------------------
+constexpr int kHeldWaves = 8;          // waves per block, sharing the block's query codes
+constexpr uint32_t kHeldTiles = 64;    // most query tiles per block (64 KiB of codes)
+
+// Rows per wave and group: four accumulators of kPer products, a 16-row tile
+// each.
+template <int kPer>
+struct Held {
+  static constexpr int kTiles = 4 * kPer;
+  static constexpr int kLoads = kTiles / 4;  // 16 bytes per lane: 64 rows each
+  static constexpr uint32_t kRows = 16 * kTiles;
+};
+
+__device__ __forceinline__ Expanded codes_from(const u32x4& v) {
+  Expanded e;
+  e.d[0] = v.x;
+  e.d[1] = v.y;
+  e.d[2] = v.z;
+  e.d[3] = v.w;
+  return e;
+}
+
+template <int kPer>
+constexpr int held_scale(int p) {
+  return p == 0 ? kScale1 : kPer == 2 ? kScale512 : p == 1 ? kScale128 : kScale32k;
+}
+
+// Query tile q against the held rows: accumulator k takes its first product
+// while k - 1 takes its second and k - 2 its third (of this query tile or, for
+// the last ones, of the one before), so no product waits for the one before
+// it; the result of the tile before is folded just before.  Once the tile
+// before has issued its last product, `refill` loads the next tile's codes
+// into its place.
+template <int kPer, int K = 0, class Refill>
+__device__ __forceinline__ void held_tile(const Expanded& q, Expanded& before, Refill&& refill,
+                                          const Expanded (&rows)[4 * kPer], const v4f& c0, uint32_t (&acc)[2],
+                                          v4f (&r)[4]) {
+  fold_flags(r[K], acc[K % 2]);
+  r[K] = mfma_acc<held_scale<kPer>(0)>(q, rows[kPer * K], c0);
+  if constexpr (kPer >= 2) {
+    constexpr int k = (K + 3) % 4;
+    r[k] = mfma_acc<held_scale<kPer>(1)>(K >= 1 ? q : before, rows[kPer * k + 1], r[k]);
+  }
+  if constexpr (kPer >= 3) {
+    constexpr int k = (K + 2) % 4;
+    r[k] = mfma_acc<held_scale<kPer>(2)>(K >= 2 ? q : before, rows[kPer * k + 2], r[k]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (K == 1) refill(before);
+  if constexpr (K + 1 < 4) held_tile<kPer, K + 1>(q, before, static_cast<Refill&&>(refill), rows, c0, acc, r);
+}
+
+// What is left after the last query tile.
+template <int kPer>
+__device__ __forceinline__ void held_last(const Expanded (&rows)[4 * kPer], const Expanded& q, uint32_t (&acc)[2],
+                                          v4f (&r)[4]) {
+  if constexpr (kPer >= 2) r[3] = mfma_acc<held_scale<kPer>(1)>(q, rows[kPer * 3 + 1], r[3]);
+  if constexpr (kPer >= 3) {
+    r[2] = mfma_acc<held_scale<kPer>(2)>(q, rows[kPer * 2 + 2], r[2]);
+    r[3] = mfma_acc<held_scale<kPer>(2)>(q, rows[kPer * 3 + 2], r[3]);
+  }
+#pragma unroll
+  for (int k = 0; k < 4; k++) fold_flags(r[k], acc[k % 2]);
+}
+
+// The block's query codes, a lane's 16 bytes of each tile side by side.
+struct HeldLds {
+  u32x4 q[kHeldTiles][64];
+  HitList<kEvenStage> hits;
+};
+
+// Codes of query tiles t0 .. t0 + n - 1 into S.q; padding queries get zero
+// codes, whose products never reach the bound.
+__device__ __forceinline__ void held_queries(HeldLds& S, const uint32_t* __restrict__ queries, uint32_t n_queries,
+                                             uint32_t t0, uint32_t n) {
+  for (uint32_t i = threadIdx.x; i < n * 64; i += 64 * kHeldWaves) {
+    const uint32_t lane = i & 63, qi = 16 * (t0 + (i >> 6)) + (lane & 15);
+    Expanded e;
+    expand_word(queries[(size_t)min(qi, n_queries - 1) * 8 + (lane >> 4)], e);
+    const uint32_t keep = qi < n_queries ? 0xffffffffu : 0u;
+    S.q[i >> 6][lane] = u32x4{e.d[0] & keep, e.d[1] & keep, e.d[2] & keep, e.d[3] & keep};
+  }
+}
+
+// Query tiles per vote.
+constexpr uint32_t kHeldVote = 8;
+
+// Rows row0 .. row0 + left - 1 against the block's n query tiles (t0 the first
+// of them among all).
+template <int kPer, bool kPlane>
+__device__ __forceinline__ void held_rows(HeldLds& S, const uint4* __restrict__ db, const uint4* __restrict__ plane,
+                                          uint64_t n_rows, uint64_t row0, uint32_t left,
+                                          const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t t0,
+                                          uint32_t n, uint32_t threshold, MatchHit* __restrict__ hits,
+                                          uint64_t capacity, unsigned long long* __restrict__ counter,
+                                          uint64_t index_base) {
+  using H = Held<kPer>;
+  const int lane = threadIdx.x & 63;
+  const int rn = lane & 15, kq = lane >> 4;
+  const uint4* base = kPlane ? plane + row0 : db + 2 * row0;  // uniform
+  // rows past the end repeat the last one; their pairs are never reported
+  auto load = [&](uint32_t r) -> uint4 {
+    r = min(r + (uint32_t)lane, left - 1);
+    return base[kPlane ? r : 2 * r];
+  };
+  uint4 raw[H::kLoads];
+#pragma unroll
+  for (int l = 0; l < H::kLoads; l++) raw[l] = load(64 * l);
+  const float bound = (float)(128 - 2 * (int)threshold);
+  const int ibound = __float_as_int(bound);
+  const v4f c0 = kPer == 3 ? flags_c0_tri(bound) : flags_c0(bound);
+  constexpr uint32_t kMask = kPer == 3 ? kFlagMaskTri : kFlagMask;
+  const Expanded zero = {{0u, 0u, 0u, 0u}};
+  auto code = [&](uint32_t t) { return codes_from(S.q[t][lane]); };
+#pragma unroll 1
+  for (uint32_t g = 0; g < left; g += H::kRows) {
+    Expanded rows[H::kTiles];
+#pragma unroll
+    for (int l = 0; l < H::kLoads; l++) {
+      uint32_t w[4] = {raw[l].x, raw[l].y, raw[l].z, raw[l].w};
+      transpose_rows(w);
+#pragma unroll
+      for (int j = 0; j < 4; j++) expand_word(w[j], rows[4 * l + j]);
+      raw[l] = load(g + H::kRows + 64 * l);
+    }
+    uint32_t acc[2] = {0u, 0u};
+    v4f r[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) r[k] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    Expanded x = code(0), y = zero;
+    // bit i: a flag among query tiles 8 i - 1 .. 8 i + 6 (a tile's results are
+    // folded with the next one); the last bit, what remains
+    uint32_t pending = 0, bit = 0;
+    auto vote = [&] {
+      const uint64_t v = __ballot(((acc[0] | acc[1]) & kMask) != 0);
+      pending |= (uint32_t)(v != 0) << bit;
+      bit++;
+      acc[0] = acc[1] = 0u;
+    };
+    uint32_t t = 0;
+#pragma unroll 1
+    for (; t + kHeldVote <= n; t += kHeldVote) {
+#pragma unroll 1
+      for (uint32_t k = 0; k < kHeldVote; k += 2) {
+        held_tile<kPer>(x, y, [&](Expanded& e) { e = code(t + k + 1); }, rows, c0, acc, r);
+        held_tile<kPer>(y, x, [&](Expanded& e) { e = code(min(t + k + 2, n - 1)); }, rows, c0, acc, r);
+      }
+      vote();
+    }
+#pragma unroll 1
+    for (; t + 2 <= n; t += 2) {
+      held_tile<kPer>(x, y, [&](Expanded& e) { e = code(t + 1); }, rows, c0, acc, r);
+      held_tile<kPer>(y, x, [&](Expanded& e) { e = code(min(t + 2, n - 1)); }, rows, c0, acc, r);
+    }
+    if (t < n) {
+      held_tile<kPer>(x, y, [&](Expanded& e) { e = x; }, rows, c0, acc, r);
+      // y holds the last tile's codes, as after a pair
+    }
+    held_last<kPer>(rows, y, acc, r);
+    vote();
+    if (pending) {
+#pragma unroll 1
+      for (uint32_t q = 0; q < n; q++) {
+        // the bits that cover tile q: its vote's, or the last one
+        const uint32_t b = min((q + 1) / kHeldVote, bit - 1);
+        if (!(pending >> b & 1u)) continue;
+        const Expanded qe = code(q);
+        uint32_t tmask = 0;
+#pragma unroll
+        for (int j = 0; j < H::kTiles; j++) {
+          const v4f c = mfma_prefix(qe, rows[j]);
+          const int m = max(max(__float_as_int(c.x), __float_as_int(c.y)),
+                            max(__float_as_int(c.z), __float_as_int(c.w)));
+          tmask |= (wave_any(m >= ibound) ? 1u : 0u) << j;
+        }
+        while (tmask) {
+          const int j = __builtin_ctz(tmask);
+          tmask &= tmask - 1;
+          Expanded e = rows[0];  // rows[j], selected (registers cannot be indexed)
+#pragma unroll
+          for (int k = 1; k < H::kTiles; k++)
+            if (j == k) e = rows[k];
+          stage_candidates(mfma_prefix(qe, e), (int)q, row0 + g + 16 * j, 16 * t0, rn, kq, bound, queries,
+                           reinterpret_cast<const uint32_t*>(db), n_queries, n_rows, threshold, S.hits, hits,
+                           capacity, counter, index_base);
+        }
+      }
+    }
+  }
+}
+
+// How a call is cut: `chunks` groups of at most `tiles` query tiles, each
+// block holding one of them; a wave's rows are `groups` row groups.
+struct HeldPlan {
+  uint32_t chunks, tiles, groups, blocks_per_xcd;  // blocks per XCD and chunk
+};
+// The cut that costs least, by a wave's products (12 of 18.1 cycles and their
+// share of the rest per tile and row group, and about two tiles' time for
+// loading and expanding the rows of a group), times the blocks that share a CU.
+// cus: of one XCD; two blocks are resident on each (72 KiB of LDS).
+inline HeldPlan held_plan(uint64_t row_groups, uint32_t tiles, uint32_t cus) {
+  const uint32_t blocks_per_xcd = 2 * cus;
+  HeldPlan best{1, 1, 1, 1};
+  uint64_t least = ~0ull;
+  const uint32_t first = (tiles + kHeldTiles - 1) / kHeldTiles;
+  for (uint32_t c = first; c < 2 * first + 16 && c <= tiles; c++) {
+    const uint32_t t = (tiles + c - 1) / c;
+    const uint32_t at_once = blocks_per_xcd / c ? blocks_per_xcd / c : 1;
+    const uint64_t waves = 8ull * kHeldWaves * at_once;  // per chunk
+    const uint64_t g = (row_groups + waves - 1) / waves;
+    const uint64_t need = (row_groups + g * 8 * kHeldWaves - 1) / (g * 8 * kHeldWaves);  // blocks per XCD
+    const uint64_t per_cu = (need * c + cus - 1) / cus;
+    const uint64_t cost = g * ((uint64_t)t * 224 + 464) * per_cu + t * 64;
+    if (cost < least) {
+      least = cost;
+      best = HeldPlan{c, t, (uint32_t)g, (uint32_t)need};
+    }
+  }
+  return best;
+}
+
+template <int kPer, bool kPlane>
+__global__ void __launch_bounds__(64 * kHeldWaves) __attribute__((amdgpu_waves_per_eu(4))) pdq_match_held_kernel(
+    const uint4* __restrict__ db, const uint4* __restrict__ plane, uint64_t n_rows,
+    const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t threshold, MatchHit* __restrict__ hits,
+    uint64_t capacity, unsigned long long* __restrict__ counter, uint64_t index_base, HeldPlan plan) {
+  __shared__ HeldLds S;
+  const uint32_t slot = blockIdx.x >> 3;
+  const uint32_t chunk = slot % plan.chunks;
+  const uint32_t t0 = chunk * plan.tiles, all = (n_queries + 15) / 16;
+  if (t0 >= all) return;  // the same for the whole block
+  const uint32_t n = min(plan.tiles, all - t0);
+  held_queries(S, queries, n_queries, t0, n);
+  hits_init(S.hits);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint64_t part = ((uint64_t)(slot / plan.chunks) * kHeldWaves + wave) * 8 + (blockIdx.x & 7);
+  const uint64_t rows = (uint64_t)plan.groups * Held<kPer>::kRows;
+  const uint64_t row0 = part * rows;
+  if (row0 < n_rows)
+    held_rows<kPer, kPlane>(S, db, plane, n_rows, row0, (uint32_t)min(n_rows - row0, rows), queries, n_queries, t0, n,
+                            threshold, hits, capacity, counter, index_base);
+  hits_flush(S.hits, hits, capacity, counter);
+}
+
 // The second kernel of the shared-rows layout, in blocks of kResolveWaves
 // waves.  Each wave takes records in turn: for every pending group of the
 // record's sub-chunk it recomputes the group's products, and for each query
@@ -1426,6 +1690,30 @@ static hipError_t with_query_tiles(int qt, F&& f) {
 static uint32_t even_waves_per_xcd(int cus) { return (uint32_t)std::max(1, cus) * 16 / 8; }
 
 // The even layout's launch.
+template <int kPer>
+static hipError_t launch_held(const void* db, const void* plane, uint64_t n_rows, const void* queries,
+                              uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
+                              unsigned long long* counter, uint64_t index_base, hipStream_t stream, bool reset) {
+  int dev = 0, cus = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+  const uint64_t row_groups = (n_rows + Held<kPer>::kRows - 1) / Held<kPer>::kRows;
+  const HeldPlan plan = held_plan(row_groups, (n_queries + 15) / 16, (uint32_t)std::max(8, cus) / 8);
+  const dim3 grid((unsigned)(8 * plan.blocks_per_xcd * plan.chunks)), block(64 * kHeldWaves);
+  const uint4* rows = static_cast<const uint4*>(db);
+  const uint4* prefix = static_cast<const uint4*>(plane);
+  const uint32_t* q = static_cast<const uint32_t*>(queries);
+  if (reset) hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(1), 0, stream, nullptr, counter);
+  if (plane)
+    hipLaunchKernelGGL((pdq_match_held_kernel<kPer, true>), grid, block, 0, stream, rows, prefix, n_rows, q, n_queries,
+                       threshold, hits, capacity, counter, index_base, plan);
+  else
+    hipLaunchKernelGGL((pdq_match_held_kernel<kPer, false>), grid, block, 0, stream, rows, prefix, n_rows, q,
+                       n_queries, threshold, hits, capacity, counter, index_base, plan);
+  return hipGetLastError();
+}
+
 template <int QT>
 static hipError_t launch_even(const void* db, const void* plane, uint64_t n_rows, const void* queries,
                               uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
@@ -1576,6 +1864,16 @@ MatchPlan match_plan(uint64_t n_rows, uint32_t n_queries) {
   return plan;
 }
 
+// The held-rows layout takes databases up to 7x10^5 rows from 193 queries, and
+// up to 5x10^4 from 65: at its lines (even layout / held, us) 7x10^5 rows x 200
+// queries 15.8 / 14.0 and x 2048 69.4 / 63.3, but 10^6 rows x 256 19.9 / 22.4;
+// 5x10^5 rows x 160 queries 11.1 / 12.7, x 200 13.5 / 13.5; 10^4 rows x 97
+// queries 9.5 / 9.2, 10^3 rows x 65 13.5 / 9.1.  Raw rows and thresholds with
+// two products per accumulator lie the same or a little further in its favour.
+static bool held_pays(uint64_t n_rows, uint32_t n_queries) {
+  return n_rows <= 700000 && n_queries > (n_rows <= 50000 ? 64u : 192u);
+}
+
 static hipError_t launch_match_mfma_any(const void* db, const void* plane, uint64_t n_rows, const void* queries,
                                         uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
                                         unsigned long long* counter, uint64_t index_base, hipStream_t stream,
@@ -1585,6 +1883,13 @@ static hipError_t launch_match_mfma_any(const void* db, const void* plane, uint6
     if (!reset_counter) return hipSuccess;
     hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(1), 0, stream, nullptr, counter);
     return hipGetLastError();
+  }
+  if (held_pays(n_rows, n_queries)) {
+    return threshold >= kTriMinThreshold
+               ? launch_held<3>(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base,
+                                stream, reset_counter)
+               : launch_held<2>(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base,
+                                stream, reset_counter);
   }
   const MatchPlan plan = match_plan(n_rows, n_queries);
   if (plan.shared) {
