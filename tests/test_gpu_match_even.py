@@ -122,3 +122,29 @@ def test_shards_around_their_groups(gpu, oracle, dev, nq):
             assert total == n and np.array_equal(triples(hits), want), threshold
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("nq", [11, 12, 13, 15, 16, 17, 24, 31])
+def test_fewer_than_two_tiles(gpu, oracle, dev, nq):
+    """The matrix cores take 12 queries and more up to threshold 40; both sides
+    of the line, single database and shards, against the oracle."""
+    import torch
+    assert gpu.match_uses_matrix_cores(nq, 40) == (nq >= 12) and not gpu.match_uses_matrix_cores(nq, 41)
+    queries = synthetic.random_db(nq, seed=nq)
+    q = torch.from_numpy(queries).to(dev)
+    for n_rows in (1, 63, 257, 5000):
+        db = planted(n_rows, queries, 70 + n_rows)
+        d = torch.from_numpy(db).to(dev)
+        plane = gpu.build_prefix_plane(d)
+        s = gpu.Shards()
+        try:
+            s.add(db[:n_rows // 3 + 1])
+            if n_rows > 1:
+                s.add(db[n_rows // 3 + 1:])
+            for threshold in (16, 31, 40, 41):
+                n, want = oracle.match_all(db, queries, threshold)
+                for total, hits in (gpu.match(d, q, threshold), gpu.match(d, q, threshold, plane=plane),
+                                    s.match(q, threshold)):
+                    assert total == n and np.array_equal(triples(hits), want), (n_rows, threshold)
+        finally:
+            s.close()

@@ -473,10 +473,9 @@ MatcherChoice BatchContext::choice_for(uint32_t nq) const {
       c.qt = best;
     }
   } else {
-    // without tuning: vector ALU below 32 queries, on the matrix cores from 32
-    // the single-database matcher's plan
+    // without tuning: the single-database matcher's choice and plan
     const MatchPlan plan = match_plan(shards_->total_rows(), nq);
-    c.mfma = threshold_ < 64 && nq >= 32;
+    c.mfma = match_mfma_applicable(nq, threshold_);
     c.qt = plan.shared ? 16 : plan.qt;
   }
   set_layout(&c, shards_->total_rows(), nq);

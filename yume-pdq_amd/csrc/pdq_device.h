@@ -150,7 +150,8 @@ hipError_t launch_match_plane_tuned(const MatchTuning& t, const void* db, const 
 hipError_t launch_match_plane(const void* db, const void* plane, uint64_t n_rows, const void* queries,
                               uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
                               unsigned long long* counter, uint64_t index_base, hipStream_t stream);
-// Matrix-core prefix filter + exact re-check (threshold < 64, >= 32 queries).
+// Matrix-core prefix filter + exact re-check: from 32 queries (threshold < 64),
+// or 12 (threshold <= 40).
 bool match_mfma_applicable(uint32_t n_queries, uint32_t threshold);
 // plane: the database's prefix plane (launch_build_prefix_plane), or null to
 // read the raw rows.  reset_counter: zero *counter first, in the one-thread

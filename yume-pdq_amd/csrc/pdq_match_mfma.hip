@@ -12,7 +12,7 @@
 // re-checked pair by pair with the full 256-bit integer distance, so the
 // result is the exact set the reference defines -- the matrix pass is only a
 // filter that can never drop a pair.  Used for t < 64 (above that the prefix
-// bound passes everything) and batches of >= 32 queries.
+// bound passes everything) and batches of 32 queries, 12 at threshold <= 40.
 //
 // Operand layout (measured on gfx950): lane l holds row/column (l & 15) and
 // K quarter (l >> 4), i.e. 32 fp4 values = one 32-bit word of the 128-bit
@@ -1831,7 +1831,15 @@ hipError_t launch_match_shared_shards(const ShardView* shards, uint32_t n_shards
   return hipGetLastError();
 }
 
-bool match_mfma_applicable(uint32_t n_queries, uint32_t threshold) { return threshold < 64 && n_queries >= 32; }
+// From 12 queries the one group of two query tiles, mostly padding, costs less
+// than the vector-ALU scan, which pays per query, as long as candidates are
+// rare.  10^7 rows over the plane, vector ALU / matrix cores in us: 8 queries
+// 27 / 31, 12 36 / 31, 16 46 / 31, 24 65 / 32, 31 82 / 31 at threshold 31; 16
+// queries 46 / 35 at 40, 48 / 57 at 44 and 65 / 144 at 48 (raw rows cross at 16
+// queries, 53 / 51; below 10^6 rows both are one launch).
+bool match_mfma_applicable(uint32_t n_queries, uint32_t threshold) {
+  return n_queries >= 32 ? threshold < 64 : n_queries >= 12 && threshold <= 40;
+}
 
 // Which layout a call runs, and its query tiles per wave.  Costs, in tenths of
 // a query tile's products over all rows (0.45 us per 10^7 rows), fitted to
