@@ -44,3 +44,33 @@ def test_lists_of_every_length(gpu, dev, n):
         assert total == 0 and len(hits) == 0
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 5, 300])
+def test_hash_launch_clears_the_count(gpu, dev, n):
+    """The counter of a hash-and-match batch starts from garbage, in every hash
+    layout and on repeated runs, with rows and without."""
+    import torch
+    planes = torch.from_numpy(synthetic.images_u8(8)).to(dev).repeat((n + 7) // 8, 1, 1)[:n].contiguous()
+    h = gpu.hash_batch(planes)[0].reshape(-1, 32)
+    rows = torch.cat([h[:5], torch.from_numpy(synthetic.random_db(100, seed=3)).to(dev)])
+    want, want_hits = gpu.match(rows, h, 10)
+    hm = gpu.HashMatch(planes, rows, 10)
+    empty = gpu.HashMatch(planes, rows[:0], 10)
+    for _ in range(3):
+        hm.count.fill_(77)
+        empty.count.fill_(77)
+        assert hm.run() == want > 0 and np.array_equal(hm.results()[1], want_hits)
+        assert empty.run() == 0 and int(empty.count) == 0
+    s = gpu.Shards()
+    s.add(rows)
+    b = gpu.Batcher(s, 300, threshold=10)
+    try:
+        for use_graph in (True, False, True):
+            b.count.fill_(77)
+            torch.cuda.synchronize()
+            _, _, _, total, hits = b.run(planes, use_graph=use_graph)
+            assert total == want and np.array_equal(hits, want_hits)
+    finally:
+        b.close()
+        s.close()

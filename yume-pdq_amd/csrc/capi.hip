@@ -462,10 +462,24 @@ int yume_pdq_amd_hash_match_batch(const void* d_planes, int input_kind, uint64_t
     }
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  int rc = yume_pdq_amd_hash_batch(d_planes, input_kind, plane_stride_bytes, n_images, dihedral_mode, d_hashes,
-                                   d_quality, d_threshold, nullptr, stream);
+  // the hash launch clears the counter; no images, and the matcher does
+  uint32_t flags = 0;
+  int rc = YUME_PDQ_AMD_OK;
+  if (n_images) {
+    HashOutputs o;
+    o.hashes = d_hashes;
+    o.quality = d_quality;
+    o.threshold = d_threshold;
+    o.pdqf = nullptr;
+    o.buf1 = nullptr;
+    o.tmp = nullptr;
+    o.dihedral_pdqf = nullptr;
+    o.clear = d_count;
+    rc = from_hip(ypdq::launch_hash(d_planes, input_kind, plane_stride_bytes, n_images, dihedral_mode, o, st));
+    flags = YUME_PDQ_AMD_MATCH_APPEND;
+  }
   if (rc == YUME_PDQ_AMD_OK)
-    rc = match_impl(d_db, d_plane, n_rows, d_hashes, 8 * n_images, threshold, d_hits, capacity, d_count, 0, 0,
+    rc = match_impl(d_db, d_plane, n_rows, d_hashes, 8 * n_images, threshold, d_hits, capacity, d_count, 0, flags,
                     stream);
   if (rc == YUME_PDQ_AMD_OK && d_h_count) {
     hipLaunchKernelGGL(store_count, dim3(1), dim3(1), 0, st, d_count, d_h_count);

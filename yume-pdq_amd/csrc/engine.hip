@@ -490,10 +490,9 @@ hipError_t BatchContext::enqueue_body(const MatcherChoice& c, hipStream_t s) {
   o.hashes = d_hashes_;
   o.quality = d_quality_;
   o.threshold = d_threshold_;
+  o.clear = d_count_;
   hipError_t e = launch_hash_device_count(d_input_, input_kind_, plane_stride_, max_images_, d_sizes_, mode_, o, s);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(1), 0, s, d_count_, 0ull);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
   return shards_->launch_match(c, d_hashes_, d_sizes_ + 1, max_images_ * 8, threshold_,
                                reinterpret_cast<MatchHit*>(d_hits_), hit_capacity_, d_count_, s, d_records_);
 }

@@ -277,6 +277,7 @@ template <typename T, int kW, int D>
 __global__ void __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(kW >= 16 ? 4 : std::is_same<T, float>::value ? 2 : 3))) pdq_hash_kernel(
     const T* __restrict__ planes, uint64_t plane_stride, uint32_t n_images, const uint32_t* __restrict__ d_n,
     uint32_t mode, HashOutputs out, Luma lc) {
+  if (out.clear && blockIdx.x == 0 && threadIdx.x == 0) *out.clear = 0;
   const uint32_t n = d_n ? min(*d_n, n_images) : n_images;
   if (blockIdx.x * kW >= n) return;
   __shared__ BlockLdsOf<kW> L;

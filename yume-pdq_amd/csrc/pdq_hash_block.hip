@@ -396,6 +396,7 @@ __global__ void __launch_bounds__(64 * kWaves) pdq_hash_block_kernel(const T* __
   static_assert(kWaves == 4 || kWaves == 8 || kWaves == 16, "four, eight or sixteen waves per image");
   static_assert(kWaves <= 8 || kPrec == kDctExact, "sixteen waves: exact arithmetic only");
   constexpr int kBand = (127 + kWaves - 1) / kWaves;  // compressed rows per wave
+  if (out.clear && blockIdx.x == 0 && threadIdx.x == 0) *out.clear = 0;
   const uint32_t n = d_n ? min(*d_n, n_images) : n_images;
   const uint32_t img = blockIdx.x;
   if (img >= n) return;
