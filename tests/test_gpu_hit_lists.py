@@ -74,3 +74,32 @@ def test_hash_launch_clears_the_count(gpu, dev, n):
     finally:
         b.close()
         s.close()
+
+
+def test_batches_enqueued_without_waiting(gpu, dev):
+    """Batches of different sizes enqueued one behind the other, with the shard
+    set replaced in between (its graphs are captured again): each has its own
+    size and count."""
+    import torch
+    planes = torch.from_numpy(synthetic.images_u8(64)).to(dev)
+    h = gpu.hash_batch(planes)[0].reshape(-1, 32)
+    rows = torch.cat([h[::3], torch.from_numpy(synthetic.random_db(1000, seed=4)).to(dev)])
+    sizes = [1, 64, 7, 2, 33, 64, 5, 1, 16, 50]
+    want = [gpu.match(rows, h[:8 * n], 20)[0] for n in sizes]
+    s = gpu.Shards()
+    s.add(rows)
+    b = gpu.Batcher(s, 64, threshold=20)
+    try:
+        for turn in range(3):
+            got = []
+            for n in sizes:
+                b.run(planes[:n], sync=False)
+                with torch.cuda.stream(b.stream):
+                    got.append(b.count.clone())
+            if turn == 1:  # a shard without a near row: the counts stay, the graphs do not
+                s.add(torch.zeros((9, 32), dtype=torch.uint8, device=dev))
+            b.stream.synchronize()
+            assert [int(c) for c in got] == want, turn
+    finally:
+        b.close()
+        s.close()

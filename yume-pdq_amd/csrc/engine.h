@@ -134,10 +134,9 @@ class BatchContext {
   hipError_t init(std::shared_ptr<ShardSet> shards, uint32_t max_images, int input_kind, uint32_t mode,
                   uint32_t threshold, uint64_t hit_capacity);
   // Hash input[0 .. n_images) and match the 8n hashes against every shard,
-  // enqueued on stream() (a graph replay unless use_graph is false).  Waits
-  // for this context's previous batch first unless the caller knows it is
-  // done (wait_previous = false).
-  hipError_t run(uint32_t n_images, bool use_graph, bool wait_previous = true);
+  // enqueued on stream() behind this context's previous batch (a graph replay
+  // unless use_graph is false).
+  hipError_t run(uint32_t n_images, bool use_graph);
   // Times the matchers per query-count bucket and stores the fastest in the
   // process-wide tuning cache, under the shard set's current shape.
   hipError_t autotune(int iterations, std::vector<TuneRecord>* records);
@@ -175,6 +174,7 @@ class BatchContext {
     hipGraphExec_t exec = nullptr;
     uint64_t version = 0;
   };
+  hipError_t set_sizes(uint32_t images, uint32_t queries);
   hipError_t enqueue_body(const MatcherChoice& c, hipStream_t s);
   hipError_t graph_for(const MatcherChoice& c, hipGraphExec_t* exec);
   void refresh_choices() const;
@@ -195,7 +195,6 @@ class BatchContext {
   void* d_hits_ = nullptr;
   unsigned long long* d_count_ = nullptr;
   uint32_t* d_sizes_ = nullptr;  // device {n_images, n_queries}
-  uint32_t* h_sizes_ = nullptr;  // pinned staging of the same
   void* d_records_ = nullptr;    // the shared-rows matcher's candidate records
   // the cache's choices for key_, read at tune generation gen_
   mutable TuneChoices choices_;

@@ -246,7 +246,7 @@ hipError_t Server::enqueue_batch(Slot& s, bool in_order) {
   hipError_t e = hipEventRecord(s.uploaded, upload_);
   if (e == hipSuccess) e = hipStreamWaitEvent(c.stream(), s.uploaded, 0);
   if (e == hipSuccess && in_order && last_computed_) e = hipStreamWaitEvent(c.stream(), last_computed_, 0);
-  if (e == hipSuccess) e = c.run(s.n_images, cfg_.use_graph, /*wait_previous=*/false);
+  if (e == hipSuccess) e = c.run(s.n_images, cfg_.use_graph);
   if (e == hipSuccess) e = hipEventRecord(s.computed, c.stream());
   if (e == hipSuccess && in_order) last_computed_ = s.computed;
   if (e == hipSuccess) {
