@@ -102,3 +102,21 @@ def test_automatic_layout_around_its_lines(gpu, dev, per_cu):
         got = gpu.hash_batch(x[n - m:])
         for a, b in zip(got, want):
             assert torch.equal(a, b[n - m:])
+
+
+@pytest.mark.parametrize("kind", ["u8", "f32", "rgb8", "rgba8"])
+def test_automatic_layout_of_small_batches(gpu, dev, kind):
+    """Batches on both sides of the change from sixteen waves to eight equal the
+    wave form's."""
+    import torch
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    n = {"u8": cus // 32, "f32": 1, "rgb8": cus // 8 * 3, "rgba8": cus // 8}[kind] + 1
+    x = torch.from_numpy(synthetic.images_u8(16)).to(dev).repeat((n + 15) // 16, 1, 1)[:n].contiguous()
+    if kind == "f32":
+        x = x.to(torch.float32) * 0.75
+    elif kind != "u8":
+        x = torch.stack([x, 255 - x, x // 2, x][:3 if kind == "rgb8" else 4], 3).contiguous()
+    want = gpu.hash_batch(x, layout=gpu.LAYOUT_WAVE)
+    for m in (n, n - 1):
+        for a, b in zip(gpu.hash_batch(x[n - m:]), want):
+            assert torch.equal(a, b[n - m:])

@@ -327,7 +327,7 @@ int yume_pdq_amd_hash_batch_ex(const void* d_planes, int input_kind, uint64_t pl
   const hipStream_t s = static_cast<hipStream_t>(stream);
   int layout = (int)o.layout;
   if (layout == YUME_PDQ_AMD_LAYOUT_AUTO) {
-    const int a = ypdq::hash_layout_for(n_images, (int)o.dct_precision);
+    const int a = ypdq::hash_layout_for(n_images, input_kind, (int)o.dct_precision);
     layout = a == 1 ? YUME_PDQ_AMD_LAYOUT_WAVE : a == 16 ? YUME_PDQ_AMD_LAYOUT_BLOCK16 : YUME_PDQ_AMD_LAYOUT_BLOCK8;
   }
   if (layout == YUME_PDQ_AMD_LAYOUT_WAVE)

@@ -77,7 +77,7 @@ hipError_t launch_hash_block(const void* planes, int input_kind, uint64_t plane_
                              const float* luma, hipStream_t stream);
 // Layout the automatic choice uses for n images: 1 = wave per image,
 // 8 = block of eight waves per image.
-int hash_layout_for(uint32_t n_images, int dct);
+int hash_layout_for(uint32_t n_images, int input_kind, int dct);
 // The precise ReferenceKernel<f32> (f32 or u8 planes): hash, quality,
 // threshold (the median) and PDQF of the NORMAL orientation per image;
 // `work` holds hash_ref_workspace_bytes(n) bytes of scratch.

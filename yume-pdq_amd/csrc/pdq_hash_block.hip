@@ -567,12 +567,19 @@ int device_cus() {
 
 }  // namespace
 
-int hash_layout_for(uint32_t n_images, int dct) {
-  // Exact arithmetic: sixteen waves per image while the images fit one per
-  // CU, then eight, until the batch is large enough that a wave per image
-  // fills the GPU with less LDS per image.  The lines cross at 5.5 images per
-  // CU (u8 and RGB8 a little above, f32 and RGBA8 there); eight waves / a wave
-  // per image, in us:
+int hash_layout_for(uint32_t n_images, int input_kind, int dct) {
+  // Exact arithmetic: blocks of sixteen waves while a handful of images leaves
+  // most CUs to themselves and the rows' conversion is what their waves do,
+  // then eight, until the batch is large enough that a wave per image fills the
+  // GPU with less LDS per image.  Sixteen / eight waves, in us:
+  //   images          1           32           64          128          256
+  //   u8       14.9 / 15.0  17.6 / 16.9  18.2 / 17.2  19.0 / 17.6  23.6 / 21.1
+  //   f32      17.7 / 16.9  19.1 / 18.4  23.4 / 22.1  30.5 / 28.7  55.0 / 51.6
+  //   RGB8     21.1 / 22.0  22.0 / 22.9  22.6 / 23.5  27.0 / 24.3  44.9 / 38.9
+  //   RGBA8    19.5 / 20.2  20.5 / 21.2  24.5 / 22.1  32.2 / 28.6  57.1 / 50.7
+  // (u8 crosses between 8 and 16 images, RGB8 at 96, RGBA8 between 32 and 48.)
+  // The upper lines cross at 5.5 images per CU (u8 and RGB8 a little above,
+  // f32 and RGBA8 there); eight waves / a wave per image:
   //   images      1100        1365        1536        2048
   //   u8        75 / 91     88 / 92     93 / 95   120 / 108
   //   RGB8     167 / 202   201 / 226   215 / 230   282 / 292
@@ -582,12 +589,16 @@ int hash_layout_for(uint32_t n_images, int dct) {
   if (dct != kDctExact) return 8;
   const uint32_t cus = (uint32_t)std::max(0, device_cus());
   if (cus == 0) return n_images > 1024 ? 1 : 8;
-  return n_images <= cus ? 16 : n_images <= cus * 11 / 2 ? 8 : 1;
+  const uint32_t sixteen = input_kind == kInputU8      ? cus / 32
+                           : input_kind == kInputRgb8  ? cus / 8 * 3
+                           : input_kind == kInputRgba8 ? cus / 8
+                                                       : 0;
+  return n_images <= sixteen ? 16 : n_images <= cus * 11 / 2 ? 8 : 1;
 }
 
 hipError_t launch_hash(const void* planes, int input_kind, uint64_t plane_stride, uint32_t n_images, uint32_t mode,
                        const HashOutputs& out, hipStream_t stream, const float* luma) {
-  const int layout = hash_layout_for(n_images, kDctExact);
+  const int layout = hash_layout_for(n_images, input_kind, kDctExact);
   if (layout == 1)
     return launch_hash_wave(planes, input_kind, plane_stride, n_images, nullptr, mode, out, luma, stream);
   return launch_hash_block(planes, input_kind, plane_stride, n_images, nullptr, mode, kDctExact, layout, out, luma,
@@ -596,7 +607,7 @@ hipError_t launch_hash(const void* planes, int input_kind, uint64_t plane_stride
 
 hipError_t launch_hash_device_count(const void* planes, int input_kind, uint64_t plane_stride, uint32_t n_max,
                                     const uint32_t* d_n, uint32_t mode, const HashOutputs& out, hipStream_t stream) {
-  const int layout = hash_layout_for(n_max, kDctExact);
+  const int layout = hash_layout_for(n_max, input_kind, kDctExact);
   if (layout == 1)
     return launch_hash_wave(planes, input_kind, plane_stride, n_max, d_n, mode, out, nullptr, stream);
   return launch_hash_block(planes, input_kind, plane_stride, n_max, d_n, mode, kDctExact, layout, out, nullptr,
