@@ -148,3 +148,24 @@ def test_fewer_than_two_tiles(gpu, oracle, dev, nq):
                     assert total == n and np.array_equal(triples(hits), want), (n_rows, threshold)
         finally:
             s.close()
+
+
+# every number of tiles from three to sixteen in one group, and two groups of an
+# odd number, over more rows than the held-rows layout takes
+@pytest.mark.parametrize("nq", [48, 49, 80, 97, 113, 129, 145, 161, 177, 193, 209, 225, 241, 280])
+def test_every_width_over_many_rows(gpu, dev, nq):
+    import torch
+    n = 60_001 if nq <= 192 else 700_101
+    g = torch.Generator(device=dev).manual_seed(nq)
+    db = torch.randint(-(1 << 63), (1 << 63) - 1, (n, 4), generator=g, device=dev).view(torch.uint8).reshape(n, 32)
+    q = torch.from_numpy(synthetic.random_db(nq, seed=13)).to(dev)
+    at = torch.randperm(n, generator=g, device=dev)[:2000]
+    db[at] = q[torch.arange(2000, device=dev) % nq] ^ (torch.randint(0, 256, (2000, 1), generator=g, device=dev)
+                                                       .to(torch.uint8) & 19)
+    db[0], db[n - 1] = q[0], q[nq - 1]
+    plane = gpu.build_prefix_plane(db)
+    for threshold in (27, 28):
+        n0, h0 = gpu.match(db, q, threshold, path="valu")
+        for p in (None, plane):
+            n1, h1 = gpu.match(db, q, threshold, plane=p)
+            assert n0 == n1 > 0 and np.array_equal(triples(h0), triples(h1)), (threshold, p is not None)

@@ -420,7 +420,7 @@ static void set_layout(MatcherChoice* c, uint64_t rows, uint32_t nq) {
   if (!c->mfma) return;
   const int tiles = (int)std::max<uint32_t>(1, (nq + 15) / 16);
   const int groups = (tiles + c->qt - 1) / c->qt;
-  c->width = ((tiles + groups - 1) / groups + 1) / 2 * 2;
+  c->width = std::max(2, (tiles + groups - 1) / groups);
   c->shared = c->qt == 16 && match_plan(rows, nq).shared;
 }
 

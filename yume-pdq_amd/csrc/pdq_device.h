@@ -117,7 +117,7 @@ struct ShardView {
 uint64_t mfma_chunks(uint64_t n_rows);       // shared-rows chunks of one shard (multiple of 8)
 uint64_t match_row_groups(uint64_t n_rows);  // the even layout's row groups of one shard
 // The matrix-core matcher for n_queries over n_rows rows: the shared-rows
-// layout, or the even layout with qt (2, 4, .. 16) query tiles per wave.
+// layout, or the even layout with qt (2 .. 16) query tiles per wave.
 struct MatchPlan {
   bool shared;
   int qt;
