@@ -798,9 +798,8 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
 // The even layout holds query tiles in registers and streams rows past them;
 // with few rows a part is a handful of loads, and a wave's time the latency of
 // loading and expanding its 256 queries first.  Here a block expands up to 64
-// query tiles into LDS once, together, and each of its waves holds 192 rows
-// (128 below the threshold of three products per accumulator) and runs all the
-// tiles past them: 12 products for one LDS read, no expansion in the loop.
+// query tiles into LDS once, together, and each of its waves holds 192 rows (or
+// 128, two products per accumulator) and runs all the tiles past them: 12 products for one LDS read, no expansion in the loop.
 // The prefix products, their flags and the exact check are the even layout's.
 // The matrix cores bound a wave's loop (24 products beside about 20 vector
 // instructions per pair of tiles); the launch, 9.3 us as measured, bounds the
@@ -808,8 +807,8 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
 //
 // Kernel times with the reset, even layout / here, us:
 //   rows       256         512        1000        2048 queries
-//   10^4    19.1 /  9.2  20.7 /  9.2  23.9 / 12.5  29.0 / 17.4
-//   10^5    11.4 /  9.7  12.5 / 10.8  17.6 / 13.1  26.3 / 19.8
+//   10^4    19.1 /  8.7  20.7 /  8.7  23.9 /  9.6  29.0 / 13.4
+//   10^5    11.4 /  9.2  12.5 / 10.8  17.6 / 13.1  26.3 / 19.9
 //   3x10^5  14.9 / 12.0  17.8 / 15.6  24.0 / 22.3  43.5 / 37.1
 //   7x10^5  17.4 / 15.7  24.0 / 22.4  38.1 / 35.4  69.4 / 63.3
 // ---------------------------------------------------------------------------
@@ -1007,15 +1006,21 @@ __device__ __forceinline__ void held_rows(HeldLds& S, const uint4* __restrict__ 
 // block holding one of them; a wave's rows are `groups` row groups.
 struct HeldPlan {
   uint32_t chunks, tiles, groups, blocks_per_xcd;  // blocks per XCD and chunk
+  uint64_t cost;
 };
-// The cut that costs least, by a wave's products (12 of 18.1 cycles and their
-// share of the rest per tile and row group, and about two tiles' time for
-// loading and expanding the rows of a group), times the blocks that share a CU.
-// cus: of one XCD; two blocks are resident on each (72 KiB of LDS).
-inline HeldPlan held_plan(uint64_t row_groups, uint32_t tiles, uint32_t cus) {
+// The cut that costs least, in cycles of a wave: its products (12 or 8 of 18.1
+// cycles and their share of the rest per tile and row group), about two tiles'
+// time for loading and expanding the rows of a group, times the blocks that
+// share a CU, and the queries' expansion.  kPer = 2 is rated a little higher
+// than it measures alone: at equal costs it lost 5 % (7x10^5 rows x 2048 queries
+// 63.8 / 67.8 us).  cus: of one XCD; two blocks are resident on each (72 KiB of
+// LDS).
+template <int kPer>
+HeldPlan held_plan(uint64_t n_rows, uint32_t tiles, uint32_t cus) {
+  constexpr uint64_t kTile = kPer == 3 ? 224 : 166, kGroup = kPer == 3 ? 464 : 330;
+  const uint64_t row_groups = (n_rows + Held<kPer>::kRows - 1) / Held<kPer>::kRows;
   const uint32_t blocks_per_xcd = 2 * cus;
-  HeldPlan best{1, 1, 1, 1};
-  uint64_t least = ~0ull;
+  HeldPlan best{1, 1, 1, 1, ~0ull};
   const uint32_t first = (tiles + kHeldTiles - 1) / kHeldTiles;
   for (uint32_t c = first; c < 2 * first + 16 && c <= tiles; c++) {
     const uint32_t t = (tiles + c - 1) / c;
@@ -1024,11 +1029,8 @@ inline HeldPlan held_plan(uint64_t row_groups, uint32_t tiles, uint32_t cus) {
     const uint64_t g = (row_groups + waves - 1) / waves;
     const uint64_t need = (row_groups + g * 8 * kHeldWaves - 1) / (g * 8 * kHeldWaves);  // blocks per XCD
     const uint64_t per_cu = (need * c + cus - 1) / cus;
-    const uint64_t cost = g * ((uint64_t)t * 224 + 464) * per_cu + t * 64;
-    if (cost < least) {
-      least = cost;
-      best = HeldPlan{c, t, (uint32_t)g, (uint32_t)need};
-    }
+    const uint64_t cost = g * (t * kTile + kGroup) * per_cu + t * 64;
+    if (cost < best.cost) best = HeldPlan{c, t, (uint32_t)g, (uint32_t)need, cost};
   }
   return best;
 }
@@ -1701,15 +1703,10 @@ static uint32_t even_waves_per_xcd(int cus) { return (uint32_t)std::max(1, cus) 
 
 // The even layout's launch.
 template <int kPer>
-static hipError_t launch_held(const void* db, const void* plane, uint64_t n_rows, const void* queries,
-                              uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
-                              unsigned long long* counter, uint64_t index_base, hipStream_t stream, bool reset) {
-  int dev = 0, cus = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
-  const uint64_t row_groups = (n_rows + Held<kPer>::kRows - 1) / Held<kPer>::kRows;
-  const HeldPlan plan = held_plan(row_groups, (n_queries + 15) / 16, (uint32_t)std::max(8, cus) / 8);
+static hipError_t launch_held_plan(const HeldPlan& plan, const void* db, const void* plane, uint64_t n_rows,
+                                   const void* queries, uint32_t n_queries, uint32_t threshold, MatchHit* hits,
+                                   uint64_t capacity, unsigned long long* counter, uint64_t index_base,
+                                   hipStream_t stream, bool reset) {
   const dim3 grid((unsigned)(8 * plan.blocks_per_xcd * plan.chunks)), block(64 * kHeldWaves);
   const uint4* rows = static_cast<const uint4*>(db);
   const uint4* prefix = static_cast<const uint4*>(plane);
@@ -1722,6 +1719,26 @@ static hipError_t launch_held(const void* db, const void* plane, uint64_t n_rows
     hipLaunchKernelGGL((pdq_match_held_kernel<kPer, false>), grid, block, 0, stream, rows, prefix, n_rows, q,
                        n_queries, threshold, hits, capacity, counter, index_base, plan);
   return hipGetLastError();
+}
+
+static hipError_t launch_held(const void* db, const void* plane, uint64_t n_rows, const void* queries,
+                              uint32_t n_queries, uint32_t threshold, MatchHit* hits, uint64_t capacity,
+                              unsigned long long* counter, uint64_t index_base, hipStream_t stream, bool reset) {
+  int dev = 0, cus = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+  const uint32_t per_xcd = (uint32_t)std::max(8, cus) / 8, tiles = (n_queries + 15) / 16;
+  const HeldPlan two = held_plan<2>(n_rows, tiles, per_xcd), three = held_plan<3>(n_rows, tiles, per_xcd);
+  // two products per accumulator serve every threshold; three take fewer
+  // instructions a product, but hold 192 rows a wave, which leaves small
+  // databases with fewer waves (10^4 rows x 2048 queries, three / two: 17.4 /
+  // 13.4 us, 3x10^4 x 2048 16.1 / 11.7, 4x10^5 x 256 14.5 / 12.5)
+  if (threshold >= kTriMinThreshold && three.cost <= two.cost)
+    return launch_held_plan<3>(three, db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter,
+                               index_base, stream, reset);
+  return launch_held_plan<2>(two, db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter,
+                             index_base, stream, reset);
 }
 
 template <int QT>
@@ -1902,13 +1919,9 @@ static hipError_t launch_match_mfma_any(const void* db, const void* plane, uint6
     hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(1), 0, stream, nullptr, counter);
     return hipGetLastError();
   }
-  if (held_pays(n_rows, n_queries)) {
-    return threshold >= kTriMinThreshold
-               ? launch_held<3>(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base,
-                                stream, reset_counter)
-               : launch_held<2>(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base,
-                                stream, reset_counter);
-  }
+  if (held_pays(n_rows, n_queries))
+    return launch_held(db, plane, n_rows, queries, n_queries, threshold, hits, capacity, counter, index_base, stream,
+                       reset_counter);
   const MatchPlan plan = match_plan(n_rows, n_queries);
   if (plan.shared) {
     bool done = false;
