@@ -686,9 +686,14 @@ __device__ __forceinline__ void median_extremes_rows(const float* __restrict__ P
 // One wave alone: a dependent operation takes 8.5 cycles, an independent one
 // 4.2, and the 32 additions in order are the longest chain, so what else an
 // iteration needs is arranged to fill their gaps:
-//  - an element that leaves the range [mn, mx] never comes back and becomes
-//    NaN when it leaves, so one comparison per element and iteration selects
-//    (not two and their AND);
+//  - an element that leaves the range [mn, mx] becomes NaN when it leaves, so
+//    one comparison per element and iteration selects (not two and their AND).
+//    That holds while the range narrows.  A guess is a mean of rounded sums
+//    and, where elements lie within a few ulps of each other, can fall behind
+//    the bound it replaces: the range widens, and elements that had left are
+//    in it again.  A lane compares each guess with its side's bound, and where
+//    one lies outside, the search is run anew by median_search8, which tests
+//    both bounds each time;
 //  - the counts decide the side, and the reciprocal of each side's count is
 //    refined, while the sums are under way; behind them remain the five
 //    operations of a correctly rounded quotient (q = s y, then twice q +=
@@ -701,6 +706,7 @@ __device__ __forceinline__ void median_search_rows(const float* __restrict__ P, 
                                                    float& bit_threshold) {
   const int l = lane & 7;
   const bool lower_side = (lane & 8) != 0;
+  constexpr uint64_t kLowerSides = 0xff00ff00ff00ff00ull;  // its lanes
   const uint32_t sign = lower_side ? 0x80000000u : 0u;
   const int row = lane >> 4;
   const int run = row ^ (row >> 1);
@@ -710,22 +716,23 @@ __device__ __forceinline__ void median_search_rows(const float* __restrict__ P, 
   float mx, mn;
   median_extremes_rows(P, x, lane, mx, mn);
   const float kGone = __builtin_nanf("");
-  {
-    const float hi = lower_side ? -mn : mx;
+  float hi = lower_side ? -mn : mx;  // this side's bound
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const float v = __uint_as_float(__float_as_uint(x[e]) ^ sign);
-      x[e] = v <= hi ? v : kGone;
-    }
+  for (int e = 0; e < 8; e++) {
+    const float v = __uint_as_float(__float_as_uint(x[e]) ^ sign);
+    x[e] = v <= hi ? v : kGone;
   }
   float guess = (mn + mx) * 0.5f;
   float last = guess;
   uint32_t num_over = 0, num_under = 0;
+  uint64_t outside = 0;
 #pragma unroll 1
   for (int iter = 0; iter < 32; iter++) {
     // this lane's side: (guess, mx] above, or [mn, guess) below (negated)
     const float lo = __uint_as_float(__float_as_uint(guess) ^ sign);
-    bool m[8];
+    outside |= __ballot(!(lo <= hi));
+    asm volatile("" : "+s"(outside));  // here: merged at the loop's end it costs two branches per turn
+    uint64_t m[8];  // lane masks, kept for the elements that leave
     float s[8];
     uint32_t n = 0;
     // the sequential sum, run after run; `between` is what fills its gaps
@@ -740,9 +747,10 @@ __device__ __forceinline__ void median_search_rows(const float* __restrict__ P, 
     };
 #pragma unroll
     for (int e = 0; e < 8; e++) {
-      m[e] = x[e] > lo;
-      s[e] = m[e] ? x[e] : 0.0f;
-      n += m[e] ? 1u : 0u;
+      m[e] = __ballot(x[e] > lo);
+      const bool in = __builtin_amdgcn_inverse_ballot_w64(m[e]);
+      s[e] = in ? x[e] : 0.0f;
+      n += in ? 1u : 0u;
       acc = acc + s[e];
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -778,7 +786,7 @@ __device__ __forceinline__ void median_search_rows(const float* __restrict__ P, 
     const bool up = gtc + num_over > 128;
     const bool down = ltc + num_under > 128;
     // up: mn becomes the guess and what lies below it goes; down: mx, above
-    const bool goes = lower_side == up;
+    const uint64_t goes = up ? kLowerSides : ~kLowerSides;
     acc = __uint_as_float(
         __builtin_amdgcn_permlane16_swap(__float_as_uint(acc), __float_as_uint(acc), false, false)[1]);
     float fix = 0.0f;
@@ -788,7 +796,11 @@ __device__ __forceinline__ void median_search_rows(const float* __restrict__ P, 
         y = __builtin_fmaf(fix, y, y);
         asm volatile("" : "+v"(y));  // not moved behind the sums
       }
-      x[e] = m[e] && goes ? kGone : x[e];
+      if (e == 4) {
+        hi = __builtin_amdgcn_inverse_ballot_w64(goes) ? lo : hi;
+        asm volatile("" : "+v"(hi));
+      }
+      x[e] = __builtin_amdgcn_inverse_ballot_w64(m[e] & goes) ? kGone : x[e];
       asm volatile("" : "+v"(x[e]));
     });
     const float sum = grp_sum8(acc);  // the AVX tree; row 2 holds the whole sums
@@ -811,6 +823,7 @@ __device__ __forceinline__ void median_search_rows(const float* __restrict__ P, 
   }
   threshold = guess;
   bit_threshold = last;
+  if (__builtin_expect(outside != 0, 0)) median_search8(P, lane, threshold, bit_threshold);
 }
 
 // Byte b (0..31) of the hash of P at bit threshold t: bit k is
