@@ -373,13 +373,15 @@ int yume_pdq_amd_shards_match(const YumePdqAmdShards *shards, const uint8_t *d_q
 
 /*
  * Batch context: device buffers for up to max_images planes and their
- * outputs, and one HIP graph per matcher choice holding the hash kernel, the
- * hit-counter reset and a persistent matcher over every shard.  Both kernels
- * read the batch size from device memory, so a batch of any size replays the
- * same graph.  run() enqueues on the context's own stream (it first waits
- * for the context's previous batch); read the outputs after synchronising
- * that stream.  Contexts over one shard set may run concurrently on their
- * streams.
+ * outputs, and one HIP graph per matcher choice holding the hash kernel, which
+ * also clears the hit counter, and a persistent matcher over every shard.  Both
+ * kernels read the batch size from device memory, so a batch of any size
+ * replays the same graph.  run() enqueues on the context's own stream and
+ * returns when everything enqueued on that stream before the call has
+ * completed: the context's previous batch, the copies into d_input (whose
+ * source may then be refilled or freed) and those out of the previous batch's
+ * outputs.  Read the new outputs after synchronising the stream.  Contexts over
+ * one shard set may run concurrently on their streams.
  */
 typedef struct YumePdqAmdBatcher YumePdqAmdBatcher;
 typedef struct YumePdqAmdBatchBuffers {
@@ -409,6 +411,9 @@ int yume_pdq_amd_batcher_buffers(const YumePdqAmdBatcher *b, YumePdqAmdBatchBuff
 /* Hash input planes [0, n_images) and match their 8 n_images hashes against
  * every shard (use_graph = 0 enqueues the same kernels without a graph). */
 int yume_pdq_amd_batcher_run(YumePdqAmdBatcher *b, uint32_t n_images, int use_graph);
+/* run without its wait, for callers that order the copies themselves or wait
+ * for the batch's outputs at once. */
+int yume_pdq_amd_batcher_enqueue(YumePdqAmdBatcher *b, uint32_t n_images, int use_graph);
 /* Time the vector-ALU matcher and the matrix-core matcher at 2/4/8/16 query
  * tiles per wave for query counts 8, 16, 32, ... 8 max_images on the set's
  * shards, and keep the fastest per bucket in the process-wide tuning cache:

@@ -147,6 +147,11 @@ int yume_pdq_amd_batcher_buffers(const YumePdqAmdBatcher* b, YumePdqAmdBatchBuff
 
 int yume_pdq_amd_batcher_run(YumePdqAmdBatcher* b, uint32_t n_images, int use_graph) {
   if (!b) return YUME_PDQ_AMD_EINVAL;
+  return status(b->ctx->run_after_input(n_images, use_graph != 0));
+}
+
+int yume_pdq_amd_batcher_enqueue(YumePdqAmdBatcher* b, uint32_t n_images, int use_graph) {
+  if (!b) return YUME_PDQ_AMD_EINVAL;
   return status(b->ctx->run(n_images, use_graph != 0));
 }
 

@@ -137,6 +137,9 @@ class BatchContext {
   // enqueued on stream() behind this context's previous batch (a graph replay
   // unless use_graph is false).
   hipError_t run(uint32_t n_images, bool use_graph);
+  // The same, and returns when what was on stream() before the call has
+  // completed: the previous batch, the copies into input().
+  hipError_t run_after_input(uint32_t n_images, bool use_graph);
   // Times the matchers per query-count bucket and stores the fastest in the
   // process-wide tuning cache, under the shard set's current shape.
   hipError_t autotune(int iterations, std::vector<TuneRecord>* records);
@@ -187,6 +190,7 @@ class BatchContext {
   uint64_t hit_capacity_ = 0;
   uint64_t plane_stride_ = 0;
   hipStream_t stream_ = nullptr;
+  hipEvent_t before_ = nullptr;  // run_after_input's mark on the stream
   void* d_input_ = nullptr;
   uint8_t* d_out_ = nullptr;  // the output block (see out_offset)
   uint8_t* d_hashes_ = nullptr;

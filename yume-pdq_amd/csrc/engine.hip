@@ -364,6 +364,7 @@ BatchContext::~BatchContext() {
   void* bufs[] = {d_input_, d_out_, d_sizes_, d_records_};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
+  if (before_) (void)hipEventDestroy(before_);
   if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -381,6 +382,7 @@ hipError_t BatchContext::init(std::shared_ptr<ShardSet> shards, uint32_t max_ima
   plane_stride_ = 512ull * 512 * (input_kind == kInputF32 ? 4 : 1);
   hipError_t e;
   if ((e = hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking)) != hipSuccess) return e;
+  if ((e = hipEventCreateWithFlags(&before_, hipEventDisableTiming)) != hipSuccess) return e;
   if ((e = hipMalloc(&d_input_, plane_stride_ * max_images)) != hipSuccess) return e;
   if ((e = hipMalloc(&d_out_, out_bytes(hit_capacity))) != hipSuccess) return e;
   d_count_ = reinterpret_cast<unsigned long long*>(d_out_ + out_offset(kOutCount));
@@ -566,6 +568,17 @@ hipError_t BatchContext::run(uint32_t n_images, bool use_graph) {
   hipGraphExec_t exec = nullptr;
   if ((e = graph_for(c, &exec)) != hipSuccess) return e;
   return hipGraphLaunch(exec, stream_);
+}
+
+// The wait comes behind the launch, so the GPU goes from the input copy to the
+// batch without the host, and the caller still may refill or free the copy's
+// source, or read what it downloaded of the previous batch.
+hipError_t BatchContext::run_after_input(uint32_t n_images, bool use_graph) {
+  hipError_t e = hipEventRecord(before_, stream_);
+  if (e != hipSuccess) return e;
+  e = run(n_images, use_graph);
+  const hipError_t w = hipEventSynchronize(before_);
+  return e != hipSuccess ? e : w;
 }
 
 hipError_t BatchContext::autotune(int iterations, std::vector<TuneRecord>* records) {

@@ -155,6 +155,7 @@ def lib():
                 ("yume_pdq_amd_batcher_destroy", None, [vp]),
                 ("yume_pdq_amd_batcher_buffers", i, [vp, C.POINTER(BatchBuffers)]),
                 ("yume_pdq_amd_batcher_run", i, [vp, u32, i]),
+                ("yume_pdq_amd_batcher_enqueue", i, [vp, u32, i]),
                 ("yume_pdq_amd_batcher_autotune", i, [vp, i]),
                 ("yume_pdq_amd_batcher_tune_records", i, [vp, C.POINTER(TuneRecord), u32,
                                                           C.POINTER(C.c_uint32)]),
@@ -816,7 +817,9 @@ class Batcher:
 
     def run(self, planes, use_graph=True, sync=True):
         """Copy n planes (CUDA tensor (n, 512, 512)) in and run one batch.
-        With sync, returns (hashes (n,8,32), quality, threshold, total, hits)."""
+        With sync, returns (hashes (n,8,32), quality, threshold, total, hits);
+        without, returns when the planes have been copied (they may be written
+        or freed) and the batch before this one is done."""
         torch = _torch()
         n = planes.shape[0]
         if n > self.max_images:
@@ -824,7 +827,12 @@ class Batcher:
         torch.cuda.current_stream().synchronize()  # planes written on torch's stream
         with torch.cuda.stream(self.stream):
             self.input[:n].copy_(planes)
-        _check(lib().yume_pdq_amd_batcher_run(self._h, n, 1 if use_graph else 0), "batcher_run")
+        # with sync, results() waits for the batch, and so for the copy
+        enqueue = lib().yume_pdq_amd_batcher_enqueue if sync else lib().yume_pdq_amd_batcher_run
+        rc = enqueue(self._h, n, 1 if use_graph else 0)
+        if rc:
+            self.stream.synchronize()  # the copy is under way all the same
+        _check(rc, "batcher_run")
         if not sync:
             return None
         return self.results(n)
