@@ -84,7 +84,11 @@ struct HitList {
   unsigned long long base;
 };
 constexpr uint32_t kStageHits = 4096;  // recheck kernel: two blocks per CU, about two million per launch
-constexpr uint32_t kEvenStage = 512;   // even layout
+// Even layout: four blocks per CU, two million per launch too (32 KiB each).
+// With 512 a block, 10^6 rows that each match one of 512 queries took 5.8 ms,
+// nearly all of it half a million appends of their own, and take 0.27.
+constexpr uint32_t kEvenStage = 2040;
+constexpr uint32_t kHeldStage = 512;  // held layout: what two blocks' query codes leave in LDS
 
 template <uint32_t kList>
 __device__ __forceinline__ void hits_init(HitList<kList>& L) {
@@ -879,7 +883,7 @@ __device__ __forceinline__ void held_last(const Expanded (&rows)[4 * kPer], cons
 // The block's query codes, a lane's 16 bytes of each tile side by side.
 struct HeldLds {
   u32x4 q[kHeldTiles][64];
-  HitList<kEvenStage> hits;
+  HitList<kHeldStage> hits;
 };
 
 // Codes of query tiles t0 .. t0 + n - 1 into S.q; padding queries get zero
