@@ -88,3 +88,35 @@ def test_a_hit_seldom_costs_a_global_atomic(gpu, dev):
             best = min(best, a.elapsed_time(b))
         times.append(best)
     assert (times[0] - times[1]) * 1e6 < 2 * len(want), times
+
+
+@pytest.mark.parametrize("nq", [64, 512])
+def test_runs_of_near_rows_spread_over_the_waves(gpu, dev, nq):
+    """Rows in a row that match (a film's frames) are not one wave's work: a few
+    thousand of them cost no multiple of the call without."""
+    import torch
+    n, length = 10_000_000, 5000
+    g = torch.Generator(device=dev).manual_seed(11)
+    db = torch.randint(-(1 << 63), (1 << 63) - 1, (n, 4), generator=g, device=dev).view(torch.uint8).reshape(n, 32)
+    q = torch.randint(-(1 << 63), (1 << 63) - 1, (nq, 4), generator=g, device=dev).view(torch.uint8).reshape(nq, 32)
+    plane = gpu.build_prefix_plane(db)
+    out = torch.empty((1 << 17, 16), dtype=torch.uint8, device=dev)
+    count = torch.zeros(1, dtype=torch.int64, device=dev)
+
+    def once():
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(5):
+            gpu.match(db, q, 31, plane=plane, hits=out, count=count, sync=False)
+        b.record()
+        b.synchronize()
+        return a.elapsed_time(b) / 5
+
+    without = min(once() for _ in range(5))
+    assert int(count) == 0
+    for k in range(8):
+        db[n // 9 * k + 17:][:length] = q[37 * k % nq]
+    plane = gpu.build_prefix_plane(db)
+    runs = min(once() for _ in range(5))
+    assert int(count) == 8 * length
+    assert runs < 1.7 * without, (runs, without)

@@ -646,20 +646,51 @@ __device__ __forceinline__ void even_step(const Expanded (&qa)[QT], const Expand
   if constexpr (S + 1 < kN + 4) even_step<QT, kTri, S + 1>(qa, rb, c0, acc, r0, r1, r2, r3);
 }
 
-// Exact check of the pairs of one 64-row group (base row `row0`) that reach
-// the bound.
+// A 64-row group of a database.
+struct RowGroup {
+  const uint4 *db, *plane;
+  uint64_t n_rows, index_base;
+  uint64_t row;  // its first
+};
+
+// Rows `row`, row + step, ... of a database, the prefix plane's 16 bytes or the
+// raw row's first: lane's row of the group k steps on.  Rows past the end repeat
+// the last one; their pairs are never reported.
+template <bool kPlane>
+struct GroupRows {
+  const uint4* base;  // uniform, as the rest
+  uint32_t step, left;
+  __device__ __forceinline__ GroupRows(const RowGroup& g, uint32_t stride)
+      : base(kPlane ? g.plane + g.row : g.db + 2 * g.row),
+        step(stride * kEvenRows),
+        left((uint32_t)min(g.n_rows - g.row, (uint64_t)0x7fffffffu)) {}
+  __device__ __forceinline__ uint4 load(uint32_t k, int lane) const {
+    const uint32_t r = min(k * step + (uint32_t)lane, left - 1);
+    return base[kPlane ? r : 2 * r];
+  }
+};
+
+// Row groups of one database: group k is `first` + k `stride`.
+struct DbGroups {
+  const uint4 *db, *plane;
+  uint64_t n_rows, index_base;
+  uint32_t first, stride;
+  __device__ __forceinline__ RowGroup at(uint32_t k) const {
+    return RowGroup{db, plane, n_rows, index_base, (uint64_t)(first + k * stride) * kEvenRows};
+  }
+};
+
+// Exact check of the pairs of one 64-row group that reach the bound.
 template <int QT, bool kPlane, uint32_t kList>
-__device__ __forceinline__ void even_check(HitList<kList>& H, const Expanded (&qa)[QT], const uint4* __restrict__ src, uint64_t row0,
-                                           uint64_t n_rows, uint32_t qbase, const uint32_t* __restrict__ queries,
-                                           const uint32_t* __restrict__ db, uint32_t n_queries, uint32_t threshold,
-                                           MatchHit* __restrict__ hits, uint64_t capacity,
-                                           unsigned long long* __restrict__ counter, uint64_t index_base) {
+__device__ __forceinline__ void even_check(HitList<kList>& H, const Expanded (&qa)[QT], const RowGroup& group,
+                                           uint32_t qbase, const uint32_t* __restrict__ queries, uint32_t n_queries,
+                                           uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity,
+                                           unsigned long long* __restrict__ counter) {
   const int lane = threadIdx.x & 63;
   const int rn = lane & 15, kq = lane >> 4;
   const float bound = (float)(128 - 2 * (int)threshold);
   const int ibound = __float_as_int(bound);
-  const uint64_t r = min(row0 + (uint64_t)lane, n_rows - 1);
-  const uint4 v = src[kPlane ? r : 2 * r];
+  const uint4 v = GroupRows<kPlane>(group, 0).load(0, lane);
   uint32_t w[4] = {v.x, v.y, v.z, v.w};
   transpose_rows(w);
 #pragma unroll 1
@@ -683,8 +714,9 @@ __device__ __forceinline__ void even_check(HitList<kList>& H, const Expanded (&q
 #pragma unroll
       for (int k = 1; k < QT; k++)
         if (t == k) a = qa[k];
-      stage_candidates(mfma_prefix(a, e), t, row0 + 16 * j, qbase, rn, kq, bound, queries, db, n_queries, n_rows,
-                       threshold, H, hits, capacity, counter, index_base);
+      stage_candidates(mfma_prefix(a, e), t, group.row + 16 * j, qbase, rn, kq, bound, queries,
+                       reinterpret_cast<const uint32_t*>(group.db), n_queries, group.n_rows, threshold, H, hits,
+                       capacity, counter, group.index_base);
     }
   }
 }
@@ -692,8 +724,20 @@ __device__ __forceinline__ void even_check(HitList<kList>& H, const Expanded (&q
 // How the rows' groups are cut: the waves of one XCD, all resident at once,
 // hold as many parts as they have room for per query group; more rows take
 // several equal rounds.  Parts are whole rounds of loads.
+//
+// 40 neighbouring parts take the groups of their stretch in turn: where many
+// rows in a row match (a film's frames), their checks, some 4 us a group, spread
+// over as many waves.  With consecutive groups in each part one wave did up to
+// 64 of them after the others had ended (10^7 rows over the plane with eight
+// runs of 5000 near rows, consecutive / in turn, us: 12 queries 188 / 33, 64
+// 209 / 40, 512 384 / 182; without runs 31 / 30, 43 / 40, 184 / 180).  Turns of
+// 64 make most stretches a power of two long, and all waves then read the same
+// channels (8.4x10^6 rows x 16 queries 28 -> 39 us; 24, 40 and 56 28); turns
+// over all parts spread a wave's rows over as many pages (10^6 raw rows x 200
+// queries 14.6 -> 17.9).
+constexpr uint32_t kEvenTurn = 40;
 struct EvenParts {
-  uint32_t groups;   // row groups per part
+  uint32_t groups;   // row groups per part, at most
   uint32_t per_xcd;  // parts per XCD
 };
 __host__ __device__ inline EvenParts even_parts(uint32_t row_groups, uint32_t query_groups, uint32_t waves_per_xcd) {
@@ -706,25 +750,29 @@ __host__ __device__ inline EvenParts even_parts(uint32_t row_groups, uint32_t qu
   n = n == 0 ? kEvenRound : n > kEvenGroups ? kEvenGroups : n;
   return EvenParts{n, (uint32_t)((((uint64_t)row_groups + n - 1) / n + 7) / 8)};
 }
+// The groups of one part: count of them, first, first + stride, ...
+struct PartGroups {
+  uint32_t first, stride, count;
+};
+__device__ __forceinline__ PartGroups part_row_groups(uint32_t part, const EvenParts& parts, uint32_t row_groups) {
+  const uint32_t turn = part / kEvenTurn * kEvenTurn;  // the stretch's first part
+  const uint32_t stride = min(kEvenTurn, parts.per_xcd * 8 - turn);
+  const uint64_t begin = (uint64_t)turn * parts.groups;
+  const uint64_t first = begin + (part - turn), end = min(begin + (uint64_t)stride * parts.groups, (uint64_t)row_groups);
+  return PartGroups{(uint32_t)first, stride, first < end ? (uint32_t)((end - first + stride - 1) / stride) : 0u};
+}
 
-// Rows row0 .. row0 + left - 1 (at most kEvenGroups groups) against query
-// group qbase.
+// `ngroups` (1 .. kEvenGroups) row groups against query group qbase.
 template <int QT, bool kPlane, bool kTri, uint32_t kList>
-__device__ __forceinline__ void even_part(HitList<kList>& H, const uint4* __restrict__ db, const uint4* __restrict__ plane,
-                                          uint64_t n_rows, uint64_t row0, uint32_t left,
+__device__ __forceinline__ void even_part(HitList<kList>& H, const DbGroups& groups, uint32_t ngroups,
                                           const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t qbase,
                                           uint32_t threshold, MatchHit* __restrict__ hits, uint64_t capacity,
-                                          unsigned long long* __restrict__ counter, uint64_t index_base) {
+                                          unsigned long long* __restrict__ counter) {
   constexpr int kAhead = even_ahead(QT);
   const int lane = threadIdx.x & 63;
   const int rn = lane & 15, kq = lane >> 4;
-  const uint4* src = kPlane ? plane : db;
-  const uint4* base = src + (kPlane ? row0 : 2 * row0);  // uniform
-  // rows past the end repeat the last one; their pairs are never reported
-  auto load = [&](uint32_t g) -> uint4 {
-    const uint32_t r = min(g * kEvenRows + (uint32_t)lane, left - 1);
-    return base[kPlane ? r : 2 * r];
-  };
+  const GroupRows<kPlane> rows(groups.at(0), groups.stride);
+  auto load = [&](uint32_t k) { return rows.load(min(k, ngroups - 1), lane); };
   uint4 ring[kAhead];
 #pragma unroll
   for (int a = 0; a < kAhead; a++) ring[a] = load(a);
@@ -744,7 +792,6 @@ __device__ __forceinline__ void even_part(HitList<kList>& H, const uint4* __rest
   }
   const float bound = (float)(128 - 2 * (int)threshold);
   const v4f c0 = kTri ? flags_c0_tri(bound) : flags_c0(bound);
-  const uint32_t ngroups = (left + kEvenRows - 1) / kEvenRows;
   uint64_t pending = 0;
 #pragma unroll 1
   for (uint32_t g0 = 0; g0 < ngroups; g0 += kAhead) {
@@ -765,11 +812,9 @@ __device__ __forceinline__ void even_part(HitList<kList>& H, const uint4* __rest
   }
   if (ngroups < 64) pending &= (1ull << ngroups) - 1;  // the last round's groups past the part
   while (pending) {
-    const uint32_t g = (uint32_t)__builtin_ctzll(pending);
+    const uint32_t k = (uint32_t)__builtin_ctzll(pending);
     pending &= pending - 1;
-    even_check<QT, kPlane>(H, qa, src, row0 + (uint64_t)g * kEvenRows, n_rows, qbase, queries,
-                           reinterpret_cast<const uint32_t*>(db), n_queries, threshold, hits, capacity, counter,
-                           index_base);
+    even_check<QT, kPlane>(H, qa, groups.at(k), qbase, queries, n_queries, threshold, hits, capacity, counter);
   }
 }
 
@@ -778,21 +823,22 @@ __device__ __forceinline__ void even_part(HitList<kList>& H, const uint4* __rest
 // caches.
 template <int QT, bool kPlane, bool kTri>
 __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(4))) pdq_match_even_kernel(
-    const uint4* __restrict__ db, const uint4* __restrict__ plane, uint64_t n_rows,
+    const uint4* __restrict__ db, const uint4* __restrict__ plane, uint64_t n_rows, uint32_t row_groups,
     const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t threshold, MatchHit* __restrict__ hits,
     uint64_t capacity, unsigned long long* __restrict__ counter, uint64_t index_base, uint32_t groups,
-    uint32_t parts_per_xcd, uint32_t part_groups) {
+    EvenParts parts) {
   __shared__ HitList<kEvenStage> H;
   hits_init(H);
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t id = (blockIdx.x >> 3) * kMfmaWaves + wave;
   const uint32_t part_x = id / groups;
-  const uint64_t row0 = ((uint64_t)part_x * 8 + (blockIdx.x & 7)) * part_groups * kEvenRows;
-  if (part_x < parts_per_xcd && row0 < n_rows)
-    even_part<QT, kPlane, kTri>(H, db, plane, n_rows, row0,
-                                (uint32_t)min(n_rows - row0, (uint64_t)part_groups * kEvenRows), queries, n_queries,
-                                (id - part_x * groups) * (uint32_t)(QT * 16), threshold, hits, capacity, counter,
-                                index_base);
+  if (part_x < parts.per_xcd) {
+    const PartGroups rows = part_row_groups(part_x * 8 + (blockIdx.x & 7), parts, row_groups);
+    if (rows.count)
+      even_part<QT, kPlane, kTri>(H, DbGroups{db, plane, n_rows, index_base, rows.first, rows.stride}, rows.count,
+                                  queries, n_queries, (id - part_x * groups) * (uint32_t)(QT * 16), threshold, hits,
+                                  capacity, counter);
+  }
   hits_flush(H, hits, capacity, counter);
 }
 
@@ -1087,6 +1133,10 @@ using ResolveLds = HitList<kStageHits>;
 // groups of six query tiles, a wave each (eight leave one block per CU).
 constexpr int kRerunQt = 6;
 constexpr uint64_t kRerunRows = (uint64_t)kEvenGroups * kEvenRows;
+// Row groups of its part `part`.
+__device__ __forceinline__ uint32_t rerun_groups(uint64_t n_rows, uint64_t part) {
+  return (uint32_t)((min(n_rows - part * kRerunRows, kRerunRows) + kEvenRows - 1) / kEvenRows);
+}
 
 // The loads of one record part that do not depend on its products: the
 // query words of its tiles and the tile words of its first pending group.  A
@@ -1283,11 +1333,11 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_kernel(
     const uint64_t items = (n_rows + kRerunRows - 1) / kRerunRows * groups;
     for (uint64_t item = (uint64_t)blockIdx.x * kResolveWaves + wave; item < items;
          item += (uint64_t)gridDim.x * kResolveWaves) {
-      const uint64_t row0 = item / groups * kRerunRows;
-      even_part<kRerunQt, kPlane, false>(L, reinterpret_cast<const uint4*>(db), reinterpret_cast<const uint4*>(plane),
-                                         n_rows, row0, (uint32_t)min(n_rows - row0, kRerunRows), queries, n_queries,
-                                         (uint32_t)(item % groups) * (kRerunQt * 16), threshold, hits, capacity,
-                                         counter, index_base);
+      even_part<kRerunQt, kPlane, false>(
+          L, DbGroups{reinterpret_cast<const uint4*>(db), reinterpret_cast<const uint4*>(plane), n_rows, index_base,
+                      (uint32_t)(item / groups) * kEvenGroups, 1},
+          rerun_groups(n_rows, item / groups), queries, n_queries, (uint32_t)(item % groups) * (kRerunQt * 16),
+          threshold, hits, capacity, counter);
     }
     hits_flush(L, hits, capacity, counter);
     return;
@@ -1399,11 +1449,10 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_shards_k
       const uint64_t items = (v.n_rows + kRerunRows - 1) / kRerunRows * groups;
       for (uint64_t item = (uint64_t)blockIdx.x * kResolveWaves + wave; item < items;
            item += (uint64_t)gridDim.x * kResolveWaves) {
-        const uint64_t row0 = item / groups * kRerunRows;
-        even_part<kRerunQt, true, false>(L, v.rows, v.plane, v.n_rows, row0,
-                                           (uint32_t)min(v.n_rows - row0, kRerunRows), queries, nq,
-                                           (uint32_t)(item % groups) * (kRerunQt * 16), threshold, hits, capacity,
-                                           counter, v.index_base);
+        even_part<kRerunQt, true, false>(
+            L, DbGroups{v.rows, v.plane, v.n_rows, v.index_base, (uint32_t)(item / groups) * kEvenGroups, 1},
+            rerun_groups(v.n_rows, item / groups), queries, nq, (uint32_t)(item % groups) * (kRerunQt * 16), threshold,
+            hits, capacity, counter);
       }
     }
     hits_flush(L, hits, capacity, counter);
@@ -1436,8 +1485,8 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_shards_k
 }
 
 // The even layout over a set of shards.  The shards' row groups, one shard
-// after the other, are cut into parts as for one database; a part that crosses
-// a shard's end is matched piece by piece.  The query count is read from device
+// after the other, are cut into parts as for one database; a part that reaches
+// over a shard's end is matched piece by piece.  The query count is read from device
 // memory (`d_nq`, capped at nq_cap), so one captured launch of resident waves
 // serves batches of any size: every wave works out the parts from it.  The
 // matrix cores bound it as they do one database.  Before, a wave took 512-row
@@ -1461,20 +1510,20 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
   for (uint32_t id = (blockIdx.x >> 3) * kMfmaWaves + wave;; id += waves_per_xcd) {
     const uint32_t part_x = id / groups;
     if (part_x >= parts.per_xcd) break;
-    const uint64_t first = ((uint64_t)part_x * 8 + (blockIdx.x & 7)) * parts.groups;
-    uint32_t g = (uint32_t)min(first, (uint64_t)row_groups);
-    const uint32_t end = (uint32_t)min(first + parts.groups, (uint64_t)row_groups);
+    PartGroups rows = part_row_groups(part_x * 8 + (blockIdx.x & 7), parts, row_groups);
     uint32_t sh = 0;
-    while (g < end) {
-      while (sh + 1 < n_shards && shards[sh + 1].group_begin <= g) sh++;
+    while (rows.count) {
+      while (sh + 1 < n_shards && shards[sh + 1].group_begin <= rows.first) sh++;
       const ShardView& v = shards[sh];
-      const uint32_t stop = sh + 1 < n_shards ? min(end, (uint32_t)shards[sh + 1].group_begin) : end;
-      const uint64_t row0 = (g - v.group_begin) * kEvenRows;
-      even_part<QT, true, kTri>(H, v.rows, v.plane, v.n_rows, row0,
-                                (uint32_t)min(v.n_rows - row0, (uint64_t)(stop - g) * kEvenRows), queries, nq,
-                                (id - part_x * groups) * (uint32_t)(QT * 16), threshold, hits, capacity, counter,
-                                v.index_base);
-      g = stop;
+      uint32_t n = rows.count;  // of them in this shard
+      if (sh + 1 < n_shards)
+        n = min(n, ((uint32_t)shards[sh + 1].group_begin - rows.first - 1) / rows.stride + 1);
+      even_part<QT, true, kTri>(H, DbGroups{v.rows, v.plane, v.n_rows, v.index_base,
+                                            rows.first - (uint32_t)v.group_begin, rows.stride},
+                                n, queries, nq, (id - part_x * groups) * (uint32_t)(QT * 16), threshold, hits,
+                                capacity, counter);
+      rows.first += n * rows.stride;
+      rows.count -= n;
     }
   }
   hits_flush(H, hits, capacity, counter);
@@ -1765,8 +1814,9 @@ static hipError_t launch_even(const void* db, const void* plane, uint64_t n_rows
   auto launch = [&](auto pl, auto tr) {
     hipLaunchKernelGGL((pdq_match_even_kernel<QT, decltype(pl)::value, decltype(tr)::value>), dim3((unsigned)blocks),
                        dim3(64 * kMfmaWaves), 0, stream, static_cast<const uint4*>(db),
-                       static_cast<const uint4*>(plane), n_rows, static_cast<const uint32_t*>(queries), n_queries,
-                       threshold, hits, capacity, counter, index_base, groups, parts.per_xcd, parts.groups);
+                       static_cast<const uint4*>(plane), n_rows, (uint32_t)row_groups,
+                       static_cast<const uint32_t*>(queries), n_queries, threshold, hits, capacity, counter,
+                       index_base, groups, parts);
   };
   using T = std::integral_constant<bool, true>;
   using F = std::integral_constant<bool, false>;
