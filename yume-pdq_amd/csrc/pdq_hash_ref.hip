@@ -23,17 +23,18 @@
 // every |x| in [2^-124, 2^127] (checked exhaustively on the CPU).  Sums lie in
 // it when every input is zero or in [2^-25, 2^100]: a sum or a third of
 // multiples of 2^-k is zero or at least 2^-(k + 2) and a multiple of
-// 2^-(k + 25).  u8 planes always do; an f32 plane with another value (NaN and
-// Inf too) makes the first pass put NaN into its row, which reaches a sample,
-// and the finish block then runs the image again in the general form, with
-// divisions, one block for all four passes.
+// 2^-(k + 25).  u8 planes always do.  The first pass of an f32 plane looks for
+// another value (NaN and Inf too): its 64 rows are then walked again with
+// divisions, and the image's later passes divide as well.  Until its hash is
+// written, byte r of an image's hash tells them whether run r found one.
 // Bounds and times (us, u8 from HBM; one block per image with IEEE divisions
 // and 64-byte row accesses before): one image 223 -> 49, 100 images 283 -> 91,
-// 1024 images 2206 -> 733; f32 248 -> 65, 344 -> 130, 2469 -> 1263.  At 100
+// 1024 images 2206 -> 733; f32 248 -> 63, 344 -> 126, 2469 -> 1263.  At 100
 // images the column pass (35 us) writes 105 MB and reads 26 MB, 3.7 TB/s, the
 // sampled rows (21 us) read them back, and the finish (28 us; 20 alone) is
-// 512 dependent steps, 127 LDS steps and the median's chain.  A plane outside
-// the range pays for both forms.
+// 512 dependent steps, 127 LDS steps and the median's chain.  With divisions one
+// image takes 95, 100 images 149 (as one block per image behind the other
+// passes, which they were before, 277 and 453).
 // Every rounding happens where the reference's scalar code rounds, so the
 // results are its bits.  Only the NORMAL orientation is computed.
 #include <hip/hip_runtime.h>
@@ -49,92 +50,6 @@ namespace {
 
 constexpr int kRefThreads = 512;
 
-// Box filter of one line (src/kernel/ref.rs:49-124 with window 3: half
-// window 2, one leading accumulation, two short-window writes, full-window
-// writes, one trailing short-window write).  The line is read and written in
-// chunks of 16 (load(k, buf): inputs 16k .. 16k+15; store(m, buf): outputs
-// 16m .. 16m+15), the next chunk loading while this one is summed.
-template <typename Load, typename Store>
-__device__ __forceinline__ void box3_line(Load load, Store store) {
-  float cur[16], nxt[16], o[16];
-  load(0, cur);
-  load(1, nxt);
-  float sum = 0.0f, cws = 0.0f;
-  sum += cur[0];
-  cws += 1.0f;
-  sum += cur[1];
-  cws += 1.0f;
-  o[0] = sum / cws;
-  sum += cur[2];
-  cws += 1.0f;
-  o[1] = sum / cws;
-  float w0 = cur[0], w1 = cur[1], w2 = cur[2];  // inputs ri - 3, ri - 2, ri - 1
-  // output j = 16m + e comes from input ri = j + 1: sum += in[ri],
-  // sum -= in[ri - 3], out[j] = sum / 3
-  auto step = [&](float x, float& out) {
-    sum += x;
-    sum -= w0;
-    out = sum / cws;
-    w0 = w1;
-    w1 = w2;
-    w2 = x;
-  };
-#pragma unroll
-  for (int e = 2; e < 15; e++) step(cur[e + 1], o[e]);
-  step(nxt[0], o[15]);
-  store(0, o);
-#pragma unroll 1
-  for (int m = 1; m < 31; m++) {
-#pragma unroll
-    for (int e = 0; e < 16; e++) cur[e] = nxt[e];
-    load(m + 1, nxt);
-#pragma unroll
-    for (int e = 0; e < 15; e++) step(cur[e + 1], o[e]);
-    step(nxt[0], o[15]);
-    store(m, o);
-  }
-#pragma unroll
-  for (int e = 0; e < 16; e++) cur[e] = nxt[e];
-#pragma unroll
-  for (int e = 0; e < 15; e++) step(cur[e + 1], o[e]);
-  // the last output: one input leaves the window (w0 = input 509)
-  sum -= w0;
-  cws += -1.0f;
-  o[15] = sum / cws;
-  store(31, o);
-}
-
-// Chunk loaders and storers of the four passes.
-template <typename T>
-__device__ __forceinline__ void load_row_chunk(const T* __restrict__ plane, int r, int k, float (&b)[16]);
-template <>
-__device__ __forceinline__ void load_row_chunk<float>(const float* __restrict__ plane, int r, int k, float (&b)[16]) {
-  const f32x4* p = reinterpret_cast<const f32x4*>(plane + r * 512 + 16 * k);
-#pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const f32x4 v = p[q];
-    b[4 * q] = v.x;
-    b[4 * q + 1] = v.y;
-    b[4 * q + 2] = v.z;
-    b[4 * q + 3] = v.w;
-  }
-}
-__device__ __forceinline__ void store_row_chunk(float* __restrict__ dst, int r, int m, const float (&o)[16]) {
-  f32x4* p = reinterpret_cast<f32x4*>(dst + r * 512 + 16 * m);
-#pragma unroll
-  for (int q = 0; q < 4; q++) p[q] = f32x4{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
-}
-
-__device__ __forceinline__ void load_col_chunk(const float* __restrict__ src, int c, int k, float (&b)[16]) {
-#pragma unroll
-  for (int e = 0; e < 16; e++) b[e] = src[(16 * k + e) * 512 + c];
-}
-
-__device__ __forceinline__ void store_col_chunk(float* __restrict__ dst, int c, int m, const float (&o)[16]) {
-#pragma unroll
-  for (int e = 0; e < 16; e++) dst[(16 * m + e) * 512 + c] = o[e];
-}
-
 struct RefLds {
   union {
     float c[127 * 128];  // samples, row stride 128
@@ -146,8 +61,13 @@ struct RefLds {
   float dct_t[127 * 16];  // D transposed: dct_t[k * 16 + i] = D[i][k]
 };
 
-// x / 3, see the top of the file.
+// x / 3, by a division or as the top of the file says.  The passes are the box
+// filter of src/kernel/ref.rs:49-124 with window 3: half window 2, one leading
+// accumulation, two short-window writes, full-window writes, one trailing
+// short-window write (a short window holds two inputs, and a half is exact).
+template <bool kDivide>
 __device__ __forceinline__ float third(float x) {
+  if constexpr (kDivide) return x / 3.0f;
   constexpr float r = 1.0f / 3.0f;
   const float q = x * r;
   return __builtin_fmaf(__builtin_fmaf(-q, 3.0f, x), r, q);
@@ -210,20 +130,19 @@ struct Range {
   }
 };
 
-// First pass of f32 planes: out[j] = box of row j, all 512 columns, into A.
-// Output j of a row is complete with input j + 1, so a tile also takes the
-// first input of the next one.
-__global__ void __launch_bounds__(64) pdq_ref_rows_kernel(const float* __restrict__ planes, uint64_t plane_stride,
-                                                          uint32_t n_images, float* __restrict__ work) {
-  __shared__ RowTiles L;
-  uint32_t img;
-  int run;
-  if (!line_block(n_images, img, run)) return;
-  const int row0 = 64 * run;
-  const int lane = threadIdx.x;
-  const float* src = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(planes) +
-                                                    (size_t)img * plane_stride) + row0 * 512;
-  float* dst = work + (size_t)img * 2 * 512 * 512 + row0 * 512;
+// Whether a pass of the image divides: a byte per run, in the image's hash.
+__device__ __forceinline__ bool divides(const uint8_t* __restrict__ hashes, uint32_t img) {
+  uint64_t runs;
+  __builtin_memcpy(&runs, hashes + (size_t)img * 32, 8);
+  return runs != 0;
+}
+
+// First pass of f32 planes: out[j] = box of row j, all 512 columns, of 64 rows.
+// Output j of a row is complete with input j + 1, so a tile also takes the first
+// input of the next one.  Returns whether this lane's row keeps third() exact.
+template <bool kDivide>
+__device__ __forceinline__ bool rows_pass(const float* __restrict__ src, float* __restrict__ dst, RowTiles& L,
+                                          int lane) {
   f32x4 pf[8];
   tile_fetch(src, lane, 0, pf);
   tile_put(L.v[0], lane, pf);
@@ -257,7 +176,7 @@ __global__ void __launch_bounds__(64) pdq_ref_rows_kernel(const float* __restric
       const float old = e < 3 ? h[e] : x[e - 3];
       if (e < kTileCols || tile + 1 < kTiles) {
         step(x[e], old);
-        o[e - 1] = third(sum);
+        o[e - 1] = third<kDivide>(sum);
       } else {
         sum -= old;  // the last output: the oldest input leaves the window
         o[e - 1] = sum * 0.5f;
@@ -267,10 +186,6 @@ __global__ void __launch_bounds__(64) pdq_ref_rows_kernel(const float* __restric
     h[0] = 0.0f;  // (unused: input 0 of a tile was taken by the one before)
     h[1] = x[kTileCols - 2];
     h[2] = x[kTileCols - 1];
-    if (tile + 1 == kTiles && !range.plain(sum)) {
-#pragma unroll
-      for (int e = 0; e < kTileCols; e++) o[e] = __builtin_nanf("");
-    }
     wave_lds_sync();
 #pragma unroll
     for (int q = 0; q < kTileCols / 4; q++)
@@ -283,6 +198,24 @@ __global__ void __launch_bounds__(64) pdq_ref_rows_kernel(const float* __restric
           *reinterpret_cast<const f32x4*>(buf + (8 * i + (lane >> 3)) * kTileStride + 4 * (lane & 7));
     wave_lds_sync();
   }
+  return range.plain(sum);
+}
+
+__global__ void __launch_bounds__(64) pdq_ref_rows_kernel(const float* __restrict__ planes, uint64_t plane_stride,
+                                                          uint32_t n_images, float* __restrict__ work,
+                                                          uint8_t* __restrict__ hashes) {
+  __shared__ RowTiles L;
+  uint32_t img;
+  int run;
+  if (!line_block(n_images, img, run)) return;
+  const int row0 = 64 * run;
+  const int lane = threadIdx.x;
+  const float* src = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(planes) +
+                                                    (size_t)img * plane_stride) + row0 * 512;
+  float* dst = work + (size_t)img * 2 * 512 * 512 + row0 * 512;
+  const bool divide = wave_any(!rows_pass<false>(src, dst, L, lane));
+  if (divide) (void)rows_pass<true>(src, dst, L, lane);
+  if (lane == 0) hashes[(size_t)img * 32 + run] = divide ? 1 : 0;
 }
 
 // One input row of the second pass at this lane's column: an f32 value of A,
@@ -331,13 +264,10 @@ struct ColumnSource<uint8_t> {
 // while these are summed.  A u8 wave reads 64 bytes of a row, too little in
 // flight for HBM: one load of 64 rows (a row per lane) brings their lines into
 // the cache two iterations ahead of the loads that use them.
-template <typename T>
-__global__ void __launch_bounds__(64) pdq_ref_cols_kernel(const T* __restrict__ planes, uint64_t plane_stride,
-                                                          uint32_t n_images, float* __restrict__ work) {
+template <typename T, bool kDivide>
+__device__ __forceinline__ void cols_pass(const T* __restrict__ planes, uint64_t plane_stride, uint32_t img, int run,
+                                          float* __restrict__ work) {
   constexpr int R = 32;
-  uint32_t img;
-  int run;
-  if (!line_block(n_images, img, run)) return;
   const uint32_t c = 64 * run + threadIdx.x;
   const float* A = work + (size_t)img * 2 * 512 * 512;
   float* out = work + (size_t)img * 2 * 512 * 512 + 512 * 512;
@@ -365,11 +295,11 @@ __global__ void __launch_bounds__(64) pdq_ref_cols_kernel(const T* __restrict__ 
       h1 = h2;
       h2 = x;
       if (e == 0) {
-        if (r0 > 0) (out + (r0 - 1) * 512)[c] = third(sum);
+        if (r0 > 0) (out + (r0 - 1) * 512)[c] = third<kDivide>(sum);
       } else if (e == 1) {
-        (out + r0 * 512)[c] = r0 == 0 ? sum * 0.5f : third(sum);
+        (out + r0 * 512)[c] = r0 == 0 ? sum * 0.5f : third<kDivide>(sum);
       } else {
-        (out + (r0 + e - 1) * 512)[c] = third(sum);
+        (out + (r0 + e - 1) * 512)[c] = third<kDivide>(sum);
       }
     }
   };
@@ -391,6 +321,18 @@ __global__ void __launch_bounds__(64) pdq_ref_cols_kernel(const T* __restrict__ 
   (out + 511 * 512)[c] = sum * 0.5f;
 }
 
+template <typename T>
+__global__ void __launch_bounds__(64) pdq_ref_cols_kernel(const T* __restrict__ planes, uint64_t plane_stride,
+                                                          uint32_t n_images, float* __restrict__ work,
+                                                          const uint8_t* __restrict__ hashes) {
+  uint32_t img;
+  int run;
+  if (!line_block(n_images, img, run)) return;
+  if constexpr (std::is_same<T, float>::value)
+    if (divides(hashes, img)) return cols_pass<T, true>(planes, plane_stride, img, run, work);
+  cols_pass<T, false>(planes, plane_stride, img, run, work);
+}
+
 // Sample k of a line is output floor((2k + 1) 512 / 254), complete with input
 //   k <= 31: 4k + 3    k = 32 .. 62: 4k + 4    k = 63 .. 94: 4k + 5
 //   k >= 95: 4k + 6
@@ -403,7 +345,7 @@ __device__ __forceinline__ constexpr int sample_input(int g) { return g < 32 ? 3
 // group that completes them (place 32 holds no sample).  A lane's samples
 // gather in LDS and are stored a quarter of a row at a time, whole 128-byte
 // lines.
-template <int kQuarter>
+template <int kQuarter, bool kDivide>
 __device__ __forceinline__ void sampled_tile(const float (&x)[kTileCols], int first_group, float& sum, float (&h)[3],
                                              float* __restrict__ out) {
 #pragma unroll
@@ -413,7 +355,7 @@ __device__ __forceinline__ void sampled_tile(const float (&x)[kTileCols], int fi
       const int i = 4 * u + e;
       sum += x[i];
       sum -= i < 3 ? h[i] : x[i - 3];
-      if (e == sample_input(32 * kQuarter)) out[(first_group + u) & 31] = third(sum);
+      if (e == sample_input(32 * kQuarter)) out[(first_group + u) & 31] = third<kDivide>(sum);
     }
   }
   h[0] = x[kTileCols - 3];
@@ -421,11 +363,8 @@ __device__ __forceinline__ void sampled_tile(const float (&x)[kTileCols], int fi
   h[2] = x[kTileCols - 1];
 }
 
-__global__ void __launch_bounds__(64) pdq_ref_sampled_kernel(uint32_t n_images, float* __restrict__ work) {
-  __shared__ RowTiles L;  // the tile, the samples
-  uint32_t img;
-  int run;
-  if (!line_block(n_images, img, run)) return;
+template <bool kDivide>
+__device__ __forceinline__ void sampled_pass(RowTiles& L, uint32_t img, int run, float* __restrict__ work) {
   const int row0 = 64 * run;
   const int lane = threadIdx.x;
   float* A = work + (size_t)img * 2 * 512 * 512;
@@ -453,7 +392,7 @@ __global__ void __launch_bounds__(64) pdq_ref_sampled_kernel(uint32_t n_images, 
     wave_lds_sync();
     float x[kTileCols];
     tile_row(L.v[0], lane, x);
-    sampled_tile<kQuarter>(x, 8 * tile, sum, h, out);
+    sampled_tile<kQuarter, kDivide>(x, 8 * tile, sum, h, out);
   };
   auto quarter = [&](auto q) {
     constexpr int t0 = kTiles / 4 * decltype(q)::value;
@@ -470,10 +409,23 @@ __global__ void __launch_bounds__(64) pdq_ref_sampled_kernel(uint32_t n_images, 
   quarter(std::integral_constant<int, 3>());
 }
 
+// kMayDivide: f32 planes.
+template <bool kMayDivide>
+__global__ void __launch_bounds__(64) pdq_ref_sampled_kernel(uint32_t n_images, float* __restrict__ work,
+                                                             const uint8_t* __restrict__ hashes) {
+  __shared__ RowTiles L;  // the tile, the samples
+  uint32_t img;
+  int run;
+  if (!line_block(n_images, img, run)) return;
+  if constexpr (kMayDivide)
+    if (divides(hashes, img)) return sampled_pass<true>(L, img, run, work);
+  sampled_pass<false>(L, img, run, work);
+}
+
 // Fourth pass (columns of the samples): lane k walks column k of the 512 x 128
 // samples in A and keeps every sampled row's value in c.  Sixteen rows at a
 // time, from LDS.
-template <int kQuarter>
+template <int kQuarter, bool kDivide>
 __device__ __forceinline__ void finish_rows(const float* __restrict__ x0, int first_group, float& sum, float (&h)[3],
                                             float* __restrict__ c) {
   float x[16];
@@ -488,7 +440,7 @@ __device__ __forceinline__ void finish_rows(const float* __restrict__ x0, int fi
       sum -= i < 3 ? h[i] : x[i - 3];
       if (e == sample_input(32 * kQuarter)) {
         const int k = first_group + u - (kQuarter == 0 ? 0 : 1);
-        if (kQuarter != 1 || k > 31) c[k * 128] = third(sum);
+        if (kQuarter != 1 || k > 31) c[k * 128] = third<kDivide>(sum);
       }
     }
   }
@@ -503,6 +455,7 @@ struct ColumnChunks {
   float v[2][64 * 128];
 };
 
+template <bool kDivide>
 __device__ __forceinline__ void finish_columns(const float* __restrict__ src, ColumnChunks& S, float* __restrict__ c) {
   const int t = threadIdx.x;
   // the sample of place t; place 32's walk goes to the unused column 127
@@ -523,7 +476,7 @@ __device__ __forceinline__ void finish_columns(const float* __restrict__ src, Co
     __syncthreads();
     if (t < 128) {
 #pragma unroll
-      for (int k = 0; k < 4; k++) finish_rows<kQuarter>(buf + k * 16 * 128 + t, 16 * m + 4 * k, sum, h, c + column);
+      for (int k = 0; k < 4; k++) finish_rows<kQuarter, kDivide>(buf + k * 16 * 128 + t, 16 * m + 4 * k, sum, h, c + column);
     }
   };
   auto quarter = [&](auto q) {
@@ -621,38 +574,9 @@ __device__ __forceinline__ float torben_median_wave(const float* __restrict__ P,
   return result;
 }
 
-// The four passes in the general form, by one block, and its samples: f32
-// planes that hold a value outside third()'s range.
-__device__ __noinline__ void general_samples(const float* __restrict__ plane, float* __restrict__ A, float* __restrict__ c) {
-  const int t = threadIdx.x;
-  float* B = A + 512 * 512;
-  // jarosz_filter_float(.., 512, 512, 3, 3, 2): rows then columns, twice
-  // (ref.rs:7-47); the input plane is not modified
-  box3_line([&](int k, float(&b)[16]) { load_row_chunk<float>(plane, t, k, b); },
-            [&](int m, const float(&o)[16]) { store_row_chunk(A, t, m, o); });
-  __syncthreads();
-  box3_line([&](int k, float(&b)[16]) { load_col_chunk(A, t, k, b); },
-            [&](int m, const float(&o)[16]) { store_col_chunk(B, t, m, o); });
-  __syncthreads();
-  box3_line([&](int k, float(&b)[16]) { load_row_chunk<float>(B, t, k, b); },
-            [&](int m, const float(&o)[16]) { store_row_chunk(A, t, m, o); });
-  __syncthreads();
-  box3_line([&](int k, float(&b)[16]) { load_col_chunk(A, t, k, b); },
-            [&](int m, const float(&o)[16]) { store_col_chunk(B, t, m, o); });
-  __syncthreads();
-  // samples at ((2o + 1) 512) / 254 (mod.rs:808-818)
-  for (int e = t; e < 127 * 127; e += kRefThreads) {
-    const int oi = e / 127, oj = e - oi * 127;
-    const int ii = ((oi * 2 + 1) * 512) / 254, jj = ((oj * 2 + 1) * 512) / 254;
-    c[oi * 128 + oj] = B[ii * 512 + jj];
-  }
-  __syncthreads();
-}
-
 // One block per image: the fourth pass, dct2d, quality, median and bits.
 template <typename T>
-__global__ void __launch_bounds__(kRefThreads) pdq_ref_finish_kernel(const T* __restrict__ planes, uint64_t plane_stride,
-                                                                     float* __restrict__ work,
+__global__ void __launch_bounds__(kRefThreads) pdq_ref_finish_kernel(float* __restrict__ work,
                                                                      uint8_t* __restrict__ hashes,
                                                                      float* __restrict__ quality,
                                                                      float* __restrict__ threshold,
@@ -664,17 +588,11 @@ __global__ void __launch_bounds__(kRefThreads) pdq_ref_finish_kernel(const T* __
   float* c = L.u.c;
   __shared__ ColumnChunks S;
   for (int e = t; e < 127 * 16; e += kRefThreads) L.dct_t[e] = kDctT.v[e];
-  finish_columns(A, S, c);
+  if (std::is_same<T, float>::value && divides(hashes, img))  // the same for the whole block
+    finish_columns<true>(A, S, c);
+  else
+    finish_columns<false>(A, S, c);
   __syncthreads();
-  if constexpr (std::is_same<T, float>::value) {
-    float z = 0.0f;
-    for (int e = t; e < 127 * 128; e += kRefThreads) z = __builtin_fmaf(c[e], 0.0f, z);
-    if (__syncthreads_or(nonfinite(z) ? 1 : 0)) {
-      general_samples(reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(planes) +
-                                                     (size_t)img * plane_stride),
-                      A, c);
-    }
-  }
 
   // dct2d (mod.rs:711-735): tmp[i][j] = sum_k D[i][k] * c[k][j], then
   // out[i][j] = sum_k tmp[i][k] * D[j][k]; each sum from 0.0, k ascending, a
@@ -725,12 +643,13 @@ void launch_ref_kind(const void* planes, uint64_t plane_stride, uint32_t n_image
                      float* quality, float* threshold, float* pdqf, hipStream_t stream) {
   const T* p = static_cast<const T*>(planes);
   const dim3 lines(64 * ((n_images + 7) / 8)), wave(64);
-  if constexpr (std::is_same<T, float>::value)
-    hipLaunchKernelGGL(pdq_ref_rows_kernel, lines, wave, 0, stream, p, plane_stride, n_images, work);
-  hipLaunchKernelGGL(pdq_ref_cols_kernel<T>, lines, wave, 0, stream, p, plane_stride, n_images, work);
-  hipLaunchKernelGGL(pdq_ref_sampled_kernel, lines, wave, 0, stream, n_images, work);
-  hipLaunchKernelGGL(pdq_ref_finish_kernel<T>, dim3(n_images), dim3(kRefThreads), 0, stream, p, plane_stride, work,
-                     hashes, quality, threshold, pdqf);
+  constexpr bool kF32 = std::is_same<T, float>::value;
+  if constexpr (kF32)
+    hipLaunchKernelGGL(pdq_ref_rows_kernel, lines, wave, 0, stream, p, plane_stride, n_images, work, hashes);
+  hipLaunchKernelGGL(pdq_ref_cols_kernel<T>, lines, wave, 0, stream, p, plane_stride, n_images, work, hashes);
+  hipLaunchKernelGGL(pdq_ref_sampled_kernel<kF32>, lines, wave, 0, stream, n_images, work, hashes);
+  hipLaunchKernelGGL(pdq_ref_finish_kernel<T>, dim3(n_images), dim3(kRefThreads), 0, stream, work, hashes, quality,
+                     threshold, pdqf);
 }
 
 }  // namespace
