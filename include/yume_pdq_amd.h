@@ -429,6 +429,8 @@ int yume_pdq_amd_tune_load(const char *path);
 int yume_pdq_amd_tune_clear(void);
 int yume_pdq_amd_batcher_tune_records(const YumePdqAmdBatcher *b, YumePdqAmdTuneRecord *out,
                                       uint32_t cap, uint32_t *n);
+/* The matcher for n_queries and, on the matrix cores, its tuned query tiles per
+ * wave; a batch's own groups may be of another width (as even as they can be). */
 int yume_pdq_amd_batcher_choice(const YumePdqAmdBatcher *b, uint32_t n_queries, uint32_t *path,
                                 uint32_t *query_tiles);
 

@@ -17,9 +17,9 @@
 namespace ypdq {
 
 // Which matcher a batch uses: the vector-ALU scan, or the matrix-core filter
-// with at most qt 16-query tiles per wave: in the even layout, whose waves hold
-// `width` tiles each (the batch spread over as many query groups as qt makes),
-// or (shared, with a record area) with a block's waves sharing their rows.
+// (qt: the 16-query tiles per wave that the choice was tuned to or reports): in
+// the even layout, whose waves hold `width` tiles each, or (shared, with a record
+// area) with a block's waves sharing their rows.
 struct MatcherChoice {
   bool mfma = false;
   int qt = 8;

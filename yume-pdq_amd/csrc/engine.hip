@@ -414,16 +414,14 @@ uint64_t BatchContext::device_bytes() const {
   return plane_stride_ * max_images_ + out_bytes(hit_capacity_) + 16 + match_record_area_bytes();
 }
 
-// What a choice of at most c.qt query tiles per wave launches for nq queries:
-// the tiles spread evenly over the query groups that qt makes, or the
-// shared-rows layout where that is the better one for these rows.
-static void set_layout(MatcherChoice* c, uint64_t rows, uint32_t nq) {
+// What a choice of at most `limit` query tiles per wave launches for nq queries:
+// the single-database matcher's plan within that limit.
+static void set_layout(MatcherChoice* c, uint64_t rows, uint32_t nq, int limit) {
   c->shared = false;
   if (!c->mfma) return;
-  const int tiles = (int)std::max<uint32_t>(1, (nq + 15) / 16);
-  const int groups = (tiles + c->qt - 1) / c->qt;
-  c->width = std::max(2, (tiles + groups - 1) / groups);
-  c->shared = c->qt == 16 && match_plan(rows, nq).shared;
+  const MatchPlan plan = match_plan(rows, nq, limit);
+  c->width = plan.qt;
+  c->shared = limit == 16 && plan.shared;
 }
 
 void BatchContext::refresh_choices() const {
@@ -441,9 +439,8 @@ bool BatchContext::tuned() const {
   return !choices_.empty();
 }
 
-// Relative cost per query of the matrix-core matcher at qt query tiles per
-// wave (a wave's row loads and expansions are shared by its 16 qt queries):
-// 10^8 rows at 512 queries take 3.75 / 2.52 / 2.04 / 2.05 ms at 2 / 4 / 8 / 16.
+// Relative cost per query at qt query tiles per wave in whole groups, for the
+// tile count that a choice reports.
 static double mfma_query_cost(int qt) { return qt >= 8 ? 1.0 : qt == 4 ? 1.25 : 1.8; }
 
 // Queries in whole groups of 16 qt for nq.
@@ -456,14 +453,22 @@ MatcherChoice BatchContext::choice_for(uint32_t nq) const {
   refresh_choices();
   auto it = choices_.upper_bound(nq);
   MatcherChoice c;
+  int limit = 16;
   if (it != choices_.begin()) {
     --it;
     c = it->second;
     if (c.mfma) {
-      // a bucket is tuned at its first query count, where every candidate's
-      // groups are full; above it, the last group of a wide tile can be mostly
-      // empty (nq = 320 at 16 tiles makes groups for 512 queries).  Take the
-      // narrower tile when its whole groups cost less.
+      // A bucket is tuned at its first query count.  A choice that held all of
+      // those queries in one group says nothing against wider groups for the
+      // rest of the bucket; one of several groups is the limit for them.  Which
+      // width is launched within it, the plan says: its groups are as even as
+      // they can be, so no count of queries needs a narrower limit (five shards,
+      // 7.5M rows: 20 images' 160 queries as three groups of 4 tiles and as one
+      // of 10, 158 / 135 us a batch; 100 images' 800 as seven of 8 and as four of
+      // 13, 349 / 317).
+      limit = (uint64_t)c.qt * 16 >= it->first ? 16 : c.qt;
+      // The reported tile count: the narrower one where whole groups of it cost
+      // less (nq = 320 at 16 tiles would be groups for 512 queries).
       int best = c.qt;
       double best_cost = (double)padded_queries(nq, c.qt) * mfma_query_cost(c.qt);
       for (int qt = c.qt / 2; qt >= 2; qt /= 2) {
@@ -481,7 +486,7 @@ MatcherChoice BatchContext::choice_for(uint32_t nq) const {
     c.mfma = match_mfma_applicable(nq, threshold_);
     c.qt = plan.shared ? 16 : plan.qt;
   }
-  set_layout(&c, shards_->total_rows(), nq);
+  set_layout(&c, shards_->total_rows(), nq, limit);
   return c;
 }
 
@@ -603,7 +608,7 @@ hipError_t BatchContext::autotune(int iterations, std::vector<TuneRecord>* recor
         MatcherChoice m;
         m.mfma = true;
         m.qt = qt;
-        set_layout(&m, shards_->total_rows(), nq);
+        set_layout(&m, shards_->total_rows(), nq, qt);
         cands.push_back(m);
       }
     float best = 1e30f;

@@ -117,12 +117,12 @@ struct ShardView {
 uint64_t mfma_chunks(uint64_t n_rows);       // shared-rows chunks of one shard (multiple of 8)
 uint64_t match_row_groups(uint64_t n_rows);  // the even layout's row groups of one shard
 // The matrix-core matcher for n_queries over n_rows rows: the shared-rows
-// layout, or the even layout with qt (2 .. 16) query tiles per wave.
+// layout, or the even layout with qt (2 .. most_qt) query tiles per wave.
 struct MatchPlan {
   bool shared;
   int qt;
 };
-MatchPlan match_plan(uint64_t n_rows, uint32_t n_queries);
+MatchPlan match_plan(uint64_t n_rows, uint32_t n_queries, int most_qt = 16);
 // The even layout over a set of shards (their prefix planes), on a GPU of
 // `cus` compute units.
 hipError_t launch_match_even_shards(int qt, const ShardView* shards, uint32_t n_shards, uint64_t row_groups,

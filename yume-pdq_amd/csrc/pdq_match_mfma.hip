@@ -1937,11 +1937,11 @@ constexpr int kEvenCost = 27;
 constexpr int kSharedCost = 733;
 constexpr uint64_t kSharedGain = 30000000;  // rows x cost units that pay for the recheck
 
-MatchPlan match_plan(uint64_t n_rows, uint32_t n_queries) {
+MatchPlan match_plan(uint64_t n_rows, uint32_t n_queries, int most_qt) {
   const uint64_t tiles = ((uint64_t)n_queries + 15) / 16;
   MatchPlan plan{false, 2};
   uint64_t best = ~0ull;
-  for (int qt = 2; qt <= 16; qt++) {
+  for (int qt = 2; qt <= most_qt; qt++) {
     const uint64_t cost = (tiles + qt - 1) / qt * (uint64_t)(kEvenCost + 10 * qt);
     if (cost < best) {
       best = cost;
