@@ -75,8 +75,8 @@ hipError_t launch_hash_wave(const void* planes, int input_kind, uint64_t plane_s
 hipError_t launch_hash_block(const void* planes, int input_kind, uint64_t plane_stride, uint32_t n_max,
                              const uint32_t* d_n, uint32_t mode, int dct, int waves, const HashOutputs& out,
                              const float* luma, hipStream_t stream);
-// Layout the automatic choice uses for n images: 1 = wave per image,
-// 8 = block of eight waves per image.
+// Layout the automatic choice uses for n images: 1 = wave per image, 8 or 16 =
+// block of as many waves per image.
 int hash_layout_for(uint32_t n_images, int input_kind, int dct);
 // The precise ReferenceKernel<f32> (f32 or u8 planes): hash, quality,
 // threshold (the median) and PDQF of the NORMAL orientation per image;

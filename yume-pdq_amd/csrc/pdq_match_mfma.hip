@@ -193,62 +193,46 @@ __device__ __forceinline__ void fold_flags(const v4f& v, uint32_t& m) {
   asm volatile("" : "+v"(m));
 }
 
-// The query pair of pair P of a row tile (of QT / 2 pairs).  Pair P's
-// products go to result register P % 4 and are folded into flag chain P % 4;
-// at QT = 16 the pairs are ordered so that chains 0 and 1 hold query tiles
-// 0-7 and chains 2 and 3 tiles 8-15, so one vote per half tells which half
-// of the query tiles has candidates.
-template <int kHalf>
+// Query tiles per wave of the shared-rows layout.
+constexpr int kSharedQt = 16;
+constexpr int kSharedPairs = kSharedQt / 2;  // per row tile
+
+// The query pair of pair P of a row tile.  Pair P's products go to result
+// register P % 4 and are folded into flag chain P % 4; the pairs are ordered so
+// that chains 0 and 1 hold query tiles 0-7 and chains 2 and 3 tiles 8-15, so one
+// vote per half tells which half of the query tiles has candidates.
 __device__ constexpr int query_pair(int p) {
-  if constexpr (kHalf == 8) {
-    constexpr int order[8] = {0, 1, 4, 5, 2, 3, 6, 7};
-    return order[p % 8];
-  }
-  return p % kHalf;
+  constexpr int order[kSharedPairs] = {0, 1, 4, 5, 2, 3, 6, 7};
+  return order[p % kSharedPairs];
 }
 
-// Pair P (row tile P / (QT/2), query tiles 2 query_pair(P) and +1): its first
+// Pair P (row tile P / 8, query tiles 2 query_pair(P) and +1): its first
 // product issues at step P into result register P % 4, its second at step
 // P + 1 (one product after, so the accumulation does not wait), and its bits
 // are folded at step P + 4, before the register takes pair P + 4.  The four
 // result registers are named, not an array, so the compiler keeps each in
 // place.
-template <int QT, int kTiles, int S>
-__device__ __forceinline__ void group_flags_step(const Expanded (&qa)[QT], const Expanded (&rb)[kTiles],
+template <int kTiles, int S>
+__device__ __forceinline__ void group_flags_step(const Expanded (&qa)[kSharedQt], const Expanded (&rb)[kTiles],
                                                  const v4f& c0, uint32_t (&acc)[kFlagChains], v4f& r0, v4f& r1,
                                                  v4f& r2, v4f& r3) {
-  constexpr int kHalf = QT / 2;
-  constexpr int kN = kHalf * kTiles;  // pairs
+  constexpr int kN = kSharedPairs * kTiles;  // pairs
   v4f& cur = (S % 4 == 0) ? r0 : (S % 4 == 1) ? r1 : (S % 4 == 2) ? r2 : r3;
   v4f& prev = (S % 4 == 1) ? r0 : (S % 4 == 2) ? r1 : (S % 4 == 3) ? r2 : r3;
   if constexpr (S >= 4) fold_flags(cur, acc[(S - 4) % kFlagChains]);
-  if constexpr (S < kN) cur = mfma_acc<kScale1>(qa[2 * query_pair<kHalf>(S)], rb[S / kHalf], c0);
+  if constexpr (S < kN) cur = mfma_acc<kScale1>(qa[2 * query_pair(S)], rb[S / kSharedPairs], c0);
   if constexpr (S >= 1 && S - 1 < kN)
-    prev = mfma_acc<kScale512>(qa[2 * query_pair<kHalf>(S - 1) + 1], rb[(S - 1) / kHalf], prev);
+    prev = mfma_acc<kScale512>(qa[2 * query_pair(S - 1) + 1], rb[(S - 1) / kSharedPairs], prev);
   // keep this order: hoisting the products runs out of registers
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (S + 1 < kN + 4) group_flags_step<QT, kTiles, S + 1>(qa, rb, c0, acc, r0, r1, r2, r3);
+  if constexpr (S + 1 < kN + 4) group_flags_step<kTiles, S + 1>(qa, rb, c0, acc, r0, r1, r2, r3);
 }
 
-template <int QT, int kTiles>
-__device__ __forceinline__ void group_flags(const Expanded (&qa)[QT], const Expanded (&rb)[kTiles], const v4f& c0,
-                                            uint32_t (&acc)[kFlagChains]) {
-  static_assert(QT % 2 == 0 && (QT / 2) * kTiles >= 4, "pairs of query tiles, four pairs in flight");
+template <int kTiles>
+__device__ __forceinline__ void group_flags(const Expanded (&qa)[kSharedQt], const Expanded (&rb)[kTiles],
+                                            const v4f& c0, uint32_t (&acc)[kFlagChains]) {
   v4f r0, r1, r2, r3;
-  group_flags_step<QT, kTiles, 0>(qa, rb, c0, acc, r0, r1, r2, r3);
-}
-
-__device__ __forceinline__ bool flags_set(const uint32_t (&acc)[kFlagChains]) {
-  return ((acc[0] | acc[1] | acc[2] | acc[3]) & kFlagMask) != 0;
-}
-
-// Flags of query tiles 0-7 (chains 0 and 1) and 8-15 (chains 2 and 3) at
-// QT = 16.
-__device__ __forceinline__ bool flags_set_low(const uint32_t (&acc)[kFlagChains]) {
-  return ((acc[0] | acc[1]) & kFlagMask) != 0;
-}
-__device__ __forceinline__ bool flags_set_high(const uint32_t (&acc)[kFlagChains]) {
-  return ((acc[2] | acc[3]) & kFlagMask) != 0;
+  group_flags_step<kTiles, 0>(qa, rb, c0, acc, r0, r1, r2, r3);
 }
 
 // Three products per accumulator (sixteen query tiles, thresholds 28..63).
@@ -296,7 +280,7 @@ __device__ constexpr int tri_chain(int p) { return 2 * ((p % 6) >= 3 ? 1 : 0) + 
 // third at step P + 2, and its bits are folded at step P + 4, before the
 // register takes accumulator P + 4.
 template <int kTiles, int S>
-__device__ __forceinline__ void group_flags_tri_step(const Expanded (&qa)[16], const Expanded (&rb)[kTiles],
+__device__ __forceinline__ void group_flags_tri_step(const Expanded (&qa)[kSharedQt], const Expanded (&rb)[kTiles],
                                                      const v4f& c0, uint32_t (&acc)[kFlagChains], v4f& r0, v4f& r1,
                                                      v4f& r2, v4f& r3) {
   constexpr int kN = 6 * kTiles;  // accumulators
@@ -316,7 +300,7 @@ __device__ __forceinline__ void group_flags_tri_step(const Expanded (&qa)[16], c
 }
 
 template <int kTiles>
-__device__ __forceinline__ void group_flags_tri(const Expanded (&qa)[16], const Expanded (&rb)[kTiles], const v4f& c0,
+__device__ __forceinline__ void group_flags_tri(const Expanded (&qa)[kSharedQt], const Expanded (&rb)[kTiles], const v4f& c0,
                                                 uint32_t (&acc)[kFlagChains]) {
   v4f r0, r1, r2, r3;
   group_flags_tri_step<kTiles, 0>(qa, rb, c0, acc, r0, r1, r2, r3);
@@ -345,18 +329,18 @@ struct RowSource {
 // (double-buffered, one barrier per group), and every wave reads the group's
 // expanded tiles with one 16-byte LDS read each.  Each wave would otherwise
 // load and expand every tile itself; shared, a product costs a quarter of the
-// loads and LUT reads, which is what more query tiles per wave would buy
+// loads and expansions, which is what more query tiles per wave would buy
 // without their registers.  A wave whose group lies past the last query still
-// loads and expands its tiles for the others.  The rare path is per wave, as
-// in mfma_item, reading its tiles' rows directly.
+// loads and expands its tiles for the others.  Candidates become records, one
+// per wave and item, for the recheck kernel.
 constexpr int kSharedTiles = 64;
 constexpr uint64_t kSharedRows = (uint64_t)kSharedTiles * 16;
 constexpr int kStagePerWave = 1;                          // tiles a wave stages per group
 constexpr int kGroupTiles = kMfmaWaves * kStagePerWave;  // tiles per barrier and per vote
 static_assert(kSharedTiles % kGroupTiles == 0 && kSharedTiles / kGroupTiles <= 32,
               "one bit of a 32-bit record mask per group of tiles");
-// At QT = 16 a record's mask holds query tiles 0-7's groups in its low bits
-// and tiles 8-15's from bit kHalfShift.
+// A record's mask holds query tiles 0-7's groups in its low bits and tiles
+// 8-15's from bit kHalfShift.
 constexpr int kHalfShift = 16;
 static_assert(kSharedTiles / kGroupTiles <= kHalfShift, "two halves in a record mask");
 static_assert((uint64_t)kMfmaWaves * kMfmaTilesPerWave * 16 % kSharedRows == 0, "sub-chunks of a chunk");
@@ -370,9 +354,8 @@ struct SharedRowsLds {
 // exist, every sub-chunk but a database's last) has a loop with fixed bounds
 // and no branch: a branch in the loop makes the compiler wait for every load
 // in flight at each group.
-template <int QT, bool kFull, bool kPlane, bool kTri>
-__device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT], 
-                                              SharedRowsLds& S, const RowSource<kPlane>& src,
+template <bool kFull, bool kPlane, bool kTri>
+__device__ __forceinline__ void stream_shared(const Expanded (&qa)[kSharedQt], SharedRowsLds& S, const RowSource<kPlane>& src,
                                               const uint32_t* __restrict__ db, uint64_t row0, uint64_t n_rows,
                                               uint32_t qbase, int wave, int lane, float bound,
                                               uint4* __restrict__ recs, uint32_t* __restrict__ rec_count,
@@ -392,11 +375,11 @@ __device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT],
     const uint64_t r = min((uint64_t)tt * 16 + rn, left - 1);
     return db[(row0 + r) * 8 + kq];
   };
-  // staging in two halves: the table reads (expand_word), then the store,
-  // with the group's products between them
+  // staging in two halves: the expansion, then the store, with the group's
+  // products between them
   auto store = [&](uint32_t g, int s, const Expanded& e, int buf) {
     const uint32_t tt = kGroupTiles * g + kMfmaWaves * s + (uint32_t)wave;
-    // zero operands (not the expansion of a zero word, which is all -1),
+    // zero operands (not the expansion of a zero word, whose every code is +1),
     // selected without a branch
     const bool have = kFull ? tt < tiles : (tt < tiles && (uint64_t)tt * 16 + rn < left);
     const uint32_t keep = have ? 0xffffffffu : 0u;
@@ -427,7 +410,6 @@ __device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT],
   uint32_t acc[kFlagChains];
 #pragma unroll
   for (int m = 0; m < kFlagChains; m++) acc[m] = 0u;
-  static_assert(!kTri || QT == 16, "three products per accumulator at sixteen query tiles");
   const v4f c0 = kTri ? flags_c0_tri(bound) : flags_c0(bound);
   uint64_t pending = 0;  // groups of tiles whose products reached the bound
 #pragma unroll 1
@@ -439,13 +421,13 @@ __device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT],
       // The group's expanded tiles, read together so their latencies
       // overlap, and before the staging below: LDS operations complete in
       // order, so the products then wait for these reads only, not for the
-      // table reads and the write of the next group.
+      // write of the next group.
       u32x4 vt[kGroupTiles];
 #pragma unroll
       for (int j = 0; j < kGroupTiles; j++) vt[j] = S.ex[g & 1][j][lane];
       __builtin_amdgcn_sched_barrier(0);
-      // The next group's table reads are issued now and its store follows
-      // the products, so neither waits for the other.  The buffer written
+      // The next group is expanded now and its store follows the products, so
+      // neither waits for the other.  The buffer written
       // here was last read before the previous barrier; after the last group
       // this stages rows nobody reads.
       Expanded next[kStagePerWave];
@@ -463,7 +445,7 @@ __device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT],
       if constexpr (kTri)
         group_flags_tri<kGroupTiles>(qa, rb, c0, acc);
       else
-        group_flags<QT, kGroupTiles>(qa, rb, c0, acc);
+        group_flags<kGroupTiles>(qa, rb, c0, acc);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int st = 0; st < kStagePerWave; st++) {
@@ -471,19 +453,12 @@ __device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT],
         ring[a][st] = word(g + 1 + kRing < ngroups ? g + 1 + kRing : ngroups - 1, st);
       }
       // the vote is a wave-uniform mask, so the pending bits stay in scalar
-      // registers; at QT = 16 one vote per half of the query tiles, the
-      // second half's bits kHalfShift above the first's
-      if constexpr (kTri) {
-        const uint64_t lo = __ballot(((acc[0] | acc[1]) & kFlagMaskTri) != 0);
-        const uint64_t hi = __ballot(((acc[2] | acc[3]) & kFlagMaskTri) != 0);
-        pending |= (uint64_t)(lo != 0) << g | (uint64_t)(hi != 0) << (g + kHalfShift);
-      } else if constexpr (QT == 16) {
-        const uint64_t lo = __ballot(flags_set_low(acc)), hi = __ballot(flags_set_high(acc));
-        pending |= (uint64_t)(lo != 0) << g | (uint64_t)(hi != 0) << (g + kHalfShift);
-      } else {
-        const uint64_t vote = __ballot(flags_set(acc));
-        pending |= (uint64_t)(vote != 0) << g;
-      }
+      // registers; one vote per half of the query tiles, the second half's bits
+      // kHalfShift above the first's
+      constexpr uint32_t kMask = kTri ? kFlagMaskTri : kFlagMask;
+      const uint64_t lo = __ballot(((acc[0] | acc[1]) & kMask) != 0);
+      const uint64_t hi = __ballot(((acc[2] | acc[3]) & kMask) != 0);
+      pending |= (uint64_t)(lo != 0) << g | (uint64_t)(hi != 0) << (g + kHalfShift);
 #pragma unroll
       for (int m = 0; m < kFlagChains; m++) acc[m] = 0u;
       __syncthreads();
@@ -500,7 +475,7 @@ __device__ __forceinline__ void stream_shared(const Expanded (&qa)[QT],
   }
 }
 
-template <int QT, bool kPlane, bool kTri>
+template <bool kPlane, bool kTri>
 __device__ __forceinline__ void mfma_item_shared(SharedRowsLds& S,
                                                  const uint32_t* __restrict__ db, const uint32_t* __restrict__ plane,
                                                  uint64_t n_rows, uint64_t sub, uint32_t sgroup,
@@ -517,26 +492,26 @@ __device__ __forceinline__ void mfma_item_shared(SharedRowsLds& S,
 
   // query operands; a wave whose group lies past the last query gets zero
   // operands (its products never reach the bound) and still stages its tiles
-  const uint32_t qbase = (sgroup * kMfmaWaves + wave) * (uint32_t)(QT * 16);
-  uint32_t qw[QT];
+  const uint32_t qbase = (sgroup * kMfmaWaves + wave) * (uint32_t)(kSharedQt * 16);
+  uint32_t qw[kSharedQt];
 #pragma unroll
-  for (int t = 0; t < QT; t++) {
+  for (int t = 0; t < kSharedQt; t++) {
     const uint32_t qi = qbase + 16 * t + rn;
     qw[t] = queries[(size_t)(qi < n_queries ? qi : n_queries - 1) * 8 + kq];
   }
-  Expanded qa[QT];
+  Expanded qa[kSharedQt];
 #pragma unroll
-  for (int t = 0; t < QT; t++) {
+  for (int t = 0; t < kSharedQt; t++) {
     expand_word(qw[t], qa[t]);
     if (qbase + 16 * t + rn >= n_queries) qa[t].d[0] = qa[t].d[1] = qa[t].d[2] = qa[t].d[3] = 0;
   }
 
   const RowSource<kPlane> src(db, plane, row0, lane);
   if (row0 + kSharedRows <= n_rows)
-    stream_shared<QT, true, kPlane, kTri>(qa, S, src, db, row0, n_rows, qbase, wave, lane, bound, recs,
+    stream_shared<true, kPlane, kTri>(qa, S, src, db, row0, n_rows, qbase, wave, lane, bound, recs,
                                           rec_count, rec_cap, rec_sub_base);
   else
-    stream_shared<QT, false, kPlane, kTri>(qa, S, src, db, row0, n_rows, qbase, wave, lane, bound, recs,
+    stream_shared<false, kPlane, kTri>(qa, S, src, db, row0, n_rows, qbase, wave, lane, bound, recs,
                                            rec_count, rec_cap, rec_sub_base);
 }
 
@@ -557,7 +532,6 @@ __device__ __forceinline__ void item_coords(uint64_t item, uint32_t groups, uint
 // stores zero to clear_rec and clear_hits where they are given: the record
 // count of the stream's next call, and this call's hit counter (this kernel
 // appends no hits).
-constexpr int kSharedQt = 16;
 template <bool kPlane, bool kTri>
 __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(3))) pdq_match_mfma_kernel(
     const uint32_t* __restrict__ db, const uint32_t* __restrict__ plane, uint64_t n_rows,
@@ -572,7 +546,7 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
   uint32_t sgroup;
   item_coords(blockIdx.x, sgroups, sub, sgroup);
   __shared__ SharedRowsLds S;
-  mfma_item_shared<kSharedQt, kPlane, kTri>(S, db, plane, n_rows, sub, sgroup, queries, n_queries, threshold, recs,
+  mfma_item_shared<kPlane, kTri>(S, db, plane, n_rows, sub, sgroup, queries, n_queries, threshold, recs,
                                             rec_count, rec_cap, 0);
 }
 
@@ -1114,9 +1088,9 @@ __global__ void __launch_bounds__(64 * kHeldWaves) __attribute__((amdgpu_waves_p
 // tile with a pair at the bound checks every such pair with the exact
 // 256-bit distance.  The block's hits gather in LDS and take their slots in
 // the hit buffer with one atomic.  If the records overflowed their area (more
-// than rec_cap: dense hits), every work item is matched again in the
-// per-wave layout instead (each half of the block an item), which checks its
-// own candidates (the first kernel appended no hits), so the set stays exact.
+// than rec_cap: dense hits), all rows are matched again in the even layout
+// instead, a part per wave, which checks its own candidates (the first kernel
+// appended no hits), so the set stays exact.
 constexpr int kResolveWaves = 8;
 // Two blocks per CU (16 waves; the kernel fits 128 VGPRs at its at most 8
 // query tiles per wave): a
@@ -1302,23 +1276,19 @@ __device__ __forceinline__ void resolve_record(ResolveLds& L, const PartLoads<QT
   }
 }
 
-// Query tiles per wave in the recheck: at most eight.  A record of a 16-tile
-// stream is checked as two halves (query tiles 0-7 and 8-15, each with its
-// own pending groups), one after the other by the wave that holds the
-// record: sixteen tiles' operands need more registers than two blocks per CU
-// leave, and a half without candidates costs nothing.
-template <int QT>
-constexpr int kResolveQt = QT > 8 ? 8 : QT;
+// Query tiles per wave in the recheck.  A record is checked as two halves (query
+// tiles 0-7 and 8-15, each with its own pending groups), one after the other by
+// the wave that holds the record: sixteen tiles' operands need more registers
+// than two blocks per CU leave, and a half without candidates costs nothing.
+constexpr int kResolveQt = kSharedQt / 2;
+constexpr uint32_t kParts = 2;
 
-// The pending groups of part `part` of a record (of kParts parts).
-template <int kParts>
+// The pending groups of half `part` of a record.
 __device__ __forceinline__ uint32_t part_groups(uint32_t mask, uint32_t part) {
-  static_assert(kParts == 1 || kParts == 2, "whole records or halves of a 16-tile record");
-  if constexpr (kParts == 1) return mask;
-  else return (mask >> (kHalfShift * part)) & ((1u << kHalfShift) - 1);
+  return (mask >> (kHalfShift * part)) & ((1u << kHalfShift) - 1);
 }
 
-template <int QT, bool kPlane>
+template <bool kPlane>
 __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_kernel(
     const uint32_t* __restrict__ db, const uint32_t* __restrict__ plane, uint64_t n_rows,
     const uint32_t* __restrict__ queries, uint32_t n_queries, uint32_t threshold, MatchHit* __restrict__ hits,
@@ -1349,7 +1319,6 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_kernel(
   // checks (a record's candidates are usually in one part).  The record of
   // the item after next is fetched, and the next item's loads are issued,
   // while this one is checked.
-  constexpr int kRq = kResolveQt<QT>, kParts = QT / kRq;
   const uint32_t w0 = blockIdx.x * kResolveWaves + wave;
   const uint32_t S = gridDim.x * kResolveWaves;
   auto rec_of = [&](uint32_t j) { return w0 + (j / kParts) * S; };
@@ -1360,14 +1329,14 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_kernel(
   auto row0_of = [](const uint4& x) { return ((uint64_t)x.y << 32 | x.x) * kSharedRows; };
   // the pending groups of item j (none past the last record)
   auto pending_of = [&](const uint4& x, uint32_t j) {
-    return rec_of(j) < n_recs ? part_groups<kParts>(x.w, j % kParts) : 0u;
+    return rec_of(j) < n_recs ? part_groups(x.w, j % kParts) : 0u;
   };
-  auto qbase_of = [](const uint4& x, uint32_t j) { return x.z + (j % kParts) * (kRq * 16); };
+  auto qbase_of = [](const uint4& x, uint32_t j) { return x.z + (j % kParts) * (kResolveQt * 16); };
   uint32_t j = 0;
   uint4 rec = fetch(0);
   uint4 rec_next = fetch(1);
-  PartLoads<kRq> P;
-  part_load<kRq, kPlane>(P, db, plane, n_rows, row0_of(rec), qbase_of(rec, 0), pending_of(rec, 0), queries,
+  PartLoads<kResolveQt> P;
+  part_load<kResolveQt, kPlane>(P, db, plane, n_rows, row0_of(rec), qbase_of(rec, 0), pending_of(rec, 0), queries,
                          n_queries);
   // The first part's words arrive here (vmcnt 0; expcnt and lgkmcnt left
   // alone), as every later part's do at the end of the previous iteration:
@@ -1376,11 +1345,11 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_kernel(
   __builtin_amdgcn_s_waitcnt(0x0F70);
   for (; rec_of(j) < n_recs; j++) {
     uint4 rec_after;
-    PartLoads<kRq> Pn;
-    resolve_record<kRq, kPlane>(L, P, db, plane, n_rows, row0_of(rec), qbase_of(rec, j), pending_of(rec, j),
+    PartLoads<kResolveQt> Pn;
+    resolve_record<kResolveQt, kPlane>(L, P, db, plane, n_rows, row0_of(rec), qbase_of(rec, j), pending_of(rec, j),
                                 queries, n_queries, threshold, hits, capacity, counter, index_base, [&] {
                                   rec_after = fetch(j + 2);
-                                  part_load<kRq, kPlane>(Pn, db, plane, n_rows, row0_of(rec_next),
+                                  part_load<kResolveQt, kPlane>(Pn, db, plane, n_rows, row0_of(rec_next),
                                                          qbase_of(rec_next, j + 1), pending_of(rec_next, j + 1),
                                                          queries, n_queries);
                                 });
@@ -1422,7 +1391,7 @@ __global__ void __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_p
     item_coords(item, sgroups, gsub, sgroup);
     const ShardView& v = shards[shard_of_chunk(shards, n_shards, gsub / kSubsPerChunk)];
     const uint64_t sub_base = v.chunk_begin * kSubsPerChunk;
-    mfma_item_shared<kSharedQt, true, kTri>(S, reinterpret_cast<const uint32_t*>(v.rows),
+    mfma_item_shared<true, kTri>(S, reinterpret_cast<const uint32_t*>(v.rows),
                                        reinterpret_cast<const uint32_t*>(v.plane), v.n_rows, gsub - sub_base, sgroup,
                                        queries, nq, threshold, recs, rec_count, rec_cap, sub_base);
   }
@@ -1459,7 +1428,6 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_shards_k
     return;
   }
   // whole records per wave, as in pdq_match_resolve_kernel
-  constexpr int kRq = kResolveQt<kSharedQt>, kParts = kSharedQt / kRq;
   const uint32_t stride = gridDim.x * kResolveWaves;
   uint32_t i = blockIdx.x * kResolveWaves + wave;
   uint4 rec = i < n_recs ? recs[i] : make_uint4(0, 0, 0, 0);
@@ -1471,12 +1439,12 @@ __global__ void __launch_bounds__(64 * kResolveWaves) pdq_match_resolve_shards_k
     const uint32_t* rows = reinterpret_cast<const uint32_t*>(v.rows);
     const uint32_t* vplane = reinterpret_cast<const uint32_t*>(v.plane);
 #pragma unroll 1
-    for (int part = 0; part < kParts; part++) {
-      const uint32_t qbase = rec.z + part * (kRq * 16);
-      const uint32_t pending = part_groups<kParts>(rec.w, part);
-      PartLoads<kRq> P;
-      part_load<kRq, true>(P, rows, vplane, v.n_rows, row0, qbase, pending, queries, nq);
-      resolve_record<kRq, true>(L, P, rows, vplane, v.n_rows, row0, qbase, pending, queries, nq, threshold, hits,
+    for (uint32_t part = 0; part < kParts; part++) {
+      const uint32_t qbase = rec.z + part * (kResolveQt * 16);
+      const uint32_t pending = part_groups(rec.w, part);
+      PartLoads<kResolveQt> P;
+      part_load<kResolveQt, true>(P, rows, vplane, v.n_rows, row0, qbase, pending, queries, nq);
+      resolve_record<kResolveQt, true>(L, P, rows, vplane, v.n_rows, row0, qbase, pending, queries, nq, threshold, hits,
                                   capacity, counter, v.index_base, [] {});
     }
     rec = next;
@@ -1704,7 +1672,7 @@ static hipError_t launch_shared(const void* db, const void* plane, uint64_t n_ro
     constexpr bool kPlane = decltype(pl)::value, kTri = decltype(tr)::value;
     hipLaunchKernelGGL((pdq_match_mfma_kernel<kPlane, kTri>), grid, block, 0, stream, d, p, n_rows, q, n_queries,
                        threshold, sgroups, ra.recs, rc, cap, rc_next, hits_clear);
-    hipLaunchKernelGGL((pdq_match_resolve_kernel<kSharedQt, kPlane>), rgrid, rblock, 0, stream, d, p, n_rows, q,
+    hipLaunchKernelGGL((pdq_match_resolve_kernel<kPlane>), rgrid, rblock, 0, stream, d, p, n_rows, q,
                        n_queries, threshold, hits, capacity, counter, index_base, ra.recs, rc, cap);
   };
   using T = std::integral_constant<bool, true>;
@@ -1754,7 +1722,7 @@ static hipError_t with_query_tiles(int qt, F&& f) {
 // The even layout's waves that are resident at once: four per SIMD.
 static uint32_t even_waves_per_xcd(int cus) { return (uint32_t)std::max(1, cus) * 16 / 8; }
 
-// The even layout's launch.
+// The held-rows layout's launch.
 template <int kPer>
 static hipError_t launch_held_plan(const HeldPlan& plan, const void* db, const void* plane, uint64_t n_rows,
                                    const void* queries, uint32_t n_queries, uint32_t threshold, MatchHit* hits,
