@@ -190,10 +190,12 @@ int yume_pdq_amd_dihedrals_batch(const float *d_pdqf, const float *d_thr_in, uin
  * visiting order) up to `capacity`; *d_count receives the exact number of
  * hits (reset first unless flags has YUME_PDQ_AMD_MATCH_APPEND).  The call
  * does not wait; read *d_count after synchronising `stream`.  Batches of 32+
- * queries at threshold < 64 run on the matrix cores (an exact fp4 +-1 dot
- * product over the first 128 bits as a filter, then the full 256-bit integer
- * distance for every surviving pair); smaller batches on the vector ALUs.
- * Both give the same set; flags MATCH_VALU / MATCH_MFMA force one.
+ * queries at threshold < 64, and of 12+ at threshold <= 40, run on the matrix
+ * cores (an exact fp4 +-1 dot product over the first 128 bits as a filter, then
+ * the full 256-bit integer distance for every surviving pair); others on the
+ * vector ALUs.  Both give the same set; flags MATCH_VALU / MATCH_MFMA force one.
+ * From a threshold of about 46, where many pairs pass the filter, MATCH_VALU is
+ * the faster path over 10^6 rows and more.
  */
 int yume_pdq_amd_match(const uint8_t *d_db, uint64_t n_rows, const uint8_t *d_queries,
                        uint32_t n_queries, uint32_t threshold, YumePdqAmdHit *d_hits,
